@@ -578,7 +578,7 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
   // the Limber launch shape, its slice partials and the staged output are
   // settled before the first launch, so a call whose buffers do not fit the
   // scratch fails before any work is queued
-  const int l_waves = auto_waves(ctx, ncols);
+  const int l_waves = nd == 0 && use_tab && !use_mx ? FWD_WAVES : auto_waves(ctx, ncols);
   const int l_slices = use_mx ? 1 : auto_slices(ctx, ncols, l_waves, Na, nd, use_tab ? 2 : 1);
   const size_t nslice = nd == 7 ? (size_t)ncols * 7 : (size_t)B * P * n_ell * (nd == 1 ? 2 : 1);
   const size_t nout = (size_t)B * P * n_ell;

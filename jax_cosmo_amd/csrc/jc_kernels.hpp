@@ -38,6 +38,39 @@ enum CoefSlot {
   CF_MU,           // halofit mu_n (0 for takahashi2012)
   NCOEF
 };
+// The record of forward calls in transfer-table mode (same size).  The
+// reference's per-point products of an a-node factor and a multipole factor
+// are split so that each slot holds everything that depends on a alone: with
+// l = ell + 1/2, k = l / max(chi, 1) and y = k R_nl,
+//   table position      u = ln(l) invh + FT_Q + FT_T
+//   Delta_L^2         d2l = T^2 k^n_s l^3 FT_G3
+//   y                     = l FT_YC,  log2 y = log2 l + FT_LA
+//   1 + mu/y + nu/y^2     = 1 + (FT_MU + FT_NU / l) / l
+//   (c f3 y)^(3-gamma)    = 2^(FT_GAM log2 y + FT_GC)
+// and M(a, ell) = l^-3 FT_AW [bracket], whose l^-3 leaves the sum over a.
+// Slots 0-15 are read as four float4.
+enum FwdSlot {
+  FT_Q = 0,  // int32 bits: floor of (-ln max(chi, 1) - lo) invh, and its
+  FT_T,      // fraction (lo, invh: the transfer table's grid)
+  FT_G3,     // D^2 pknorm / (2 pi^2 max(chi, 1)^3)
+  FT_LA,     // log2(R_nl / max(chi, 1))
+  FT_YC,     // R_nl / max(chi, 1)
+  FT_MU,     // mu_n max(chi, 1) / R_nl
+  FT_NU,     // nu_n (max(chi, 1) / R_nl)^2
+  FT_BETA,
+  FT_F1X3,
+  FT_F2,
+  FT_GAM,    // 3 - gamma_n
+  FT_GC,     // (3 - gamma_n) log2(c_n f3)
+  FT_ALPHA,
+  FT_BN,
+  FT_AN,
+  FT_AW,     // 2 pi^2 max(chi, 1)^3 x Simpson weight x dchi/da / max(chi^2, 1) / c^2
+  FT_CHI = CF_CHI,
+  FT_LNHI = 18,  // -ln max(chi, 1) as a float and
+  FT_LNLO = 19,  // the rest
+};
+static_assert(NCOEF == 20, "FwdSlot shares the record of CoefSlot");
 // Per-cosmology record (EH98 constants and the lensing prefactor).
 enum CrecSlot {
   CR_FB = 0, CR_FC, CR_INV13KEQ, CR_BETAC18, CR_C14A, CR_SHD, CR_ALPHAB, CR_BETAB,
@@ -171,6 +204,10 @@ struct LimberArgs {
   int slices;               // 1 = no split
   float* part;
 };
+
+// waves per block of the forward kernel in table mode (it ignores
+// LimberArgs::waves, the tile of the other Limber kernels)
+constexpr int FWD_WAVES = 4;
 
 struct PkArgs {            // P(k, a) evaluation at (k_i, a_i) pairs
   int n;                   // points for one cosmology

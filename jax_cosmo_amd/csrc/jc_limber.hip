@@ -51,30 +51,6 @@ JC_D Sf limber_point(const EHc<Sf>& eh, const Sf& ns, const PointCoefs<Sf, W>& p
   return pc.wgt * halofit_pnl(pc.hf, lgy, y, iy, k3, ik3, plin);
 }
 
-// The same with T(k) k^(n_s/2) read from the cosmology's transfer table in
-// LDS (cubic Hermite pieces uniform in ln k).  The table position is formed
-// in FP64 so that it matches the node placement exactly; the remaining
-// uncertainty is that of the float ln k itself.
-JC_D float limber_point_tab(const float4* tab, double invh, double lo_invh, const PointCoefs<float, 1>& pc,
-                            const EllC& lc) {
-  const float k = lc.lph * pc.invchi;
-  const float invk = lc.ilph * pc.chi1;
-  const float lnk = lc.lnlph + pc.lninvchi;
-  const double u = __builtin_fma((double)lnk, invh, -lo_invh);
-  int q = (int)u;
-  q = q < 0 ? 0 : (q > NEHQ - 1 ? NEHQ - 1 : q);
-  const float t = (float)(u - (double)q);
-  const float4 cc = tab[q];
-  const float tn = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cc.w, t, cc.z), t, cc.y), t, cc.x);
-  const float plin = (tn * tn) * pc.g2p;               // power.py:48-51
-  const float k3 = k * k * k;
-  const float ik3 = invk * invk * invk;
-  const float lgy = __builtin_fmaf(lnk, 1.4426950408889634f, pc.lgRnl);  // log2 y
-  const float y = k * pc.Rnl;                          // power.py:252
-  const float iy = invk * pc.knl;
-  return pc.wgt * halofit_pnl(pc.hf, lgy, y, iy, k3, ik3, plin);
-}
-
 // Adjoint kernel: M = weight * P_nl at one point and its 7 parameter
 // derivatives.  T(k) stays a forward dual (the EH98 constants and k carry
 // theta); everything after it is differentiated in reverse, once per point:
@@ -239,11 +215,8 @@ __device__ inline int xcd_group(int b, int n) {
 template <int NACC>
 struct RedChunk { static constexpr int value = NACC < 32 ? NACC : 32; };
 
-// PF: 0 = the a-node's records are loaded when needed, 1 = the per-a
-// coefficients of the next node are loaded one node ahead (the tracer
-// kernels are loaded at the top of each node and used after P_nl).
 // (forward kernels are held to 128 VGPRs: 4 waves per SIMD)
-template <int T, int ND, bool TAB, int PF>
+template <int T, int ND, bool TAB>
 __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A) {
   using Sf = typename Types<ND>::F;
   constexpr int W = ND + 1;
@@ -251,7 +224,7 @@ __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A)
   constexpr bool VJP = (ND == 7);
   constexpr int NACC = VJP ? 7 : P * W;
   constexpr int RCH = RedChunk<NACC>::value;
-  static_assert(!TAB || ND == 0 || ND == 7, "the transfer table serves the forward and adjoint kernels");
+  static_assert(!TAB || ND == 7, "forward calls in table mode run k_limber_tab");
   // TAB: [2][NEHQ] tables (the adjoint reads its theta-derivative rows from
   // global memory); after the a loop, [waves-1][RCH][64] partial sums
   extern __shared__ float4 lds4[];
@@ -328,9 +301,7 @@ __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A)
 #pragma unroll
     for (int i = 0; i < T; ++i) Rv[i] = Mem<Sf>::ld(rp + i * W);
     if constexpr (!VJP) {
-      Sf M;
-      if constexpr (TAB) M = limber_point_tab(tab, invh, lo_invh, pc, lc);
-      else M = limber_point<Sf, W>(eh, ns, pc, lc);
+      const Sf M = limber_point<Sf, W>(eh, ns, pc, lc);
       int p = 0;
 #pragma unroll
       for (int i = 0; i < T; ++i) {
@@ -366,24 +337,7 @@ __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A)
       }
     }
   };
-  if constexpr (PF) {
-    // two register sets in turn: the next node's coefficients load while the
-    // current node computes, with no copies between the sets
-    constexpr int CS = NCOEF * W;
-    const int RS = A.Tpad * W;
-    PointCoefs<Sf, W> pa, pb;
-    if (m0 < m1) pa = load_coefs<Sf, W>(cf);
-    for (int m = m0; m < m1; m += 2, cf += 2 * CS, rr += 2 * RS) {
-      const bool has_b = m + 1 < m1;
-      if (has_b) pb = load_coefs<Sf, W>(cf + CS);
-      point(pa, rr);
-      if (!has_b) break;
-      if (m + 2 < m1) pa = load_coefs<Sf, W>(cf + 2 * CS);
-      point(pb, rr + RS);
-    }
-  } else {
-    for (int m = m0; m < m1; ++m, cf += NCOEF * W, rr += A.Tpad * W) point(load_coefs<Sf, W>(cf), rr);
-  }
+  for (int m = m0; m < m1; ++m, cf += NCOEF * W, rr += A.Tpad * W) point(load_coefs<Sf, W>(cf), rr);
 
   // deterministic reduction over the waves of the block, RCH accumulators
   // per pass (the LDS space of the tables is reused)
@@ -494,7 +448,6 @@ __global__ __launch_bounds__(512, 4) void k_limber_mx(LimberArgs A) {
   const int cB = min(col0 + 31, A.ncols - 1) / A.n_ell;
   const bool mixed = cA != cB;  // uniform over the block
   const double ell = A.ell[li];
-  const EllC lc = ell_consts(ell);
   const float lf = (float)(::sqrt((ell - 1.0) * ell * (ell + 1.0) * (ell + 2.0)) / ((ell + 0.5) * (ell + 0.5)));
 
   // tracer indices of this lane's A-operand rows
@@ -509,18 +462,18 @@ __global__ __launch_bounds__(512, 4) void k_limber_mx(LimberArgs A) {
 
   float ns = 0.0f;
   EHc<float> eh;
+  EllC lc;
+  EllT lt;
   const float4* tab = nullptr;
-  double invh = 0.0, lo_invh = 0.0;
   if constexpr (TAB) {
     const int cb0 = (blockIdx.x * 64) / A.n_ell;
     const int ce0 = min(blockIdx.x * 64 + 63, A.ncols - 1) / A.n_ell;
     for (int e = threadIdx.x; e < (ce0 - cb0 + 1) * NEHQ; e += blockDim.x) lds4[e] = A.ehtab[(size_t)cb0 * NEHQ + e];
     tab = lds4 + (c - cb0) * NEHQ;
-    const float* cr = A.crec + (size_t)c * NCREC;
-    invh = (double)cr[CR_EHINVH];
-    lo_invh = (double)cr[CR_EHLO] * invh;
+    lt = ell_tab(ell, (double)A.crec[(size_t)c * NCREC + CR_EHINVH]);
     __syncthreads();
   } else {
+    lc = ell_consts(ell);
     eh = load_eh<float, 1>(A.crec + (size_t)c * NCREC, ns);
   }
 
@@ -548,13 +501,19 @@ __global__ __launch_bounds__(512, 4) void k_limber_mx(LimberArgs A) {
   const int q0 = wave * chunk;
   const int q1 = min(np, q0 + chunk);
 
-  auto step = [&](int q, const PointCoefs<float, 1>& pc) {
+  using Rec = typename std::conditional<TAB, FwdRec, PointCoefs<float, 1>>::type;
+  auto step = [&](int q, const Rec& pc) {
     const int m = 2 * q + kk;
     const bool vm = m < A.Na;
     const int mm = vm ? m : A.Na - 1;
     float M;
-    if constexpr (TAB) M = limber_point_tab(tab, invh, lo_invh, pc, lc);
-    else M = limber_point<float, 1>(eh, ns, pc, lc);
+    if constexpr (TAB) {
+      float t;
+      const int piece = tab_piece(pc, lt, t);
+      M = fwd_point(tab[piece], t, pc, lt);
+    } else {
+      M = limber_point<float, 1>(eh, ns, pc, lc);
+    }
     M = (vm && valid) ? M : 0.0f;
     // the loads are unconditional (in-bounds rows) and masked afterwards
     const int ro = mm * A.Tpad;
@@ -579,9 +538,10 @@ __global__ __launch_bounds__(512, 4) void k_limber_mx(LimberArgs A) {
   const float* cbase = A.coef + (size_t)c * A.Na * NCOEF;
   auto rec = [&](int q) {
     const int m = min(2 * q + kk, A.Na - 1);
-    return load_coefs<float, 1>(cbase + (size_t)m * NCOEF);
+    if constexpr (TAB) return load_fwd(cbase + (size_t)m * NCOEF);
+    else return load_coefs<float, 1>(cbase + (size_t)m * NCOEF);
   };
-  PointCoefs<float, 1> pa_, pb_;
+  Rec pa_, pb_;
   if (q0 < q1) pa_ = rec(q0);
   for (int q = q0; q < q1; q += 2) {
     const bool has_b = q + 1 < q1;
@@ -623,18 +583,168 @@ __global__ __launch_bounds__(512, 4) void k_limber_mx(LimberArgs A) {
       if (p < P) {
         int ti, tj;
         pair_ij(p, T, ti, tj);
-        const float f = (((A.wl_mask >> ti) & 1u) ? lf : 1.0f) * (((A.wl_mask >> tj) & 1u) ? lf : 1.0f);
+        float f = (((A.wl_mask >> ti) & 1u) ? lf : 1.0f) * (((A.wl_mask >> tj) & 1u) ? lf : 1.0f);
+        if constexpr (TAB) f *= ell_m3(ell);
         A.out[((size_t)c * P + p) * A.n_ell + li] = acc[rb][r] * f;
       }
     }
   }
 }
 
-// record prefetch per mode (measured on MI355X: the table mode's shorter
-// point leaves load latency exposed; the closed form hides it and is
-// register-bound)
-constexpr int PF_TAB = 1;
-constexpr int PF_CLOSED = 0;
+// ------------------------------------------------------------------ forward kernel, table mode
+// Forward C_ell with the transfer function from the cosmologies' tables (calls
+// with n_ell >= 64, so that 64 consecutive columns span at most two
+// cosmologies).  Bound by VALU issue: a point costs 34 simple and 6
+// transcendental instructions plus one FMA per pair and a multiply per tracer.
+// The a-node records and tracer kernels are the same for all lanes of a
+// cosmology; read as broadcast loads through the L1 (16 cycles per float4 and
+// CU) they took longer than the arithmetic, so each wave stages its next FCH
+// nodes in LDS (one coalesced float4 of each per lane, in flight while the
+// current nodes compute) and reads them back as broadcasts at 4.5 cycles.
+// 4 waves (FWD_WAVES) split the a range of a block's 64 columns and share the
+// 32 KB of tables: 4 blocks fit a CU's LDS and fill the 4 waves per SIMD that
+// 128 VGPRs allow.  Measured, 10 tracers: 2048 cosmologies x 200 ell x n_z 1024
+// 2127 -> 933 us (2 waves 1392, 8 waves 960), 1024 x 100 x 512 237 -> 162 us.
+// The pair sums stay on the VALU: FP32 matrix instructions issue through it (a
+// 32x32x2 takes 64 cycles and none of them overlap other waves' VALU work),
+// and this kernel with its pairs on them ran 1194 us.
+constexpr int FCH = 8;  // a-nodes staged per wave
+
+template <int T>
+struct FwdShape {
+  static constexpr int P = T * (T + 1) / 2;
+  static constexpr int TP = (T + 3) / 4 * 4;
+  static constexpr int RCH = RedChunk<P>::value;        // accumulators reduced per pass
+  static constexpr int WAVE_LDS = 2 * FCH * (16 + TP);  // floats staged per wave
+  static size_t lds(int waves) {
+    const size_t run = (size_t)2 * NEHQ * sizeof(float4) + (size_t)waves * WAVE_LDS * sizeof(float);
+    const size_t red = (size_t)(waves - 1) * RCH * 64 * sizeof(float);
+    return run > red ? run : red;
+  }
+};
+
+template <int T>
+__global__ __launch_bounds__(64 * FWD_WAVES, 4) void k_limber_tab(LimberArgs A) {
+  using S = FwdShape<T>;
+  constexpr int P = S::P, TP = S::TP, RCH = S::RCH;
+  constexpr int nwv = FWD_WAVES;
+  extern __shared__ float4 lds4[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float4* srec = lds4 + 2 * NEHQ + wave * (S::WAVE_LDS / 4);  // [2][FCH][4]
+  float4* sR = srec + 2 * FCH * 4;                            // [2][FCH][TP / 4]
+
+  const int g0 = xcd_group(blockIdx.x, gridDim.x) * 64;
+  const int g = g0 + lane;
+  const bool valid = g < A.ncols;
+  const int gc = valid ? g : A.ncols - 1;
+  const int c = gc / A.n_ell;
+  const int li = gc - c * A.n_ell;
+  const int c0 = g0 / A.n_ell;
+  const int c1 = min(A.ncols - 1, g0 + 63) / A.n_ell;
+  const double ell = A.ell[li];
+  const int own = c - c0;  // 0 or 1: the lane's cosmology
+  for (int e = threadIdx.x; e < (c1 - c0 + 1) * NEHQ; e += blockDim.x) lds4[e] = A.ehtab[(size_t)c0 * NEHQ + e];
+  const EllT lt = ell_tab(ell, (double)A.crec[(size_t)c * NCREC + CR_EHINVH]);
+  __syncthreads();
+  const float4* tab = lds4 + own * NEHQ;
+
+  // the a range of this wave: one of slices x waves contiguous chunks
+  const int nsl = A.slices;
+  const int chunk = (A.Na + nsl * nwv - 1) / (nsl * nwv);
+  const int m0 = min(A.Na, ((int)blockIdx.y * nwv + wave) * chunk);
+  const int m1 = min(A.Na, m0 + chunk);
+
+  // staging: lane -> (cosmology, node, float4) of the records and, for lanes
+  // below 4 TP, of the tracer kernels
+  static_assert(FCH == 8 && TP <= 16, "the staging map deals 2 x 8 x 4 float4 to 64 lanes");
+  const int rs = lane >> 5, rn = (lane >> 2) & 7;
+  const int tl = min(lane, 4 * TP - 1), ts = tl / (2 * TP), tn = (tl % (2 * TP)) / (TP / 4);
+  const float4* grec = reinterpret_cast<const float4*>(A.coef + (size_t)(rs ? c1 : c0) * A.Na * NCOEF) + (lane & 3);
+  const float4* gR = reinterpret_cast<const float4*>(A.R + (size_t)(ts ? c1 : c0) * A.Na * TP) + tl % (TP / 4);
+  auto fetch = [&](int m, float4& r, float4& k) {
+    r = grec[(size_t)min(m + rn, A.Na - 1) * (NCOEF / 4)];
+    k = gR[(size_t)min(m + tn, A.Na - 1) * (TP / 4)];
+  };
+
+  float acc[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) acc[p] = 0.0f;
+  const float4* rec = srec + own * FCH * 4;
+  const float* ker = reinterpret_cast<const float*>(sR + own * FCH * (TP / 4));
+  auto point = [&](int n) {
+    const FwdRec r{rec[4 * n], rec[4 * n + 1], rec[4 * n + 2], rec[4 * n + 3]};
+    float t;
+    const int q = tab_piece(r, lt, t);
+    const float M = fwd_point(tab[q], t, r, lt);
+    const float* k = ker + n * TP;
+    float Rv[T];
+#pragma unroll
+    for (int i = 0; i < T; ++i) Rv[i] = k[i];
+    int p = 0;
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+      const float u = Rv[i] * M;
+#pragma unroll
+      for (int j = i; j < T; ++j) acc[p++] += Rv[j] * u;
+    }
+  };
+
+  float4 nr, nk;
+  if (m0 < m1) fetch(m0, nr, nk);
+  for (int mc = m0; mc < m1; mc += FCH) {
+    // wave-private staging: the wave's LDS operations complete in order, so
+    // these writes follow the previous nodes' reads
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    srec[lane] = nr;
+    if (lane < 4 * TP) sR[lane] = nk;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (mc + FCH < m1) fetch(mc + FCH, nr, nk);
+    const int nn = min(FCH, m1 - mc);
+    for (int n = 0; n < nn; n += 2) {  // two nodes per turn: more would spill
+      point(n);
+      if (n + 1 < nn) point(n + 1);
+    }
+  }
+
+  // deterministic reduction over the waves of the block, RCH accumulators
+  // per pass (the LDS space of the tables is reused)
+  float* red = reinterpret_cast<float*>(lds4);
+#pragma unroll
+  for (int q0 = 0; q0 < P; q0 += RCH) {
+    __syncthreads();
+    if (wave > 0) {
+#pragma unroll
+      for (int q = q0; q < q0 + RCH && q < P; ++q) red[((wave - 1) * RCH + (q - q0)) * 64 + lane] = acc[q];
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll 1
+      for (int w = 1; w < nwv; ++w) {
+#pragma unroll
+        for (int q = q0; q < q0 + RCH && q < P; ++q) acc[q] += red[((w - 1) * RCH + (q - q0)) * 64 + lane];
+      }
+    }
+  }
+  if (wave != 0 || !valid) return;
+  // with slices, this block's share goes to part[slice] in the layout of out
+  float* out = nsl > 1 ? A.part + (size_t)blockIdx.y * A.ncols * P : A.out;
+  const float lf = (float)(::sqrt((ell - 1.0) * ell * (ell + 1.0) * (ell + 2.0)) / ((ell + 0.5) * (ell + 0.5)));
+  const float lm3 = ell_m3(ell);
+  int p = 0;
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const float Fi = lm3 * (((A.wl_mask >> i) & 1u) ? lf : 1.0f);
+#pragma unroll
+    for (int j = i; j < T; ++j) {
+      const float Fj = ((A.wl_mask >> j) & 1u) ? lf : 1.0f;
+      out[((size_t)c * P + p) * A.n_ell + li] = acc[p] * Fi * Fj;
+      ++p;
+    }
+  }
+}
 
 template <int T, int ND>
 static hipError_t launch_T(const LimberArgs& a, hipStream_t s) {
@@ -659,10 +769,10 @@ static hipError_t launch_T(const LimberArgs& a, hipStream_t s) {
       return hipGetLastError();
     }
     if (a.ehtab) {
-      if (a.n_ell < 64) return hipErrorInvalidValue;  // a block would span more than two cosmologies
-      const size_t tab = (size_t)2 * NEHQ * sizeof(float4);
-      hipLaunchKernelGGL((k_limber<T, 0, true, PF_TAB>), dim3(blocks, a.slices), dim3(64 * a.waves),
-                         tab > red ? tab : red, s, a);
+      // a block would span more than two cosmologies; the staged rows are TP wide
+      if (a.n_ell < 64 || a.Tpad != FwdShape<T>::TP) return hipErrorInvalidValue;
+      hipLaunchKernelGGL((k_limber_tab<T>), dim3(blocks, a.slices), dim3(64 * FWD_WAVES),
+                         FwdShape<T>::lds(FWD_WAVES), s, a);
       return hipGetLastError();
     }
   }
@@ -670,12 +780,12 @@ static hipError_t launch_T(const LimberArgs& a, hipStream_t s) {
     if (a.ehtab) {
       if (a.n_ell < 64 || !a.ehtab7) return hipErrorInvalidValue;
       const size_t tab = (size_t)2 * NEHQ * sizeof(float4);
-      hipLaunchKernelGGL((k_limber<T, 7, true, PF_CLOSED>), dim3(blocks, a.slices), dim3(64 * a.waves),
+      hipLaunchKernelGGL((k_limber<T, 7, true>), dim3(blocks, a.slices), dim3(64 * a.waves),
                          tab > red ? tab : red, s, a);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((k_limber<T, ND, false, PF_CLOSED>), dim3(blocks, a.slices), dim3(64 * a.waves), red, s, a);
+  hipLaunchKernelGGL((k_limber<T, ND, false>), dim3(blocks, a.slices), dim3(64 * a.waves), red, s, a);
   return hipGetLastError();
 }
 
@@ -810,7 +920,6 @@ __device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int t
   const int c = jb.c;
   const uint32_t wl_mask = jb.wl_mask;
   const double ell = valid ? col.ell : A.cols[tile0].ell;
-  const EllC lc = ell_consts(ell);
 
   int slot = 0;
   if constexpr (STAGED) {
@@ -823,9 +932,7 @@ __device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int t
     __syncthreads();
   }
   const float4* gtab = A.ehtab + (size_t)c * NEHQ;
-  const float* cr = A.crec + (size_t)c * NCREC;
-  const double invh = (double)cr[CR_EHINVH];
-  const double lo_invh = (double)cr[CR_EHLO] * invh;  // exact in FP64
+  const EllT lt = ell_tab(ell, (double)A.crec[(size_t)c * NCREC + CR_EHINVH]);
   // this wave's share of the a range
   const int chunk = (A.Na + nsl * nwv - 1) / (nsl * nwv);
   const int m0 = min(A.Na, ((int)blockIdx.y * nwv + wave) * chunk);
@@ -835,29 +942,17 @@ __device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int t
 #pragma unroll
   for (int q = 0; q < P; ++q) acc[q] = 0.0f;
 
-  // one (column, a-node) point: limber_point_tab with the table row from
-  // LDS or global memory, then the contraction
-  auto point = [&](const PointCoefs<float, 1>& pc, const float* rp) {
-    const float k = lc.lph * pc.invchi;
-    const float invk = lc.ilph * pc.chi1;
-    const float lnk = lc.lnlph + pc.lninvchi;
-    const double u = __builtin_fma((double)lnk, invh, -lo_invh);
-    int q = (int)u;
-    q = q < 0 ? 0 : (q > NEHQ - 1 ? NEHQ - 1 : q);
-    const float t = (float)(u - (double)q);
+  // one (column, a-node) point: the table piece from LDS or global memory,
+  // P_nl, then the contraction
+  auto point = [&](const FwdRec& pc, const float* rp) {
+    float t;
+    const int q = tab_piece(pc, lt, t);
     // the table row first: the tracer kernels below are needed only after P_nl
     const float4 cc = STAGED ? lds4[slot + q] : gtab[q];
     float Rv[T];
 #pragma unroll
     for (int i = 0; i < T; ++i) Rv[i] = rp[i];
-    const float tn = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cc.w, t, cc.z), t, cc.y), t, cc.x);
-    const float plin = (tn * tn) * pc.g2p;
-    const float k3 = k * k * k;
-    const float ik3 = invk * invk * invk;
-    const float lgy = __builtin_fmaf(lnk, 1.4426950408889634f, pc.lgRnl);
-    const float y = k * pc.Rnl;
-    const float iy = invk * pc.knl;
-    const float M = pc.wgt * halofit_pnl(pc.hf, lgy, y, iy, k3, ik3, plin);
+    const float M = fwd_point(cc, t, pc, lt);
     int p = 0;
 #pragma unroll
     for (int i = 0; i < T; ++i) {
@@ -875,14 +970,14 @@ __device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int t
     // two register sets in turn: the next node's coefficients load while
     // the current node computes
     const int RS = A.Tpad;
-    PointCoefs<float, 1> pa, pb;
-    if (m0 < m1) pa = load_coefs<float, 1>(cf);
+    FwdRec pa, pb;
+    if (m0 < m1) pa = load_fwd(cf);
     for (int m = m0; m < m1; m += 2, cf += 2 * NCOEF, rr += 2 * RS) {
       const bool has_b = m + 1 < m1;
-      if (has_b) pb = load_coefs<float, 1>(cf + NCOEF);
+      if (has_b) pb = load_fwd(cf + NCOEF);
       point(pa, rr);
       if (!has_b) break;
-      if (m + 2 < m1) pa = load_coefs<float, 1>(cf + 2 * NCOEF);
+      if (m + 2 < m1) pa = load_fwd(cf + 2 * NCOEF);
       point(pb, rr + RS);
     }
   }
@@ -908,10 +1003,11 @@ __device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int t
   if (wave != 0 || !valid) return;
   const float lf = (float)(::sqrt((ell - 1.0) * ell * (ell + 1.0) * (ell + 2.0)) / ((ell + 0.5) * (ell + 0.5)));
   float* out = nsl > 1 ? A.part + (size_t)blockIdx.y * A.part_stride : A.out;
+  const float lm3 = ell_m3(ell);
   int p = 0;
 #pragma unroll
   for (int i = 0; i < T; ++i) {
-    const float Fi = ((wl_mask >> i) & 1u) ? lf : 1.0f;
+    const float Fi = lm3 * (((wl_mask >> i) & 1u) ? lf : 1.0f);
 #pragma unroll
     for (int j = i; j < T; ++j) {
       const float Fj = ((wl_mask >> j) & 1u) ? lf : 1.0f;

@@ -166,7 +166,7 @@ JC_D Sd hermite(const Tt& t, double h, const Sd& f0, const Sd& f1, const Sd& d0,
 }
 
 template <int W>
-JC_D void ehtab_build(int c, int Na, int n_ell, const double* ell, int ell_stride, const float* coef, float* crec,
+JC_D void ehtab_build(int c, int Na, int n_ell, const double* ell, int ell_stride, float* coef, float* crec,
                       float4* ehtab, float* ehtab7, float* s_red, float2* s_nd);
 
 template <int ND, int NT, int MINW>
@@ -742,27 +742,51 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
     Sd invchi = 1.0 / chi1;
 
     float* cf = A.coef + ((size_t)c * A.Na + m) * NCOEF * W;
-    Mem<Sf>::st(cf + CF_INV_CHI * W, conv<Sf>(invchi));
-    Mem<Sf>::st(cf + CF_CHI1 * W, conv<Sf>(chi1));
-    // the logarithms stored as floats are taken to float accuracy
-    Mem<Sf>::st(cf + CF_LNINVCHI * W, conv<Sf>(-jm::logf_acc(chi1)));
-    Mem<Sf>::st(cf + CF_KNL * W, conv<Sf>(1.0 / Rnl));
-    Mem<Sf>::st(cf + CF_MU * W, conv<Sf>(hf.mu_n));
-    Mem<Sf>::st(cf + CF_WGT * W, conv<Sf>(wgt));
-    Mem<Sf>::st(cf + CF_G2P * W, conv<Sf>(g2 * pknorm));
-    Mem<Sf>::st(cf + CF_LGRNL * W, conv<Sf>(jm::logf_acc(Rnl) * 1.4426950408889634));
-    Mem<Sf>::st(cf + CF_RNL * W, conv<Sf>(Rnl));
-    Mem<Sf>::st(cf + CF_AN * W, conv<Sf>(hf.a_n));
-    Mem<Sf>::st(cf + CF_BN * W, conv<Sf>(hf.b_n));
-    Mem<Sf>::st(cf + CF_LGCF3 * W, conv<Sf>(hf.lg_cf3));
-    Mem<Sf>::st(cf + CF_GAM3 * W, conv<Sf>(hf.gam3));
-    Mem<Sf>::st(cf + CF_ALPHA * W, conv<Sf>(hf.alpha_n));
-    Mem<Sf>::st(cf + CF_BETA * W, conv<Sf>(hf.beta_n));
-    Mem<Sf>::st(cf + CF_NU * W, conv<Sf>(hf.nu_n));
-    Mem<Sf>::st(cf + CF_F1X3 * W, conv<Sf>(hf.f1x3));
-    Mem<Sf>::st(cf + CF_F2 * W, conv<Sf>(hf.f2));
-    Mem<Sf>::st(cf + CF_CHI * W, conv<Sf>(chi));
-    Mem<Sf>::st(cf + CF_GROWTH * W, conv<Sf>(g));
+    if (ND == 0 && A.ehtab) {  // forward record (FwdSlot); FT_Q, FT_T follow in ehtab_build
+      if constexpr (ND == 0) {
+        const double yc = Rnl * invchi, iyc = chi1 / Rnl, c3 = chi1 * chi1 * chi1;
+        const double lnchi = jm::logf_acc(chi1);
+        cf[FT_G3] = (float)(g2 * pknorm / (2.0 * PI * PI * c3));
+        cf[FT_LA] = (float)((jm::logf_acc(Rnl) - lnchi) * 1.4426950408889634);
+        cf[FT_YC] = (float)yc;
+        cf[FT_MU] = (float)(hf.mu_n * iyc);
+        cf[FT_NU] = (float)(hf.nu_n * (iyc * iyc));
+        cf[FT_BETA] = (float)hf.beta_n;
+        cf[FT_F1X3] = (float)hf.f1x3;
+        cf[FT_F2] = (float)hf.f2;
+        cf[FT_GAM] = (float)hf.gam3;
+        cf[FT_GC] = (float)(hf.gam3 * hf.lg_cf3);
+        cf[FT_ALPHA] = (float)hf.alpha_n;
+        cf[FT_BN] = (float)hf.b_n;
+        cf[FT_AN] = (float)hf.a_n;
+        cf[FT_AW] = (float)(2.0 * PI * PI * c3 * wgt);
+        cf[FT_CHI] = (float)chi;
+        cf[FT_LNHI] = (float)-lnchi;
+        cf[FT_LNLO] = (float)(-lnchi - (double)(float)-lnchi);
+      }
+    } else {
+      Mem<Sf>::st(cf + CF_INV_CHI * W, conv<Sf>(invchi));
+      Mem<Sf>::st(cf + CF_CHI1 * W, conv<Sf>(chi1));
+      // the logarithms stored as floats are taken to float accuracy
+      Mem<Sf>::st(cf + CF_LNINVCHI * W, conv<Sf>(-jm::logf_acc(chi1)));
+      Mem<Sf>::st(cf + CF_KNL * W, conv<Sf>(1.0 / Rnl));
+      Mem<Sf>::st(cf + CF_MU * W, conv<Sf>(hf.mu_n));
+      Mem<Sf>::st(cf + CF_WGT * W, conv<Sf>(wgt));
+      Mem<Sf>::st(cf + CF_G2P * W, conv<Sf>(g2 * pknorm));
+      Mem<Sf>::st(cf + CF_LGRNL * W, conv<Sf>(jm::logf_acc(Rnl) * 1.4426950408889634));
+      Mem<Sf>::st(cf + CF_RNL * W, conv<Sf>(Rnl));
+      Mem<Sf>::st(cf + CF_AN * W, conv<Sf>(hf.a_n));
+      Mem<Sf>::st(cf + CF_BN * W, conv<Sf>(hf.b_n));
+      Mem<Sf>::st(cf + CF_LGCF3 * W, conv<Sf>(hf.lg_cf3));
+      Mem<Sf>::st(cf + CF_GAM3 * W, conv<Sf>(hf.gam3));
+      Mem<Sf>::st(cf + CF_ALPHA * W, conv<Sf>(hf.alpha_n));
+      Mem<Sf>::st(cf + CF_BETA * W, conv<Sf>(hf.beta_n));
+      Mem<Sf>::st(cf + CF_NU * W, conv<Sf>(hf.nu_n));
+      Mem<Sf>::st(cf + CF_F1X3 * W, conv<Sf>(hf.f1x3));
+      Mem<Sf>::st(cf + CF_F2 * W, conv<Sf>(hf.f2));
+      Mem<Sf>::st(cf + CF_CHI * W, conv<Sf>(chi));
+      Mem<Sf>::st(cf + CF_GROWTH * W, conv<Sf>(g));
+    }
 
     // z-local kernels, H = H0 sqrt(E^2) (background.py:129-148): number
     // counts n(z) b H (probes.py:87-99) and the NLA terms (probes.py:114-124)
@@ -911,7 +935,7 @@ hipError_t launch_tables(int nd, const TablesArgs& a, hipStream_t s, int variant
 // fixed k) at the same NEHQ + 1 nodes, for 4-point Lagrange interpolation in
 // the adjoint kernel.
 template <int W>
-JC_D void ehtab_build(int c, int Na, int n_ell, const double* ell, int ell_stride, const float* coef, float* crec,
+JC_D void ehtab_build(int c, int Na, int n_ell, const double* ell, int ell_stride, float* coef, float* crec,
                       float4* ehtab, float* ehtab7, float* s_red, float2* s_nd) {
   const int tid = threadIdx.x;
   float ll = 3.0e38f, lh = -3.0e38f, cl = 3.0e38f, ch = -3.0e38f;
@@ -921,16 +945,30 @@ JC_D void ehtab_build(int c, int Na, int n_ell, const double* ell, int ell_strid
     lh = fmaxf(lh, v);
   }
   for (int m = tid; m < Na; m += blockDim.x) {
-    const float v = coef[(((size_t)c * Na + m) * NCOEF + CF_LNINVCHI) * W];
+    const float v = coef[(((size_t)c * Na + m) * NCOEF + (W == 1 ? (int)FT_LNHI : (int)CF_LNINVCHI)) * W];
     cl = fminf(cl, v);
     ch = fmaxf(ch, v);
   }
-  const float lo = block_min(ll, s_red) + block_min(cl, s_red);
-  const float hi = block_max(lh, s_red) + block_max(ch, s_red);
+  // a margin of a few float ulps of ln k on both sides: every point's
+  // position lies inside the table whichever way it is rounded
+  constexpr float MARGIN = 2e-5f;
+  const float lo = block_min(ll, s_red) + block_min(cl, s_red) - MARGIN;
+  const float hi = block_max(lh, s_red) + block_max(ch, s_red) + MARGIN;
   const double span = fmax((double)hi - (double)lo, 1e-3);
   float invh = (float)(NEHQ / span);
   if ((double)invh * span > (double)NEHQ) invh = nextafterf(invh, 0.0f);
   const double h = 1.0 / (double)invh;
+  if constexpr (W == 1) {
+    // the a-nodes' part of the table position, floor and fraction (each
+    // thread's own records, as in the per-a loop)
+    for (int m = tid; m < Na; m += blockDim.x) {
+      float* cf = coef + ((size_t)c * Na + m) * NCOEF;
+      const double u = ((double)cf[FT_LNHI] + (double)cf[FT_LNLO] - (double)lo) * (double)invh;
+      const double f = ::floor(u);
+      cf[FT_Q] = __builtin_bit_cast(float, (int)f);
+      cf[FT_T] = (float)(u - f);
+    }
+  }
 
   using D1 = Dual<float, 1>;
   float ns;
