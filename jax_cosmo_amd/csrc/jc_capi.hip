@@ -1044,7 +1044,8 @@ int jc_dense_cholesky(jc_ctx* ctx, const double* cov, int64_t N, double* L, doub
   HIPCHK(ctx->dn_dlog.reserve((size_t)N));
   HIPCHK(ctx->dn_bad.reserve(1));
   HIPCHK(hipMemsetAsync(ctx->dn_bad.p, 0, sizeof(int), s));
-  HIPCHK(launch_dense_cholesky(A, N, ctx->dn_dlog.p, ctx->dn_bad.p, s));
+  HIPCHK(ctx->dn_inv.reserve((size_t)DENSE_PANEL * DENSE_PANEL));
+  HIPCHK(launch_dense_cholesky(A, N, ctx->dn_inv.p, ctx->dn_dlog.p, ctx->dn_bad.p, s));
   std::vector<double> dl((size_t)N);
   int bad = 0;
   HIPCHK(hipMemcpyAsync(dl.data(), ctx->dn_dlog.p, (size_t)N * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -1070,16 +1071,23 @@ int jc_dense_solve(jc_ctx* ctx, const double* L, int64_t N, const double* R, int
   const double* d_L = nullptr;
   int rc = to_device(ctx, ctx->dn_mat, L, (size_t)N * N, dev, &d_L);
   if (rc) return rc;
-  double* Z = X;
-  if (!dev) {
-    HIPCHK(ctx->dn_z.reserve(n));
-    Z = ctx->dn_z.p;
+  // the solves are out of place: from a copy of R into the result, and, for
+  // C^-1 R, through a second workspace
+  HIPCHK(ctx->dn_z.reserve(n));
+  HIPCHK(ctx->dn_inv.reserve(tri_inverse_size(N)));
+  if (!dev || mode == 2) HIPCHK(ctx->dn_x.reserve(n));
+  double* res = dev ? X : ctx->dn_x.p;
+  HIPCHK(hipMemcpyAsync(ctx->dn_z.p, R, n * sizeof(double), dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
+  HIPCHK(launch_tri_inverse(d_L, N, ctx->dn_inv.p, s));
+  if (mode == 2) {
+    HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_z.p, ctx->dn_x.p, nrhs, 0, s));
+    res = dev ? X : ctx->dn_z.p;
+    HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_x.p, res, nrhs, 1, s));
+  } else {
+    HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_z.p, res, nrhs, mode, s));
   }
-  if (Z != R) HIPCHK(hipMemcpyAsync(Z, R, n * sizeof(double), dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-  if (mode != 1) HIPCHK(launch_dense_solve(d_L, N, Z, nrhs, 0, s));
-  if (mode != 0) HIPCHK(launch_dense_solve(d_L, N, Z, nrhs, 1, s));
   if (!dev) {
-    HIPCHK(hipMemcpyAsync(X, Z, n * sizeof(double), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(X, res, n * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
   }
   return JC_OK;
@@ -1115,7 +1123,9 @@ int jc_gaussian_loglike_dense(jc_ctx* ctx, const float* mu, int64_t B, int64_t N
     d_ll = ctx->lk_out.p;
   }
   HIPCHK(ctx->dn_z.reserve(nmu));
-  HIPCHK(launch_dense_loglike(d_mu, B, N, d_data, d_L, c0, ctx->dn_z.p, d_ll, d_s, s));
+  HIPCHK(ctx->dn_x.reserve(nmu));
+  HIPCHK(ctx->dn_inv.reserve(tri_inverse_size(N)));
+  HIPCHK(launch_dense_loglike(d_mu, B, N, d_data, d_L, c0, ctx->dn_inv.p, ctx->dn_z.p, ctx->dn_x.p, d_ll, d_s, s));
   if (!dev) {
     HIPCHK(hipMemcpyAsync(loglike, d_ll, (size_t)B * sizeof(double), hipMemcpyDeviceToHost, s));
     if (dloglike_dmu) HIPCHK(hipMemcpyAsync(dloglike_dmu, d_s, nmu * sizeof(float), hipMemcpyDeviceToHost, s));
@@ -1154,6 +1164,8 @@ int jc_gaussian_loglike_grad_dense(jc_ctx* ctx, const double* cosmo, int64_t B, 
   HIPCHK(ctx->lk_mu.reserve(nmu));
   HIPCHK(ctx->lk_s.reserve(nmu));
   HIPCHK(ctx->dn_z.reserve(nmu));
+  HIPCHK(ctx->dn_x.reserve(nmu));
+  HIPCHK(ctx->dn_inv.reserve(tri_inverse_size(N)));
   double* d_ll = loglike;
   double* d_g = grad;
   if (!dev) {
@@ -1167,7 +1179,8 @@ int jc_gaussian_loglike_grad_dense(jc_ctx* ctx, const double* cosmo, int64_t B, 
   rc = run_pipeline(ctx, 0, d_cosmo, nullptr, B, set_id, d_ell, n_ell, n_z, ctx->lk_mu.p, nullptr, nullptr, nullptr,
                     JC_DEVICE_PTRS);
   if (rc) return rc;
-  HIPCHK(launch_dense_loglike(ctx->lk_mu.p, B, N, d_data, d_L, c0, ctx->dn_z.p, d_ll, ctx->lk_s.p, s));
+  HIPCHK(launch_dense_loglike(ctx->lk_mu.p, B, N, d_data, d_L, c0, ctx->dn_inv.p, ctx->dn_z.p, ctx->dn_x.p, d_ll,
+                              ctx->lk_s.p, s));
   rc = run_pipeline(ctx, 7, d_cosmo, nullptr, B, set_id, d_ell, n_ell, n_z, nullptr, nullptr, ctx->lk_s.p, d_g,
                     JC_DEVICE_PTRS);
   if (rc) return rc;

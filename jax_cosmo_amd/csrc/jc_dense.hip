@@ -1,21 +1,22 @@
 // Dense Gaussian likelihood algebra on the device (likelihood.py:43-61, the
 // covariance as one N x N matrix, N = pairs x ell: 5500 for 10 tracers and
 // 100 ell).  FP64 throughout, row-major N x N (numpy's layout; the matrix is
-// symmetric, so rows and columns are interchangeable on input).
+// symmetric, so rows and columns are interchangeable on input).  All products
+// run on the FP64 matrix cores (v_mfma_f64_16x16x4): a lane holds 4 consecutive
+// k of one row, so operands whose k is contiguous in memory come straight from
+// global memory as whole 128-byte segments, without LDS.
 //
-// Cholesky C = L L^T, right-looking in 64-column panels:
-//   k_potf2       the panel's 64 x 64 diagonal block, unblocked, in LDS; the
-//                 logarithms of its diagonal (log det C = 2 sum log L_ii) and
-//                 a flag for a non-positive pivot;
-//   k_trsm_panel  the panel below it, L21 = A21 L11^-T, one row per thread;
-//   k_syrk        the trailing lower triangle, A22 -= L21 L21^T, 64 x 64 tiles
-//                 (4 x 4 per thread) from LDS.  FP64 FMA issues at the rate
-//                 of the FP64 matrix cores on MI355X (78.6 TFLOP/s both), so
-//                 the update stays on the VALU.
+// Cholesky C = L L^T, right-looking in 64-column panels, two launches a panel:
+//   k_chol_panel  the panel below its 64 x 64 diagonal block, L21 = A21 L11^-T,
+//                 as a product with the block's inverse;
+//   k_chol_syrk   the trailing lower triangle, A22 -= L21 L21^T, 64 x 64 tiles;
+//                 its first block then factors and inverts the next panel's
+//                 diagonal block (chol64) beside the other tiles.
 // Triangular solves for B right-hand sides stored as rows ([B][N]), in
-// 64-row blocks: k_trsv_diag solves a block's triangle, k_solve_update
-// removes it from the remaining rows (z = L^-1 r forwards, y = L^-T z
-// backwards).
+// 256-row blocks whose triangles are inverted first, all at once
+// (k_tri_inv64, k_tri_merge): per block one product with its inverse
+// (k_solve_diag) and one that removes it from the remaining rows
+// (k_solve_update).
 // The likelihood of a batch of means: r = data - mu, z = L^-1 r,
 // -1/2 |z|^2 + c0 per mean (fixed-order sums), and its derivative with
 // respect to the mean, C^-1 r = L^-T z, the adjoint's cotangent.
@@ -25,118 +26,316 @@
 
 namespace jc {
 
-constexpr int DB = 64;  // panel width and tile size
+constexpr int DB = 64;              // panel width and tile size
+constexpr int SB = DENSE_SOLVE_BLOCK;  // rows a solve step takes
 
-__global__ __launch_bounds__(256) void k_potf2(double* __restrict__ A, int64_t N, int k0, double* __restrict__ dlog,
-                                               int* __restrict__ bad) {
-  __shared__ double S[DB][DB + 1];
-  const int nb = (int)min((int64_t)DB, N - k0);
-  for (int e = threadIdx.x; e < DB * DB; e += blockDim.x) {
-    const int i = e / DB, j = e - i * DB;
-    S[i][j] = (i < nb && j < nb && j <= i) ? A[(size_t)(k0 + i) * N + k0 + j] : 0.0;
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// (Kernels here ask for 2 waves per SIMD: with a budget above 256 registers the
+// compiler keeps accumulators in the accumulation file and copies them in and
+// out of every product's loop.)
+// D[i][j] += sum_k A[i][k] B[k][j] over 4 k: lane l passes A[l % 16][l / 16]
+// and B[l / 16][l % 16] and holds D[l / 16 + 4 r][l % 16] in register r
+__device__ __forceinline__ d4 mfma64(double a, double b, d4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Operands of 16 k: lane l takes k = 4 (l / 16) .. + 3 of row l % 16 (element q
+// of both operands in one instruction, so any assignment of k to lanes serves).
+// row: p[0 .. n) along k, n valid elements from the lane's first (n >= 4: all).
+__device__ __forceinline__ d4 frag_row(const double* p, int n) {
+  d4 v = {0.0, 0.0, 0.0, 0.0};
+  if (n >= 4) {
+    const d2u a = *reinterpret_cast<const d2u*>(p), b = *reinterpret_cast<const d2u*>(p + 2);
+    v[0] = a[0];
+    v[1] = a[1];
+    v[2] = b[0];
+    v[3] = b[1];
+  } else {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      if (q < n) v[q] = p[q];
   }
-  __syncthreads();
-  for (int j = 0; j < nb; ++j) {
-    if (threadIdx.x == 0) {
-      double d = S[j][j];
-      if (!(d > 0.0)) {
-        *bad = 1;
-        d = 1.0;  // keeps the rest finite; the caller reports the failure
+  return v;
+}
+// column: the elements are ld apart
+__device__ __forceinline__ d4 frag_col(const double* p, size_t ld, int n) {
+  d4 v = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (q < n) v[q] = p[q * ld];
+  return v;
+}
+__device__ __forceinline__ void mma16(const d4& a, const d4& b, d4& c) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) c = mfma64(a[q], b[q], c);
+}
+
+// n steps of 16 k with the operands of the next D in flight (a load from L
+// outside the L2 takes longer than a step's products): load(s, q) fills slot q
+// with step s, use(q) consumes it.  n is uniform over the wave.
+template <int D, class Load, class Use>
+__device__ __forceinline__ void pipelined(int n, Load&& load, Use&& use) {
+#pragma unroll
+  for (int q = 0; q < D; ++q)
+    if (q < n) load(q, q);
+  for (int s = 0; s < n; s += D) {
+#pragma unroll
+    for (int q = 0; q < D; ++q) {
+      if (s + q < n) {
+        use(q);
+        if (s + q + D < n) load(s + q + D, q);
       }
-      d = sqrt(d);
-      S[j][j] = d;
-      dlog[k0 + j] = log(d);
     }
-    __syncthreads();
-    const double id = 1.0 / S[j][j];
-    for (int i = j + 1 + threadIdx.x; i < nb; i += blockDim.x) S[i][j] *= id;
-    __syncthreads();
-    // trailing lower triangle of the block: (i, c) with j < c <= i
-    const int m = nb - j - 1;
-    for (int e = threadIdx.x; e < m * m; e += blockDim.x) {
-      const int i = j + 1 + e / m, c = j + 1 + e % m;
-      if (c <= i) S[i][c] -= S[i][j] * S[c][j];
-    }
-    __syncthreads();
-  }
-  for (int e = threadIdx.x; e < nb * nb; e += blockDim.x) {
-    const int i = e / nb, j = e - i * nb;
-    if (j <= i) A[(size_t)(k0 + i) * N + k0 + j] = S[i][j];
   }
 }
 
-// rows i >= k0 + 64: x = a L11^-T, i.e. x_j = (a_j - sum_{t<j} x_t L_jt) / L_jj
-__global__ __launch_bounds__(256) void k_trsm_panel(double* __restrict__ A, int64_t N, int k0) {
-  __shared__ double L11[DB][DB];
-  for (int e = threadIdx.x; e < DB * DB; e += blockDim.x) {
-    const int i = e / DB, j = e - i * DB;
-    L11[i][j] = (j <= i) ? A[(size_t)(k0 + i) * N + k0 + j] : 0.0;
+// ------------------------------------------------------------------ Cholesky
+constexpr int LS = DB + 2;  // LDS row stride of a 64 x 64 block
+
+__device__ __forceinline__ double lane_d(double x, int src) {  // src uniform
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, src);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), src);
+  return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+
+// 16 x 16 block product from LDS: acc += A B^T (NT: rows of B) or A B
+template <bool NT>
+__device__ __forceinline__ void lds_mma(const double* A, const double* B, int lane, d4& acc) {
+  const int i = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int k = 4 * q + g;
+    acc = mfma64(A[i * LS + k], NT ? B[i * LS + k] : B[k * LS + i], acc);
+  }
+}
+__device__ __forceinline__ void lds_put(double* D, int lane, const d4& v) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) D[((lane >> 4) + 4 * r) * LS + (lane & 15)] = v[r];
+}
+
+// sqrt(d) and its reciprocal for normal d > 0, by Newton from v_rsq_f64
+__device__ __forceinline__ double sqrt_rsqrt(double d, double& r) {
+  double y = __builtin_amdgcn_rsq(d);
+  y = __builtin_fma(0.5 * y, __builtin_fma(-d * y, y, 1.0), y);
+  y = __builtin_fma(0.5 * y, __builtin_fma(-d * y, y, 1.0), y);
+  r = y;
+  const double s = d * y;
+  return __builtin_fma(0.5 * y, __builtin_fma(-s, s, d), s);
+}
+
+// V (lower triangle by 16 x 16 blocks) = the inverse of the lower triangular
+// 64 x 64 block in S, by the 256 threads of a block: wave w substitutes its
+// 16 x 16 diagonal block (column i in lane i), then
+// V21 = -V22 (S21 V11), 16 and 32 wide.
+__device__ void tri64_inverse(const double* S, double* V) {
+  double* Tm = V + 32;  // rows 0-31, columns 32-63: above the inverse's diagonal, not part of it
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  {
+    const int o = 16 * wave, i = lane & 15;
+    const double* L = S + o * LS + o;
+    double x[16];
+    const double rd = 1.0 / L[i * LS + i];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      double s0 = i == r ? 1.0 : 0.0, s1 = 0.0;
+#pragma unroll
+      for (int t = 0; t < r; ++t) {
+        if (t & 1) s1 -= L[r * LS + t] * x[t];
+        else s0 -= L[r * LS + t] * x[t];
+      }
+      x[r] = (s0 + s1) * lane_d(rd, r);
+    }
+    if (lane < 16) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) V[(o + r) * LS + o + i] = x[r];
+    }
   }
   __syncthreads();
-  const int64_t i = (int64_t)k0 + DB + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  double* row = A + (size_t)i * N + k0;
-  double x[DB];
+  const d4 zero = {0.0, 0.0, 0.0, 0.0};
+  if (wave < 2) {
+    const int o = 32 * wave;
+    d4 v = zero;
+    lds_mma<false>(S + (o + 16) * LS + o, V + o * LS + o, lane, v);
+    lds_put(Tm + 16 * wave * LS, lane, v);
+  }
+  __syncthreads();
+  if (wave < 2) {
+    const int o = 32 * wave;
+    d4 v = zero;
+    lds_mma<false>(V + (o + 16) * LS + o + 16, Tm + 16 * wave * LS, lane, v);
+    lds_put(V + (o + 16) * LS + o, lane, -v);
+  }
+  __syncthreads();
+  // 32 wide: the blocks above V's diagonal inside its halves are not stored
+  const int ra = 16 * (wave >> 1), cb = 16 * (wave & 1);
+  d4 t = zero;
+  for (int c = cb; c < 32; c += 16) lds_mma<false>(S + (32 + ra) * LS + c, V + c * LS + cb, lane, t);
+  __syncthreads();  // the 16-wide Tm has been read
+  lds_put(Tm + ra * LS + cb, lane, t);
+  __syncthreads();
+  t = zero;
+  for (int c = 0; c <= ra; c += 16) lds_mma<false>(V + (32 + ra) * LS + 32 + c, Tm + c * LS + cb, lane, t);
+  lds_put(V + (32 + ra) * LS + cb, lane, -t);
+  __syncthreads();
+}
+
+// Factors the 64 x 64 block in S (lower triangle; identity past nb) in place
+// and leaves the inverse of its factor in the lower triangle (by 16 x 16
+// blocks) of V, by the 256 threads of a block.  16 columns at a time: one wave
+// factors them down all rows of the block (row o + i in lane i, so the rows
+// below the diagonal come with it; pivots and multipliers by readlane, no
+// barrier), then all waves update the rest as 16 x 16 products.
+// A chain of 64 pivots with barriers between them took 97 us.
+__device__ void chol64(double* S, double* V, int nb, double* dlog, int* bad) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __syncthreads();  // the caller has written S
+  for (int jb = 0; jb < 4; ++jb) {
+    const int o = 16 * jb;
+    if (wave == 0) {
+      double* row = S + min(o + lane, DB - 1) * LS + o;
+      double a[16];
 #pragma unroll
-  for (int t = 0; t < DB; ++t) x[t] = row[t];
+      for (int c = 0; c < 16; ++c) a[c] = row[c];
+      double dg = 1.0;
+      bool ok = true;
 #pragma unroll
-  for (int j = 0; j < DB; ++j) {
-    double s = x[j];
+      for (int j = 0; j < 16; ++j) {
+        const double p = lane_d(a[j], j);
+        ok = ok && p > 0.0;
+        const double d = p > 0.0 ? p : 1.0;  // keeps the rest finite; the caller reports the failure
+        double r;
+        const double s = sqrt_rsqrt(d, r);
+        dg = lane == j ? s : dg;
+        a[j] = lane == j ? s : a[j] * r;
 #pragma unroll
-    for (int t = 0; t < j; ++t) s -= x[t] * L11[j][t];
-    x[j] = s / L11[j][j];
+        for (int c = j + 1; c < 16; ++c) a[c] -= a[j] * lane_d(a[j], c);
+      }
+      if (o + lane < DB) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) row[c] = lane >= c ? a[c] : 0.0;
+      }
+      if (lane < 16 && o + lane < nb) dlog[o + lane] = ::log(dg);
+      if (!ok && lane == 0) *bad = 1;
+    }
+    __syncthreads();
+    int t = 0;
+    for (int ib = jb + 1; ib < 4; ++ib)
+      for (int kb = jb + 1; kb <= ib; ++kb, ++t) {
+        if ((t & 3) != wave) continue;
+        d4 v = {0.0, 0.0, 0.0, 0.0};
+        lds_mma<true>(S + 16 * ib * LS + o, S + 16 * kb * LS + o, lane, v);
+        double* D = S + 16 * ib * LS + 16 * kb;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) D[((lane >> 4) + 4 * r) * LS + (lane & 15)] -= v[r];
+      }
+    __syncthreads();
+  }
+  tri64_inverse(S, V);
+}
+
+// the diagonal block in S (written by the caller) -> factor in A, inverse in inv
+__device__ __forceinline__ void chol64_store(double* A, int64_t N, int64_t k0, double* S, double* V, double* inv,
+                                             double* dlog, int* bad) {
+  const int nb = (int)min((int64_t)DB, N - k0);
+  chol64(S, V, nb, dlog + k0, bad);
+  for (int e = threadIdx.x; e < DB * DB; e += 256) {
+    const int i = e / DB, j = e - i * DB;
+    if (j <= i && i < nb) A[(size_t)(k0 + i) * N + k0 + j] = S[i * LS + j];
+    inv[e] = V[i * LS + j];
+  }
+}
+
+__global__ __launch_bounds__(256, 2) void k_chol_first(double* __restrict__ A, int64_t N, double* __restrict__ inv,
+                                                     double* __restrict__ dlog, int* __restrict__ bad) {
+  __shared__ double S[DB * LS], V[DB * LS];
+  const int nb = (int)min((int64_t)DB, N);
+  for (int e = threadIdx.x; e < DB * DB; e += 256) {
+    const int i = e / DB, j = e - i * DB;
+    S[i * LS + j] = i < nb && j <= i ? A[(size_t)i * N + j] : (i == j ? 1.0 : 0.0);
+  }
+  chol64_store(A, N, 0, S, V, inv, dlog, bad);
+}
+
+// rows i >= k0 + 64: x = a L11^-T, 16 rows a wave (which reads its rows' 64
+// columns before it writes them)
+__global__ __launch_bounds__(256, 2) void k_chol_panel(double* __restrict__ A, int64_t N, int64_t k0,
+                                                     const double* __restrict__ inv) {
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int64_t r0 = k0 + DB + ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
+  if (r0 >= N) return;
+  const double* row = A + (size_t)min(r0 + i, N - 1) * N + k0 + 4 * g;
+  d4 a[4], acc[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) a[s] = frag_row(row + 16 * s, 4);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    acc[c] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s <= c; ++s) mma16(a[s], frag_row(inv + (16 * c + i) * DB + 16 * s + 4 * g, 4), acc[c]);
   }
 #pragma unroll
-  for (int t = 0; t < DB; ++t) row[t] = x[t];
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (r0 + g + 4 * r < N) A[(size_t)(r0 + g + 4 * r) * N + k0 + 16 * c + i] = acc[c][r];
 }
 
 // trailing update of the lower triangle from row/column r0 = k0 + 64: tile
-// (ti, tj), tj <= ti, of 64 x 64; thread (tr, tc) owns rows 4 tr .. 4 tr + 3
-// and columns 4 tc .. 4 tc + 3 of the tile
-__global__ __launch_bounds__(256) void k_syrk(double* __restrict__ A, int64_t N, int k0) {
-  __shared__ double Pi[DB][DB + 2];  // [t][row of tile i]
-  __shared__ double Pj[DB][DB + 2];  // [t][row of tile j]
-  const int64_t r0 = (int64_t)k0 + DB;
+// (ti, tj), tj <= ti, of 64 x 64, 32 x 32 a wave; block 0 (the next panel's
+// diagonal block) goes on to factor it
+__global__ __launch_bounds__(256, 2) void k_chol_syrk(double* __restrict__ A, int64_t N, int64_t k0,
+                                                    double* __restrict__ inv, double* __restrict__ dlog,
+                                                    int* __restrict__ bad) {
+  __shared__ double S[DB * LS], V[DB * LS];
+  const int64_t r0 = k0 + DB;
   const int64_t idx = blockIdx.x;
   int64_t ti = (int64_t)((sqrt(8.0 * (double)idx + 1.0) - 1.0) * 0.5);
   while (ti * (ti + 1) / 2 > idx) --ti;
   while ((ti + 1) * (ti + 2) / 2 <= idx) ++ti;
   const int64_t tj = idx - ti * (ti + 1) / 2;
-  const int64_t ri = r0 + ti * DB, rj = r0 + tj * DB;
-  for (int e = threadIdx.x; e < DB * DB; e += blockDim.x) {
-    const int r = e / DB, t = e - r * DB;
-    Pi[t][r] = (ri + r < N) ? A[(size_t)(ri + r) * N + k0 + t] : 0.0;
-    Pj[t][r] = (rj + r < N) ? A[(size_t)(rj + r) * N + k0 + t] : 0.0;
-  }
-  __syncthreads();
-  const int tr = threadIdx.x >> 4, tc = threadIdx.x & 15;
-  double acc[4][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int64_t ri = r0 + ti * DB + 32 * (wave >> 1), rj = r0 + tj * DB + 32 * (wave & 1);
+  d4 acc[2][2];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-#pragma unroll 8
-  for (int t = 0; t < DB; ++t) {
-    const double2 a01 = *reinterpret_cast<const double2*>(&Pi[t][tr * 4]);
-    const double2 a23 = *reinterpret_cast<const double2*>(&Pi[t][tr * 4 + 2]);
-    const double2 b01 = *reinterpret_cast<const double2*>(&Pj[t][tc * 4]);
-    const double2 b23 = *reinterpret_cast<const double2*>(&Pj[t][tc * 4 + 2]);
-    const double av[4] = {a01.x, a01.y, a23.x, a23.y}, bv[4] = {b01.x, b01.y, b23.x, b23.y};
+    for (int b = 0; b < 2; ++b) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
+  const double* pa[2];
+  const double* pb[2];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] += av[a] * bv[b];
+  for (int a = 0; a < 2; ++a) {
+    pa[a] = A + (size_t)min(ri + 16 * a + i, N - 1) * N + k0 + 4 * g;
+    pb[a] = A + (size_t)min(rj + 16 * a + i, N - 1) * N + k0 + 4 * g;
   }
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const int64_t row = ri + tr * 4 + a;
-    if (row >= N) continue;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int64_t col = rj + tc * 4 + b;
-      if (col <= row && col < N) A[(size_t)row * N + col] -= acc[a][b];
-    }
+  for (int s = 0; s < 4; ++s) {
+    const d4 a0 = frag_row(pa[0] + 16 * s, 4), a1 = frag_row(pa[1] + 16 * s, 4);
+    const d4 b0 = frag_row(pb[0] + 16 * s, 4), b1 = frag_row(pb[1] + 16 * s, 4);
+    mma16(a0, b0, acc[0][0]);
+    mma16(a0, b1, acc[0][1]);
+    mma16(a1, b0, acc[1][0]);
+    mma16(a1, b1, acc[1][1]);
   }
+  const int nb = (int)min((int64_t)DB, N - r0);
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t row = ri + 16 * a + g + 4 * r, col = rj + 16 * b + i;
+        if (idx == 0) {
+          const int x = (int)(row - r0), y = (int)(col - r0);
+          S[x * LS + y] = x < nb && y <= x ? A[(size_t)row * N + col] - acc[a][b][r] : (x == y ? 1.0 : 0.0);
+        } else if (col <= row && row < N) {
+          A[(size_t)row * N + col] -= acc[a][b][r];
+        }
+      }
+  if (idx != 0) return;  // uniform over the block
+  chol64_store(A, N, r0, S, V, inv, dlog, bad);
 }
 
 // the strict upper triangle of the factor is zeroed at the end
@@ -146,96 +345,165 @@ __global__ void k_zero_upper(double* __restrict__ A, int64_t N) {
     A[(size_t)row * N + c] = 0.0;
 }
 
-// Triangular solves for B right-hand sides stored as rows of Z ([B][N]), in
-// 64-row blocks.  For each block: solve its triangle for every right-hand
-// side (k_trsv_diag), then remove the solved block from the rows still to
-// come (k_solve_update).
-//   forward (z = L^-1 r):    rows after the block, z_i -= sum_t L[i][k0+t] z_{k0+t}
-//   transpose (y = L^-T z):  rows before the block, y_i -= sum_t L[k0+t][i] y_{k0+t}
-// k_trsv_diag: the block's 64 x 64 triangle staged in LDS once per four
-// right-hand sides; one wave per right-hand side, lane i holding row k0 + i,
-// the solved value of step j passed to the other lanes by a shuffle (no
-// barriers inside the solve).
-__global__ __launch_bounds__(256) void k_trsv_diag(const double* __restrict__ L, int64_t N, int k0, int transpose,
-                                                   int64_t B, double* __restrict__ Z) {
-  __shared__ double T[DB][DB + 1];
-  const int nb = (int)min((int64_t)DB, N - k0);
-  for (int e = threadIdx.x; e < DB * DB; e += blockDim.x) {
+// ------------------------------------------------------------------ triangular solves
+// Inverses of the SB x SB diagonal blocks of L, one block after another in
+// inv ([ceil(N / SB)][SB][SB], row-major; rows past N count as identity; the
+// 64 x 64 sub-blocks above the diagonal are not written).  The forward error
+// of a product with a triangle's inverse has the bound of substitution,
+// |L^-1| |L| |x|, and the 64 divisions and broadcasts a substitution chains
+// per block are gone.
+// k_tri_inv64: the 64 x 64 diagonal blocks.
+__global__ __launch_bounds__(256, 2) void k_tri_inv64(const double* __restrict__ L, int64_t N, double* __restrict__ inv) {
+  __shared__ double S[DB * LS], V[DB * LS];
+  const int64_t k0 = (int64_t)blockIdx.x * DB;
+  for (int e = threadIdx.x; e < DB * DB; e += 256) {
     const int r = e / DB, c = e - r * DB;
-    T[r][c] = (r < nb && c < nb && c <= r) ? L[(size_t)(k0 + r) * N + k0 + c] : 0.0;
+    S[r * LS + c] = k0 + r < N && c <= r ? L[(size_t)(k0 + r) * N + k0 + c] : (r == c ? 1.0 : 0.0);
   }
   __syncthreads();
-  const int i = threadIdx.x & 63;
-  const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (b >= B) return;  // after the block's only barrier
-  double* z = Z + (size_t)b * N;
-  double s = i < nb ? z[k0 + i] : 0.0;  // rows past nb stay zero (their T entries are zero)
-  if (!transpose) {
-    for (int j = 0; j < nb; ++j) {
-      const double zj = __shfl(s, j, 64) / T[j][j];
-      if (i == j) s = zj;
-      else if (i > j) s -= T[i][j] * zj;
-    }
-  } else {
-    for (int j = nb - 1; j >= 0; --j) {
-      const double zj = __shfl(s, j, 64) / T[j][j];
-      if (i == j) s = zj;
-      else if (i < j) s -= T[j][i] * zj;
-    }
+  tri64_inverse(S, V);
+  double* o = inv + (size_t)(blockIdx.x / (SB / DB)) * SB * SB + (size_t)(blockIdx.x % (SB / DB)) * DB * (SB + 1);
+  for (int e = threadIdx.x; e < DB * DB; e += 256) {
+    const int r = e / DB, c = e - r * DB;
+    o[(size_t)r * SB + c] = c / 16 <= r / 16 ? V[r * LS + c] : 0.0;
   }
-  if (i < nb) z[k0 + i] = s;
 }
 
-// k_solve_update: rows r of the tile (64 per block, grid x) and 16
-// right-hand sides (grid y); thread (row r = t % 64, group g = t / 64)
-// updates 4 right-hand sides from the 64 x 64 tile of L and the solved
-// values in LDS.  (Measured: 64 right-hand sides per block with 4 x 4 per
-// thread ran 25 us per step against 19 for this form, fewer blocks in
-// flight at the small trailing sizes.)
-constexpr int SU_R = 16;  // right-hand sides per update block
+// k_tri_merge: two inverted neighbours of H rows to one of 2 H:
+// inv21 = -inv22 (L21 inv11), 32 columns per block (grid y), 16 rows a wave.
+constexpr int MS = 34;  // LDS row stride of the [H][32] product
 
-__global__ __launch_bounds__(256) void k_solve_update(const double* __restrict__ L, int64_t N, int k0, int transpose,
-                                                      int64_t B, double* __restrict__ Z) {
-  __shared__ double Lt[DB][DB + 1];   // [t][r]: the coupling of row r to solved row k0 + t
-  __shared__ double zs[SU_R][DB];     // solved values of the block's right-hand sides
-  const int nb = (int)min((int64_t)DB, N - k0);
-  // the rows this block updates: after the block (forward) or before it (transpose)
-  const int64_t row0 = transpose ? (int64_t)blockIdx.x * DB : (int64_t)k0 + DB + (int64_t)blockIdx.x * DB;
-  const int64_t row_end = transpose ? (int64_t)k0 : N;
-  const int64_t b0 = (int64_t)blockIdx.y * SU_R;
-  const int t = threadIdx.x;
-  for (int e = t; e < DB * DB; e += 256) {
-    const int x = e / DB, y = e - x * DB;
-    double v = 0.0;
-    if (!transpose) {
-      // x = row offset, y = t: L[row0 + x][k0 + y] (coalesced in y)
-      if (row0 + x < row_end && y < nb) v = L[(size_t)(row0 + x) * N + k0 + y];
-      Lt[y][x] = v;
-    } else {
-      // x = t, y = row offset: L[k0 + x][row0 + y] (coalesced in y)
-      if (x < nb && row0 + y < row_end) v = L[(size_t)(k0 + x) * N + row0 + y];
-      Lt[x][y] = v;
-    }
+template <int H>
+__global__ __launch_bounds__(4 * H, 2) void k_tri_merge(const double* __restrict__ L, int64_t N, double* __restrict__ inv) {
+  __shared__ double tm[H * MS];
+  constexpr int per = SB / (2 * H);
+  const int64_t k0 = (int64_t)blockIdx.x * 2 * H;
+  double* V = inv + (size_t)(blockIdx.x / per) * SB * SB + (size_t)(blockIdx.x % per) * 2 * H * (SB + 1);
+  const int j0 = blockIdx.y * 32;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
+  const int w0 = wave * 16;
+  const int64_t lrow = k0 + H + w0 + i;  // rows past N: zero (their columns lie below N)
+  d4 c0 = {0.0, 0.0, 0.0, 0.0}, c1 = c0;
+  for (int k = j0; k < H; k += 16) {  // inv11 has no rows above its column
+    const double* v = V + (size_t)(k + 4 * g) * SB + j0 + i;
+    const d4 x = lrow < N ? frag_row(L + (size_t)lrow * N + k0 + k + 4 * g, 4) : d4{0.0, 0.0, 0.0, 0.0};
+    mma16(x, frag_col(v, SB, 4), c0);
+    mma16(x, frag_col(v + 16, SB, 4), c1);
   }
-  for (int e = t; e < SU_R * DB; e += 256) {
-    const int q = e / DB, c = e - q * DB;
-    zs[q][c] = (b0 + q < B && c < nb) ? Z[(size_t)(b0 + q) * N + k0 + c] : 0.0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    tm[(w0 + g + 4 * r) * MS + i] = c0[r];
+    tm[(w0 + g + 4 * r) * MS + 16 + i] = c1[r];
   }
   __syncthreads();
-  const int r = t & (DB - 1), g = t >> 6;  // 4 groups of 4 right-hand sides
-  const int64_t row = row0 + r;
-  if (row >= row_end) return;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int c = 0; c < nb; ++c) {
-    const double l = Lt[c][r];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] += l * zs[g * 4 + q][c];
+  c0 = c1 = d4{0.0, 0.0, 0.0, 0.0};
+  for (int k = 0; k <= w0; k += 16) {
+    const d4 x = frag_row(V + (size_t)(H + w0 + i) * SB + H + k + 4 * g, 4);
+    const double* t = tm + (k + 4 * g) * MS + i;
+    mma16(x, frag_col(t, MS, 4), c0);
+    mma16(x, frag_col(t + 16, MS, 4), c1);
   }
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int64_t bb = b0 + g * 4 + q;
-    if (bb < B) Z[(size_t)bb * N + row] -= acc[q];
+  for (int r = 0; r < 4; ++r) {
+    double* o = V + (size_t)(H + w0 + g + 4 * r) * SB + j0 + i;
+    o[0] = -c0[r];
+    o[16] = -c1[r];
   }
+}
+
+// k_solve_diag: x_k = inv_k r_k (TR: with inv_k's transpose) for the block's
+// rows, 64 rows (grid y) of 16 right-hand sides per workgroup, 16 rows a wave;
+// R [B][N] what is left of the right-hand sides, X [B][N] the solution.
+template <bool TR>
+__global__ __launch_bounds__(256, 2) void k_solve_diag(const double* __restrict__ inv, int64_t N, int64_t k0, int64_t B,
+                                                     const double* __restrict__ R, double* __restrict__ X) {
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int w0 = 64 * blockIdx.y + 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nb = (int)min((int64_t)SB, N - k0);
+  if (w0 >= nb) return;
+  const int64_t b0 = (int64_t)blockIdx.x * 16;
+  const double* V = inv + (size_t)(k0 / SB) * SB * SB;
+  const double* r = R + (size_t)min(b0 + i, B - 1) * N + k0 + 4 * g;
+  const int row = w0 + i;
+  const int kb = TR ? w0 : 0;
+  const int ke = min((nb + 15) & ~15, TR ? SB : w0 + 16);
+  constexpr int D = 4;
+  d4 acc = {0.0, 0.0, 0.0, 0.0}, x[D], v[D];
+  auto load = [&](int s, int q, int left) {  // left: columns from the lane's first on (4: all)
+    const int k = kb + 16 * s;
+    x[q] = frag_row(r + k, left);
+    v[q] = TR ? frag_col(V + (size_t)(k + 4 * g) * SB + row, SB, 4) : frag_row(V + (size_t)row * SB + k + 4 * g, 4);
+  };
+  auto use = [&](int q) { mma16(x[q], v[q], acc); };
+  const int n = (ke - kb) / 16;
+  if (nb == SB) pipelined<D>(n, [&](int s, int q) { load(s, q, 4); }, use);
+  else pipelined<D>(n, [&](int s, int q) { load(s, q, nb - (kb + 16 * s) - 4 * g); }, use);
+  if (row >= nb) return;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (b0 + g + 4 * q < B) X[(size_t)(b0 + g + 4 * q) * N + k0 + row] = acc[q];
+}
+
+// k_solve_update: removes the solved block from the rows still to come
+// (forward: after it, r_i -= sum_t L[i][k0+t] x_{k0+t}; TR: before it,
+// r_i -= sum_t L[k0+t][i] x_{k0+t}).  A workgroup takes WR x 32 rows x 64
+// right-hand sides, a wave 16 WR x 32 right-hand sides.  What bounds it is the
+// L2: L and x cross it once per 64 right-hand sides and once per WR x 32 rows,
+// so the wide tile is used while there are enough of them to fill the chip, and
+// workgroups are numbered so that one XCD's L2 holds the same rows of L for all
+// right-hand sides.
+template <bool TR, int WR>
+__global__ __launch_bounds__(256, 2) void k_solve_update(const double* __restrict__ L, int64_t N, int64_t k0, int64_t B,
+                                                      int gy, const double* __restrict__ X, double* __restrict__ R) {
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nb = (int)min((int64_t)SB, N - k0);
+  const int n = gridDim.x, q8 = n >> 3, r8 = n & 7, xc = blockIdx.x & 7;  // block b runs on XCD b % 8
+  const int id = xc * q8 + min(xc, r8) + (blockIdx.x >> 3);
+  const int64_t row0 = (TR ? 0 : k0 + SB) + (int64_t)(id / gy) * (32 * WR) + 16 * WR * (wave & 1);
+  const int64_t row_end = TR ? k0 : N;
+  const int64_t b0 = (int64_t)(id % gy) * 64 + 32 * (wave >> 1);
+  if (b0 >= B || row0 >= row_end) return;
+  const double* x[2];
+  int64_t rw[WR];
+#pragma unroll
+  for (int a = 0; a < 2; ++a) x[a] = X + (size_t)min(b0 + 16 * a + i, B - 1) * N + k0;
+#pragma unroll
+  for (int c = 0; c < WR; ++c) rw[c] = min(row0 + 16 * c + i, row_end - 1);
+  d4 acc[2][WR];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int c = 0; c < WR; ++c) acc[a][c] = d4{0.0, 0.0, 0.0, 0.0};
+  constexpr int D = 3;
+  d4 xv[D][2], lv[D][WR];
+  auto load = [&](int s, int q, int left) {  // left: columns from the lane's first on (4: all)
+    const int kk = 16 * s + 4 * g;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) xv[q][a] = frag_row(x[a] + kk, left);
+#pragma unroll
+    for (int c = 0; c < WR; ++c)
+      lv[q][c] = TR ? frag_col(L + (size_t)(k0 + kk) * N + rw[c], N, left)
+                    : frag_row(L + (size_t)rw[c] * N + k0 + kk, left);
+  };
+  auto use = [&](int q) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int c = 0; c < WR; ++c) mma16(xv[q][a], lv[q][c], acc[a][c]);
+  };
+  if (nb == SB) pipelined<D>(SB / 16, [&](int s, int q) { load(s, q, 4); }, use);
+  else pipelined<D>((nb + 15) / 16, [&](int s, int q) { load(s, q, nb - 16 * s - 4 * g); }, use);
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int64_t b = b0 + 16 * a + g + 4 * q;
+      if (b >= B) continue;
+#pragma unroll
+      for (int c = 0; c < WR; ++c)
+        if (row0 + 16 * c + i < row_end) R[(size_t)b * N + row0 + 16 * c + i] -= acc[a][c][q];
+    }
 }
 
 // r = data - mu (FP64), [B][N]
@@ -266,16 +534,13 @@ __global__ void k_to_float(const double* __restrict__ x, int64_t n, float* __res
   if (e < n) y[e] = (float)x[e];
 }
 
-hipError_t launch_dense_cholesky(double* A, int64_t N, double* dlog, int* bad, hipStream_t s) {
+hipError_t launch_dense_cholesky(double* A, int64_t N, double* inv, double* dlog, int* bad, hipStream_t s) {
   if (N < 1) return hipErrorInvalidValue;
-  for (int64_t k0 = 0; k0 < N; k0 += DB) {
-    hipLaunchKernelGGL(k_potf2, dim3(1), dim3(256), 0, s, A, N, (int)k0, dlog, bad);
-    const int64_t rest = N - k0 - DB;
-    if (rest > 0) {
-      hipLaunchKernelGGL(k_trsm_panel, dim3((unsigned)((rest + 255) / 256)), dim3(256), 0, s, A, N, (int)k0);
-      const int64_t T = (rest + DB - 1) / DB;
-      hipLaunchKernelGGL(k_syrk, dim3((unsigned)(T * (T + 1) / 2)), dim3(256), 0, s, A, N, (int)k0);
-    }
+  hipLaunchKernelGGL(k_chol_first, dim3(1), dim3(256), 0, s, A, N, inv, dlog, bad);
+  for (int64_t k0 = 0; N - k0 > DB; k0 += DB) {
+    const int64_t rest = N - k0 - DB, T = (rest + DB - 1) / DB;
+    hipLaunchKernelGGL(k_chol_panel, dim3((unsigned)T), dim3(256), 0, s, A, N, k0, inv);
+    hipLaunchKernelGGL(k_chol_syrk, dim3((unsigned)(T * (T + 1) / 2)), dim3(256), 0, s, A, N, k0, inv, dlog, bad);
   }
   hipLaunchKernelGGL(k_zero_upper, dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((N + 255) / 256, 64)),
                                          (unsigned)N),
@@ -283,30 +548,53 @@ hipError_t launch_dense_cholesky(double* A, int64_t N, double* dlog, int* bad, h
   return hipGetLastError();
 }
 
-hipError_t launch_dense_solve(const double* L, int64_t N, double* Z, int64_t B, int transpose, hipStream_t s) {
-  if (N < 1 || B < 1) return hipErrorInvalidValue;
-  const unsigned gy = (unsigned)((B + SU_R - 1) / SU_R);
-  const int64_t last = (N - 1) / DB * DB;
-  for (int64_t step = 0; step <= last; step += DB) {
-    const int64_t k0 = transpose ? last - step : step;
-    hipLaunchKernelGGL(k_trsv_diag, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, L, N, (int)k0, transpose, B, Z);
-    const int64_t rows = transpose ? k0 : N - k0 - DB;
-    if (rows > 0)
-      hipLaunchKernelGGL(k_solve_update, dim3((unsigned)((rows + DB - 1) / DB), gy), dim3(256), 0, s, L, N, (int)k0,
-                         transpose, B, Z);
+hipError_t launch_tri_inverse(const double* L, int64_t N, double* inv, hipStream_t s) {
+  if (N < 1) return hipErrorInvalidValue;
+  // whole SB blocks: the merges of a partial last block read identity rows
+  const int64_t ns = (N + SB - 1) / SB;
+  hipLaunchKernelGGL(k_tri_inv64, dim3((unsigned)(ns * (SB / DB))), dim3(256), 0, s, L, N, inv);
+  static_assert(SB == 256, "the merges go 64 -> 128 -> 256");
+  if (N > 64) hipLaunchKernelGGL((k_tri_merge<64>), dim3((unsigned)(ns * 2), 2), dim3(256), 0, s, L, N, inv);
+  if (N > 128) hipLaunchKernelGGL((k_tri_merge<128>), dim3((unsigned)ns, 4), dim3(512), 0, s, L, N, inv);
+  return hipGetLastError();
+}
+
+template <bool TR>
+static void solve_pass(const double* L, int64_t N, const double* inv, double* R, double* X, int64_t B, hipStream_t s) {
+  const int gy = (int)((B + 63) / 64);
+  const int64_t last = (N - 1) / SB * SB;
+  for (int64_t step = 0; step <= last; step += SB) {
+    const int64_t k0 = TR ? last - step : step;
+    const int64_t nb = std::min<int64_t>(SB, N - k0), rows = TR ? k0 : N - k0 - SB;
+    const dim3 gd((unsigned)((B + 15) / 16), (unsigned)((nb + 63) / 64));
+    hipLaunchKernelGGL((k_solve_diag<TR>), gd, dim3(256), 0, s, inv, N, k0, B, R, X);
+    if (rows <= 0) continue;
+    const int64_t wide = (rows + 63) / 64 * gy, narrow = (rows + 31) / 32 * gy;
+    if (wide >= 256)
+      hipLaunchKernelGGL((k_solve_update<TR, 2>), dim3((unsigned)wide), dim3(256), 0, s, L, N, k0, B, gy, X, R);
+    else
+      hipLaunchKernelGGL((k_solve_update<TR, 1>), dim3((unsigned)narrow), dim3(256), 0, s, L, N, k0, B, gy, X, R);
   }
+}
+
+hipError_t launch_dense_solve(const double* L, int64_t N, const double* inv, double* R, double* X, int64_t B,
+                              int transpose, hipStream_t s) {
+  if (N < 1 || B < 1 || R == X) return hipErrorInvalidValue;
+  if (transpose) solve_pass<true>(L, N, inv, R, X, B, s);
+  else solve_pass<false>(L, N, inv, R, X, B, s);
   return hipGetLastError();
 }
 
 hipError_t launch_dense_loglike(const float* mu, int64_t B, int64_t N, const double* data, const double* L, double c0,
-                                double* Z, double* loglike, float* dmu, hipStream_t s) {
+                                double* inv, double* Z, double* X, double* loglike, float* dmu, hipStream_t s) {
   const int64_t n = B * N;
-  hipLaunchKernelGGL(k_resid, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, mu, data, N, B, Z);
-  hipError_t e = launch_dense_solve(L, N, Z, B, 0, s);
+  hipError_t e = launch_tri_inverse(L, N, inv, s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_sq_sum, dim3((unsigned)B), dim3(256), 0, s, Z, N, c0, loglike);
+  hipLaunchKernelGGL(k_resid, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, mu, data, N, B, Z);
+  if ((e = launch_dense_solve(L, N, inv, Z, X, B, 0, s)) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_sq_sum, dim3((unsigned)B), dim3(256), 0, s, X, N, c0, loglike);
   if (dmu) {
-    if ((e = launch_dense_solve(L, N, Z, B, 1, s)) != hipSuccess) return e;
+    if ((e = launch_dense_solve(L, N, inv, X, Z, B, 1, s)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_to_float, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, Z, n, dmu);
   }
   return hipGetLastError();
