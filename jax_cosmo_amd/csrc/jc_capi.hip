@@ -55,6 +55,8 @@ std::vector<double> logspace(double a, double b, int n) {
   return v;
 }
 
+constexpr double PI_D = 3.141592653589793;
+
 int ctx_init_tables(jc_ctx* ctx) {
   hipStream_t s = ctx->stream;
   ctx->atab_chi_h = logspace(-3.0, 0.0, NCHI);  // background.py:225
@@ -85,14 +87,21 @@ int ctx_init_tables(jc_ctx* ctx) {
     }
   }
   HIPCHK(ctx->hf_lnk.upload(lnk, s));
-  HIPCHK(ctx->hf_w.upload(w, s));
   HIPCHK(ctx->logr.upload(logr, s));
   HIPCHK(ctx->hf_E.upload(E, s));
   HIPCHK(ctx->hf_k32.upload(k32, s));
   HIPCHK(ctx->hf_kp.upload(kp, s));
-  std::vector<double> kd(NHF_K);
-  for (int i = 0; i < NHF_K; ++i) kd[i] = exp(lnk[i]);
-  HIPCHK(ctx->hf_kd.upload(kd, s));
+  std::vector<double> hn((size_t)NHF_K * 4), r2(NHF_R);
+  for (int i = 0; i < NHF_K; ++i) {
+    const double k = exp(lnk[i]);
+    hn[(size_t)i * 4] = k;
+    hn[(size_t)i * 4 + 1] = 1.0 / k;
+    hn[(size_t)i * 4 + 2] = lnk[i];
+    hn[(size_t)i * 4 + 3] = w[i] * (k * k * k) / (2.0 * PI_D * PI_D);
+  }
+  for (int j = 0; j < NHF_R; ++j) r2[j] = exp(logr[j]) * exp(logr[j]);
+  HIPCHK(ctx->hf_nodes.upload(hn, s));
+  HIPCHK(ctx->hf_R2.upload(r2, s));
   // chi table nodes: RK4 in t = ln a with midpoints t_{i-1} + h/2
   // (background.py:223-233, scipy/ode.py:6-22)
   std::vector<double> cn((size_t)NCHI * 8, 0.0);
@@ -149,16 +158,30 @@ int ctx_init_tables(jc_ctx* ctx) {
   }
   HIPCHK(ctx->g_nodes.upload(gn, s));
   // sigma_8 Romberg nodes: ln k = -4 + 7 j / 128 (power.py:66-76, the
-  // log10/ln bounds as in the reference), top-hat window of R = 8
-  std::vector<double> rb((size_t)NROMB * 3);
+  // log10/ln bounds as in the reference), top-hat window of R = 8.  The
+  // extrapolated integral (integrate.py:67-159, divmax = 7) is linear in the
+  // samples: the weight of sample j is the result for f = delta_j.
+  std::vector<double> rb((size_t)NROMB * 4);
   for (int j = 0; j < NROMB; ++j) {
+    double prev[8] = {0.0}, cur[8];
+    for (int l = 0; l <= 7; ++l) {
+      const int stride = 128 >> l;
+      cur[0] = j % stride ? 0.0 : (j == 0 || j == 128 ? 0.5 : 1.0) * 7.0 / (1 << l);
+      double p4 = 1.0;
+      for (int q = 1; q <= l; ++q) {
+        p4 *= 4.0;
+        cur[q] = (p4 * cur[q - 1] - prev[q - 1]) / (p4 - 1.0);
+      }
+      std::copy(cur, cur + l + 1, prev);
+    }
     const double lk = -4.0 + j * (7.0 / 128.0);
     const double k = exp(lk);
     const double x = k * 8.0;
     const double wv = 3.0 * (sin(x) - x * cos(x)) / (x * x * x);
-    rb[(size_t)j * 3] = k;
-    rb[(size_t)j * 3 + 1] = 1.0 / k;
-    rb[(size_t)j * 3 + 2] = k * ((k * wv) * (k * wv));
+    rb[(size_t)j * 4] = k;
+    rb[(size_t)j * 4 + 1] = 1.0 / k;
+    rb[(size_t)j * 4 + 2] = lk;
+    rb[(size_t)j * 4 + 3] = cur[7] * k * ((k * wv) * (k * wv)) / (2.0 * PI_D * PI_D);
   }
   HIPCHK(ctx->romb.upload(rb, s));
   return JC_OK;
@@ -229,13 +252,22 @@ int build_grid(jc_ctx* ctx, TracerSet* ts, int N, GridTables** out) {
   HIPCHK(g->a_list.upload(a, s));
   HIPCHK(g->a_wgt.upload(aw, s));
   {
-    std::vector<double> aln(a.size()), al10(a.size());
+    std::vector<double> aln(a.size());
+    std::vector<ASeg> seg(a.size());
     for (size_t m = 0; m < a.size(); ++m) {
       aln[m] = log(a[m]);
-      al10[m] = log10(a[m]);
+      int i, j;
+      interp_nodes(a[m], ctx->atab_chi_h, i, j);
+      seg[m].ci = (int16_t)i;
+      seg[m].cj = (int16_t)j;
+      seg[m].tc = (a[m] - ctx->atab_chi_h[i]) / (ctx->atab_chi_h[j] - ctx->atab_chi_h[i]);
+      interp_nodes(a[m], ctx->atab_g_h, i, j);
+      seg[m].gi = (int16_t)i;
+      seg[m].gj = (int16_t)j;
+      seg[m].tg = (a[m] - ctx->atab_g_h[i]) / (ctx->atab_g_h[j] - ctx->atab_g_h[i]);
     }
     HIPCHK(g->a_ln.upload(aln, s));
-    HIPCHK(g->a_l10.upload(al10, s));
+    HIPCHK(g->a_seg.upload(seg, s));
   }
   HIPCHK(g->zp1.upload(zp1, s));
   // weak-lensing bins, one group per probe
@@ -544,7 +576,7 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
   ta.Na = Na;
   ta.a_list = g->a_list.p;
   ta.a_ln = g->a_ln.p;
-  ta.a_l10 = g->a_l10.p;
+  ta.a_seg = g->a_seg.p;
   ta.a_wgt = g->a_wgt.p;
   resident_tables(ctx, ta);
   ta.nLoc = g->nLoc;
@@ -593,7 +625,7 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
       d_out_t = ctx->out_t.p;
     }
   }
-  HIPCHK(timed(ctx, JC_KERNEL_TABLES, [&] { return launch_tables(nd, ta, s, ctx->tables_variant); }));
+  HIPCHK(timed(ctx, JC_KERNEL_TABLES, [&] { return launch_tables(nd, ta, s, ctx->num_cu, ctx->tables_variant); }));
 
   for (auto& wg : g->wl) {
     WLArgs wa{};
@@ -707,7 +739,7 @@ int tables_on_alist(jc_ctx* ctx, const double* cosmo, const double* a, int64_t n
     ta.dbg = ctx->dbg.p;
     ta.dbg_stride = (int)stride;
   }
-  HIPCHK(launch_tables(0, ta, s));
+  HIPCHK(launch_tables(0, ta, s, ctx->num_cu));
   return JC_OK;
 }
 
@@ -1377,7 +1409,7 @@ int jc_debug_tables(jc_ctx* ctx, const double* cosmo, int64_t set_id, int64_t n_
   ta.Na = Na;
   ta.a_list = g->a_list.p;
   ta.a_ln = g->a_ln.p;
-  ta.a_l10 = g->a_l10.p;
+  ta.a_seg = g->a_seg.p;
   ta.a_wgt = g->a_wgt.p;
   resident_tables(ctx, ta);
   ta.nLoc = g->nLoc;
@@ -1391,7 +1423,7 @@ int jc_debug_tables(jc_ctx* ctx, const double* cosmo, int64_t set_id, int64_t n_
   ta.R = ctx->R.p;
   ta.dbg = ctx->dbg.p;
   ta.dbg_stride = (int)stride;
-  HIPCHK(launch_tables(0, ta, s));
+  HIPCHK(launch_tables(0, ta, s, ctx->num_cu));
   HIPCHK(hipMemcpyAsync(out, ctx->dbg.p, stride * 8, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   return JC_OK;

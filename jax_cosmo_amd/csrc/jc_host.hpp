@@ -110,15 +110,16 @@ inline double linspace_at(double a, double b, int num, int i) {
   return a + i * ((b - a) / (num - 1));
 }
 
-// nearest-node segment of interpolate.py:12-37 on logspace(-3, 0, n):
-// returns the lower node L of the segment the reference evaluates.
-inline int interp_segment(double x, const std::vector<double>& xp) {
+// nearest-node segment of interpolate.py:12-37 on logspace(-3, 0, n): the
+// node `ind` nearest to x (clipped to the interior) and its neighbour `nb` on
+// x's side.
+inline void interp_nodes(double x, const std::vector<double>& xp, int& ind, int& nb) {
   const int n = (int)xp.size();
   double u = (log10(x) + 3.0) * (n - 1) / 3.0;
   int i0 = (int)floor(u);
   i0 = std::min(std::max(i0, 0), n - 1);
   int lo = std::max(i0 - 1, 0), hi = std::min(i0 + 2, n - 1);
-  int ind = i0;
+  ind = i0;
   double best = 1e300;
   for (int j = lo; j <= hi; ++j) {
     const double d = (x - xp[j]) * (x - xp[j]);
@@ -129,7 +130,12 @@ inline int interp_segment(double x, const std::vector<double>& xp) {
   }
   ind = std::min(std::max(ind, 1), n - 2);
   double xc = std::min(std::max(x, xp[1]), xp[n - 2]);
-  const int nb = (xc - xp[ind] < 0.0) ? ind - 1 : ind + 1;
+  nb = (xc - xp[ind] < 0.0) ? ind - 1 : ind + 1;
+}
+// the lower node of the segment the reference evaluates
+inline int interp_segment(double x, const std::vector<double>& xp) {
+  int ind, nb;
+  interp_nodes(x, xp, ind, nb);
   return std::min(ind, nb);
 }
 
@@ -144,7 +150,8 @@ struct WLGroup {
 
 struct GridTables {
   int N = 0, Na = 0;
-  DevBuf<double> a_list, a_wgt, loc_nb, a_ln, a_l10;
+  DevBuf<double> a_list, a_wgt, loc_nb, a_ln;
+  DevBuf<jc::ASeg> a_seg;
   DevBuf<int> loc_col, loc_mode;
   DevBuf<float> zp1;
   int nLoc = 0;
@@ -182,10 +189,10 @@ struct jc_ctx {
   hipStream_t own = nullptr;
   hipStream_t stream = nullptr;
   std::vector<double> atab_chi_h, atab_g_h;
-  DevBuf<double> atab_chi, atab_g, hf_lnk, hf_w, hf_E, logr;
+  DevBuf<double> atab_chi, atab_g, hf_lnk, hf_E, logr;
   DevBuf<float> hf_k32;
   DevBuf<double> hf_kp;
-  DevBuf<double> chi_nodes, g_nodes, gg_nodes, romb, hf_kd;
+  DevBuf<double> chi_nodes, g_nodes, gg_nodes, romb, hf_nodes, hf_R2;
   std::map<int64_t, std::unique_ptr<TracerSet>> sets;
   int64_t next_set = 1;
   // workspace
@@ -222,7 +229,6 @@ inline void resident_tables(const jc_ctx* ctx, jc::TablesArgs& ta) {
   ta.atab_chi = ctx->atab_chi.p;
   ta.atab_g = ctx->atab_g.p;
   ta.hf_lnk = ctx->hf_lnk.p;
-  ta.hf_w = ctx->hf_w.p;
   ta.hf_k32 = ctx->hf_k32.p;
   ta.hf_kp = ctx->hf_kp.p;
   ta.hf_E = ctx->hf_E.p;
@@ -231,7 +237,8 @@ inline void resident_tables(const jc_ctx* ctx, jc::TablesArgs& ta) {
   ta.g_nodes = ctx->g_nodes.p;
   ta.gg_nodes = ctx->gg_nodes.p;
   ta.romb = ctx->romb.p;
-  ta.hf_kd = ctx->hf_kd.p;
+  ta.hf_nodes = ctx->hf_nodes.p;
+  ta.hf_R2 = ctx->hf_R2.p;
   ta.transfer_model = ctx->transfer_model;
   ta.halofit_model = ctx->halofit_model;
   ta.growth_model = ctx->growth_model;

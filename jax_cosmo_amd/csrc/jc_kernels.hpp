@@ -67,8 +67,6 @@ enum FwdSlot {
   FT_AN,
   FT_AW,     // 2 pi^2 max(chi, 1)^3 x Simpson weight x dchi/da / max(chi^2, 1) / c^2
   FT_CHI = CF_CHI,
-  FT_LNHI = 18,  // -ln max(chi, 1) as a float and
-  FT_LNLO = 19,  // the rest
 };
 static_assert(NCOEF == 20, "FwdSlot shares the record of CoefSlot");
 // Per-cosmology record (EH98 constants and the lensing prefactor).
@@ -93,6 +91,14 @@ constexpr int NEHD_ROW = 8;
 struct RJob;
 struct RCol;
 
+// Segments of the chi and growth tables at a node of the a-grid
+// (interpolate.py:12-37): table nodes i, j and the fraction t of
+// f[i] + (f[j] - f[i]) t.
+struct ASeg {
+  double tc, tg;
+  int16_t ci, cj, gi, gj;
+};
+
 struct TablesArgs {
   const double* params;   // [B][8] Cosmology(...) parameters
   const double* seeds;    // [B][8][ND] d param / d direction (ND > 0)
@@ -102,7 +108,6 @@ struct TablesArgs {
   const double* atab_chi; // [256]
   const double* atab_g;   // [128]
   const double* hf_lnk;   // [257]
-  const double* hf_w;     // [257] Simpson weights incl. dx/3
   const float* hf_k32;    // [257] exp(hf_lnk) as float
   const double* hf_kp;    // [257][4] k^2, k^4, k^6, 0 at k = exp(hf_lnk)
   const double* hf_E;     // [257][256] exp(-(k_i R_j)^2)
@@ -111,10 +116,11 @@ struct TablesArgs {
   const double* chi_nodes;  // [256][8]: a_i, ln a_i, 1/a_i, a_mid, ln a_mid, 1/a_mid, h_i (chi RK4 in ln a)
   const double* g_nodes;    // [128][8]: x_i, ln x_i, 1/x_i, x_mid, ln x_mid, 1/x_mid (growth RK4 in a)
   const double* gg_nodes;   // [128][8]: as chi_nodes on the growth grid (gamma growth RK4 in ln a)
-  const double* romb;       // [129][3]: k, 1/k, k (k W(8k))^2 at the sigma_8 Romberg nodes
-  const double* hf_kd;      // [257] exp(hf_lnk)
+  const double* romb;       // [129][4]: k, 1/k, ln k, Romberg weight x k (k W(8k))^2/(2 pi^2) at the sigma_8 nodes
+  const double* hf_nodes;   // [257][4]: k, 1/k, ln k, Simpson weight x k^3/(2 pi^2) at k = exp(hf_lnk)
+  const double* hf_R2;      // [256] R^2 at R = exp(logr)
   const double* a_ln;       // [Na] ln a of the a-grid, or null (computed in the kernel)
-  const double* a_l10;      // [Na] log10 a of the a-grid, or null
+  const ASeg* a_seg;        // [Na] table segments of the a-grid, or null
   // kernels local in z: number counts n b H (probes.py:77-99) and the NLA
   // intrinsic-alignment terms of weak-lensing bins (probes.py:102-129)
   int nLoc;
@@ -287,7 +293,7 @@ __host__ __device__ inline int ragged_slices(int tiles, int waves, int Na, int m
 }
 
 // launchers (defined next to their kernels)
-hipError_t launch_tables(int nd, const TablesArgs& a, hipStream_t s, int variant = 0);
+hipError_t launch_tables(int nd, const TablesArgs& a, hipStream_t s, int num_cu, int variant = 0);
 hipError_t launch_wl(int nd, int ctile, const WLArgs& a, hipStream_t s);
 // Gaussian likelihood on block-diagonal covariances (jc_likelihood.hip)
 hipError_t launch_block_inv(const double* cov, int P, int n_ell, double* inv, double* piv, hipStream_t s);

@@ -270,7 +270,7 @@ TablesArgs tables_args(jc_server* S, int g, const GroupBufs& b, int nd, const in
   ta.growth_model = S->growth_model;
   ta.gamma = S->gamma;
   ta.a_ln = gt->a_ln.p;
-  ta.a_l10 = gt->a_l10.p;
+  ta.a_seg = gt->a_seg.p;
   ta.nLoc = gt->nLoc;
   ta.loc_nb = gt->loc_nb.p;
   ta.loc_col = gt->loc_col.p;
@@ -315,7 +315,7 @@ hipError_t enqueue_pass(jc_server* S, Slot* sl, int pass, hipStream_t ps, const 
       TablesArgs ta = tables_args(S, g, b, nd, cnt + (pass ? 2 : 0), k);
       if (stage == 0) {
         if ((e = hipStreamWaitEvent(st, sl->ev_fork[pass], 0)) != hipSuccess) return e;
-        if ((e = launch_tables(nd, ta, st, S->tables_variant)) != hipSuccess) return e;
+        if ((e = launch_tables(nd, ta, st, S->ctx->num_cu, S->tables_variant)) != hipSuccess) return e;
       } else if (stage == 1) {
         for (auto& wg : S->grid[g]->wl) {
           WLArgs wa{};
