@@ -434,19 +434,18 @@ int auto_waves(jc_ctx* ctx, int64_t ncols) {
 }
 // Splits of each column group's a range over blocks (grid y), each wave
 // keeping at least 8 a-nodes: small batches take enough slices for about
-// 1024 waves.  The adjoint kernel holds `occ` waves per SIMD (1 with the
-// EH98 closed form, 2 with the transfer table), so its blocks run in rounds
-// of (CUs x 4 x occ / waves): it takes the fewest slices (up to 8) whose last
-// round is at least 90 % full (measured on the 256-cosmology gradient, 400
-// blocks: 3 slices with the closed form, -10 %; 5 with the table, -8 %).
+// 1024 waves.  The adjoint kernel (closed form) holds one wave per SIMD, so
+// its blocks run in rounds of (CUs x 4 / waves): it takes the fewest slices (up
+// to 8) whose last round is at least 90 % full (measured on the 256-cosmology
+// gradient, 400 blocks: 3 slices, -10 %).
 // The forward kernels keep 4 waves per SIMD, which hide their tail, and
 // take 1 slice at large batches.
-int auto_slices(const jc_ctx* ctx, int64_t ncols, int waves, int Na, int nd, int occ) {
+int auto_slices(const jc_ctx* ctx, int64_t ncols, int waves, int Na, int nd) {
   const int64_t blocks = (ncols + 63) / 64;
   const int64_t smax = std::max(1, Na / (8 * waves));
   int64_t s = std::min<int64_t>((1024 + blocks * waves - 1) / (blocks * waves), smax);
   if (nd == 7 && s <= 1) {
-    const double per_round = (double)ctx->num_cu * 4.0 * occ / waves;
+    const double per_round = (double)ctx->num_cu * 4.0 / waves;
     for (int64_t k = 1; k <= std::min<int64_t>(8, smax); ++k) {
       const double r = (double)(blocks * k) / per_round;
       if (r / std::ceil(r) >= 0.9) {
@@ -456,6 +455,16 @@ int auto_slices(const jc_ctx* ctx, int64_t ncols, int waves, int Na, int nd, int
     }
   }
   return (int)std::max<int64_t>(1, std::min<int64_t>(s, 64));
+}
+// Blocks that share the multipoles of a (cosmology, node group) in the
+// adjoint's table mode: enough to fill the 3 blocks a CU holds, each keeping a
+// turn of 8 multipoles.  Measured (100 ell, n_z 512, 10 tracers): twice the
+// blocks 46 against 31 us at 16 cosmologies and 65 against 61 at 64 (the tables
+// are staged and the derivatives contracted per block); turns of 4 multipoles
+// 31.6 against 22.1 us at 4 cosmologies, 16.1 against 17.2 at one.
+int adjoint_slices(const jc_ctx* ctx, int64_t B, int n_ell, int Na) {
+  const int64_t units = B * adj_groups(Na);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(3 * (int64_t)ctx->num_cu / units, n_ell / 8));
 }
 int auto_ctile(jc_ctx* ctx, int64_t B, int nd) {
   if (nd != 0) return 1;
@@ -611,11 +620,14 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
   // settled before the first launch, so a call whose buffers do not fit the
   // scratch fails before any work is queued
   const int l_waves = nd == 0 && use_tab && !use_mx ? FWD_WAVES : auto_waves(ctx, ncols);
-  const int l_slices = use_mx ? 1 : auto_slices(ctx, ncols, l_waves, Na, nd, use_tab ? 2 : 1);
+  const bool adj_tab = nd == 7 && use_tab;
+  const int l_slices = use_mx    ? 1
+                       : adj_tab ? adjoint_slices(ctx, B, (int)n_ell, Na)
+                                 : auto_slices(ctx, ncols, l_waves, Na, nd);
   const size_t nslice = nd == 7 ? (size_t)ncols * 7 : (size_t)B * P * n_ell * (nd == 1 ? 2 : 1);
   const size_t nout = (size_t)B * P * n_ell;
   float* w_part = nullptr;
-  if (l_slices > 1 && (rc = workspace(ctx->part, (size_t)l_slices * nslice, sc, &w_part))) return rc;
+  if (l_slices > 1 && !adj_tab && (rc = workspace(ctx->part, (size_t)l_slices * nslice, sc, &w_part))) return rc;
   float* d_out = cl;
   float* d_out_t = cl_dot;
   if (!dev && nd != 7) {
@@ -669,17 +681,21 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
     const float* d_cbar = nullptr;
     rc = to_device(ctx, ctx->cbar, cl_bar, nout, dev, &d_cbar);
     if (rc) return rc;
-    HIPCHK(ctx->theta_col.reserve((size_t)ncols * 7));
+    const int adj_parts = adj_groups(Na) * l_slices;  // per cosmology, in table mode
+    HIPCHK(ctx->theta_col.reserve((adj_tab ? (size_t)B * adj_parts : (size_t)ncols) * 7));
     la.cbar = d_cbar;
     la.theta_col = ctx->theta_col.p;
-    HIPCHK(timed(ctx, JC_KERNEL_LIMBER, [&] { return launch_limber(nd, T, la, s); }));
+    HIPCHK(timed(ctx, JC_KERNEL_LIMBER,
+                 [&] { return adj_tab ? launch_adjoint(T, la, s) : launch_limber(nd, T, la, s); }));
     double* d_th = theta_bar;
     if (!dev) {
       HIPCHK(ctx->theta.reserve((size_t)B * 7));
       d_th = ctx->theta.p;
     }
     // the slices' partials are added inside the reduction
-    HIPCHK(launch_theta_reduce(la.slices > 1 ? la.part : ctx->theta_col.p, la.slices, (int)B, (int)n_ell, d_th, s));
+    HIPCHK(adj_tab ? launch_theta_reduce(ctx->theta_col.p, 1, (int)B, adj_parts, d_th, s)
+                   : launch_theta_reduce(la.slices > 1 ? la.part : ctx->theta_col.p, la.slices, (int)B, (int)n_ell,
+                                         d_th, s));
     if (!dev) {
       HIPCHK(hipMemcpyAsync(theta_bar, d_th, (size_t)B * 7 * sizeof(double), hipMemcpyDeviceToHost, s));
       HIPCHK(hipStreamSynchronize(s));

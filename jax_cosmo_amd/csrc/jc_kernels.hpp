@@ -198,7 +198,7 @@ struct LimberArgs {
   float* out;               // [B][P][n_ell]
   float* out_t;             // [B][P][n_ell] tangent (JVP)
   const float* cbar;        // [B][P][n_ell] cotangent (VJP)
-  float* theta_col;         // [ncols][7] per-column parameter cotangent (VJP)
+  float* theta_col;         // VJP partials: [ncols][7] per column; launch_adjoint: [B][adj_groups(Na)][slices][7]
   int waves;                // waves per block splitting the a range
   const float4* ehtab;      // [B][NEHQ] transfer table, or null: evaluate EH98 per point
   const float* ehtab7;      // adjoint: [B][NEHQ + 1][8] d/dtheta of the table's function at its nodes
@@ -255,31 +255,38 @@ struct RaggedArgs {
   int Tpad;
   float* out;
   const float* cbar;
-  float* theta_col;      // adjoint: [max_slices][colcap][7] per-slice column partials
+  const int* njobs;      // adjoint: device count of requests
+  float* theta_part;     // adjoint: per block partials, adj_ragged_blocks() rows of 7
   int waves;
   // per-cosmology transfer tables (row c of the launch's tables) and, for
   // the adjoint, their theta derivatives
   const float4* ehtab;   // [rows][NEHQ]
   const float* ehtab7;   // [rows][NEHQ + 1][NEHD_ROW]
-  // the a range of each 64-column tile is split over ragged_slices(live
-  // tiles) blocks (grid y, at most max_slices); forward partials of slice s
-  // go to part + s * part_stride in the layout of out when there is more
-  // than one, adjoint partials to theta_col + s * part_stride
+  // forward: the a range of each 64-column tile is split over
+  // ragged_slices(live tiles) blocks (grid y, at most max_slices); partials of
+  // slice s go to part + s * part_stride in the layout of out when there is
+  // more than one
   int max_slices;
   float* part;
   int64_t part_stride;
 };
 
-struct RReduceArgs {
-  const int* njobs;      // device count
-  const RJob* jobs;
-  const float* theta_col;
-  double* theta;         // [njobs][7]
-  // slices of the adjoint launch (recomputed from its live column count)
-  const int* ncols;
-  int waves, Na, max_slices;
-  int64_t part_stride;
-};
+// The adjoint's blocks (jc_adjoint.hip): a cosmology's a-nodes in groups of up
+// to 64 (lanes), its multipoles dealt to ADJ_WAVES waves and, where that leaves
+// the chip idle, to several blocks.
+constexpr int ADJ_WAVES = 4;
+__host__ __device__ inline int adj_groups(int Na) { return (Na + 63) / 64; }
+// Served batches: enough slices of the multipoles for ADJ_FILL blocks (the
+// device chooses by its live requests), within a grid of adj_ragged_blocks.
+constexpr int ADJ_FILL = 768;
+__host__ __device__ inline int adj_ragged_slices(int units) {
+  const int s = units < 1 ? 1 : ADJ_FILL / units;
+  return s < 1 ? 1 : (s > 16 ? 16 : s);
+}
+inline int adj_ragged_blocks(int max_jobs, int Na) {
+  const int u = max_jobs * adj_groups(Na);
+  return u > ADJ_FILL ? u : ADJ_FILL;
+}
 
 // Slices of a ragged launch with `tiles` live 64-column tiles: enough for
 // about 2048 waves, each wave keeping at least 8 a-nodes.
@@ -309,13 +316,17 @@ hipError_t launch_slice_sum(const float* part, int slices, int64_t n, float* out
 hipError_t launch_kde(const double* z, int64_t n, const double* cz, const double* cw, int64_t ncat, double bw,
                       double wsum, double* out, hipStream_t s);
 hipError_t launch_limber(int nd, int T, const LimberArgs& a, hipStream_t s);
+// the adjoint in transfer-table mode; its partials theta_col are then summed by
+// launch_theta_reduce(theta_col, 1, B, adj_groups(Na) * slices, ...)
+hipError_t launch_adjoint(int T, const LimberArgs& a, hipStream_t s);
 // theta[B][7] = sum over slices and ell of the per-column partials
 // [nsl][B][n_ell][7] (nsl = 1: the partials of an unsliced launch)
 hipError_t launch_theta_reduce(const float* theta_col, int nsl, int B, int n_ell, double* theta, hipStream_t s);
 hipError_t launch_pk_eval(const PkArgs& a, hipStream_t s);
 // grid sized for max_cols columns; blocks beyond *ncols exit at once
-hipError_t launch_limber_ragged(int nd, int max_cols, const RaggedArgs& a, hipStream_t s);
-hipError_t launch_ragged_reduce(int max_jobs, const RReduceArgs& a, hipStream_t s);
+hipError_t launch_limber_ragged(int max_cols, const RaggedArgs& a, hipStream_t s);
+hipError_t launch_ragged_adjoint(int max_jobs, const RaggedArgs& a, hipStream_t s);
+hipError_t launch_ragged_reduce(int max_jobs, const RaggedArgs& a, double* theta, hipStream_t s);
 // dense covariances (jc_dense.hip): in-place lower Cholesky factor of the
 // row-major N x N matrix A (log L_ii into dlog[N], *bad set on a
 // non-positive pivot; the strict upper triangle is zeroed; inv: DENSE_PANEL^2

@@ -16,7 +16,8 @@
 // Modes (ND = number of dual directions):
 //   ND = 0  forward C_ell;
 //   ND = 1  forward plus one directional derivative (JVP);
-//   ND = 7  adjoint: contracts dC/dtheta with a cotangent Cbar on the fly
+//   ND = 7  adjoint (calls without transfer tables; with them, jc_adjoint.hip):
+//           contracts dC/dtheta with a cotangent Cbar on the fly
 //           (theta = Omega_c, Omega_b, h, n_s, sigma8, w0, wa) using
 //           sum_{i<=j} c_ij d(R_i R_j) = sum_i dR_i V_i, V_i = sum_j ct_ij R_j.
 #include "jc_records.hpp"
@@ -58,9 +59,8 @@ JC_D Sf limber_point(const EHc<Sf>& eh, const Sf& ns, const PointCoefs<Sf, W>& p
 // fields, n_s, T), and dM/dtheta_d = sum_x dM/dx dx/dtheta_d with dx/dtheta
 // the dual parts the table kernel stored.  The forward order of operations
 // is limber_point's (halofit_pnl in base 2 with one shared reciprocal).
-// tn = T(k) k^(n_s/2) is a forward dual: from the EH98 closed form (duals
-// through the constants and k), or read from the transfer table with its
-// theta derivatives (adj_tn_tab); plin = tn^2 D^2 pknorm.
+// tn = T(k) k^(n_s/2) is a forward dual from the EH98 closed form (duals
+// through the constants and k); plin = tn^2 D^2 pknorm.
 template <int W>
 JC_D void limber_point_adj(const Dual<float, 7>& tn, const PointCoefs<Dual<float, 7>, W>& pc, const EllC& lc,
                            float& Mv, float* Md) {
@@ -163,44 +163,6 @@ JC_D Dual<float, 7> adj_tn_closed(const EHc<Dual<float, 7>>& eh, const Dual<floa
   return eh_transfer(eh, kd, invkd, lnkd) * jm::exp(ns * (0.5f * lnkd));
 }
 
-// ... and from the cosmology's transfer table: the value and its ln k slope
-// from the cubic piece (as the forward kernel), the theta derivatives at
-// fixed k by 4-point Lagrange interpolation of their values at the table's
-// nodes q-1 .. q+2 (clamped at the ends; rows of 8 floats read through the
-// L2), plus slope x d ln k.  Linear interpolation on a 4x coarser grid was
-// 1.3e-3 off in d/d Omega_b: its baryon-wiggle part oscillates in ln k with
-// a period of a few coarse nodes near k ~ 0.3 h/Mpc.
-template <int W>
-JC_D Dual<float, 7> adj_tn_tab(const float4* tab, const float* __restrict__ dtab, double invh, double lo_invh,
-                               const PointCoefs<Dual<float, 7>, W>& pc, const EllC& lc) {
-  const float lnk = lc.lnlph + pc.lninvchi.v;
-  const double u = __builtin_fma((double)lnk, invh, -lo_invh);
-  int q = (int)u;
-  q = q < 0 ? 0 : (q > NEHQ - 1 ? NEHQ - 1 : q);
-  const float t = (float)(u - (double)q);
-  const float4 cc = tab[q];
-  Dual<float, 7> tn;
-  tn.v = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cc.w, t, cc.z), t, cc.y), t, cc.x);
-  const float slope = __builtin_fmaf(__builtin_fmaf(3.0f * cc.w, t, 2.0f * cc.z), t, cc.y) * (float)invh;
-  // nodes j0 .. j0 + 3 with j0 = clamp(q - 1, 0, NEHQ - 3); s = position from j0
-  const int j0 = q < 1 ? 0 : (q > NEHQ - 2 ? NEHQ - 3 : q - 1);
-  const float s = t + (float)(q - j0);
-  const float s1 = s - 1.0f, s2 = s - 2.0f, s3 = s - 3.0f;
-  const float w0 = -(1.0f / 6.0f) * s1 * s2 * s3, w1 = 0.5f * s * s2 * s3;
-  const float w2 = -0.5f * s * s1 * s3, w3 = (1.0f / 6.0f) * s * s1 * s2;
-  const float4* r = reinterpret_cast<const float4*>(dtab + (size_t)j0 * NEHD_ROW);
-  const float4 a0 = r[0], b0 = r[1], a1 = r[2], b1 = r[3], a2 = r[4], b2 = r[5], a3 = r[6], b3 = r[7];
-  const float n0[7] = {a0.x, a0.y, a0.z, a0.w, b0.x, b0.y, b0.z};
-  const float n1[7] = {a1.x, a1.y, a1.z, a1.w, b1.x, b1.y, b1.z};
-  const float n2[7] = {a2.x, a2.y, a2.z, a2.w, b2.x, b2.y, b2.z};
-  const float n3[7] = {a3.x, a3.y, a3.z, a3.w, b3.x, b3.y, b3.z};
-#pragma unroll
-  for (int d = 0; d < 7; ++d)
-    tn.d[d] = __builtin_fmaf(w3, n3[d], __builtin_fmaf(w2, n2[d], __builtin_fmaf(w1, n1[d], w0 * n0[d]))) +
-              slope * pc.lninvchi.d[d];
-  return tn;
-}
-
 // The dispatcher deals blocks to the 8 XCDs in turn (block b to XCD b % 8),
 // and each XCD has its own L2.  Neighbouring column groups read the same
 // cosmology's records, so blocks are renumbered to give each XCD one
@@ -216,7 +178,7 @@ template <int NACC>
 struct RedChunk { static constexpr int value = NACC < 32 ? NACC : 32; };
 
 // (forward kernels are held to 128 VGPRs: 4 waves per SIMD)
-template <int T, int ND, bool TAB>
+template <int T, int ND>
 __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A) {
   using Sf = typename Types<ND>::F;
   constexpr int W = ND + 1;
@@ -224,11 +186,7 @@ __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A)
   constexpr bool VJP = (ND == 7);
   constexpr int NACC = VJP ? 7 : P * W;
   constexpr int RCH = RedChunk<NACC>::value;
-  static_assert(!TAB || ND == 7, "forward calls in table mode run k_limber_tab");
-  // TAB: [2][NEHQ] tables (the adjoint reads its theta-derivative rows from
-  // global memory); after the a loop, [waves-1][RCH][64] partial sums
-  extern __shared__ float4 lds4[];
-  float* red = reinterpret_cast<float*>(lds4);
+  extern __shared__ float red[];  // [waves-1][RCH][64] partial sums
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -247,25 +205,7 @@ __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A)
   for (int i = 0; i < T; ++i) F[i] = ((A.wl_mask >> i) & 1u) ? lf : 1.0f;
 
   Sf ns;
-  EHc<Sf> eh;
-  const float4* tab = nullptr;
-  const float* dtab = nullptr;
-  double invh = 0.0, lo_invh = 0.0;
-  if constexpr (TAB) {
-    // the block's 64 columns span at most two cosmologies (n_ell >= 64)
-    const int cb = (grp * 64) / A.n_ell;
-    const int ce = min(A.ncols - 1, grp * 64 + 63) / A.n_ell;
-    for (int e = threadIdx.x; e < (ce - cb + 1) * NEHQ; e += blockDim.x)
-      lds4[e] = A.ehtab[(size_t)cb * NEHQ + e];
-    tab = lds4 + (c - cb) * NEHQ;
-    if constexpr (VJP) dtab = A.ehtab7 + (size_t)c * (NEHQ + 1) * NEHD_ROW;
-    const float* cr = A.crec + (size_t)c * NCREC * W;
-    invh = (double)cr[CR_EHINVH * W];
-    lo_invh = (double)cr[CR_EHLO * W] * invh;  // exact in FP64
-    __syncthreads();
-  } else {
-    eh = load_eh<Sf, W>(A.crec + (size_t)c * NCREC * W, ns);
-  }
+  const EHc<Sf> eh = load_eh<Sf, W>(A.crec + (size_t)c * NCREC * W, ns);
 
   // the a range of this wave: one of slices x waves contiguous chunks
   const int nsl = A.slices;
@@ -316,8 +256,7 @@ __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A)
       }
     } else {
       float Mv, Md[7];
-      if constexpr (TAB) limber_point_adj<W>(adj_tn_tab<W>(tab, dtab, invh, lo_invh, pc, lc), pc, lc, Mv, Md);
-      else limber_point_adj<W>(adj_tn_closed<W>(eh, ns, pc, lc), pc, lc, Mv, Md);
+      limber_point_adj<W>(adj_tn_closed<W>(eh, ns, pc, lc), pc, lc, Mv, Md);
       float V[T];
       float G = 0.0f;
 #pragma unroll
@@ -340,7 +279,7 @@ __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A)
   for (int m = m0; m < m1; ++m, cf += NCOEF * W, rr += A.Tpad * W) point(load_coefs<Sf, W>(cf), rr);
 
   // deterministic reduction over the waves of the block, RCH accumulators
-  // per pass (the LDS space of the tables is reused)
+  // per pass
   if (nwv > 1) {
 #pragma unroll
     for (int q0 = 0; q0 < NACC; q0 += RCH) {
@@ -776,16 +715,8 @@ static hipError_t launch_T(const LimberArgs& a, hipStream_t s) {
       return hipGetLastError();
     }
   }
-  if constexpr (ND == 7) {
-    if (a.ehtab) {
-      if (a.n_ell < 64 || !a.ehtab7) return hipErrorInvalidValue;
-      const size_t tab = (size_t)2 * NEHQ * sizeof(float4);
-      hipLaunchKernelGGL((k_limber<T, 7, true>), dim3(blocks, a.slices), dim3(64 * a.waves),
-                         tab > red ? tab : red, s, a);
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((k_limber<T, ND, false>), dim3(blocks, a.slices), dim3(64 * a.waves), red, s, a);
+  if (a.ehtab) return hipErrorInvalidValue;  // adjoint calls in table mode: launch_adjoint
+  hipLaunchKernelGGL((k_limber<T, ND>), dim3(blocks, a.slices), dim3(64 * a.waves), red, s, a);
   return hipGetLastError();
 }
 
@@ -1065,146 +996,14 @@ __global__ __launch_bounds__(256, 4) void k_limber_ragged_fwd(RaggedArgs A) {
   }
 }
 
-// The adjoint: per column, the 7 parameter cotangents of the request's
-// C_ell against its cotangent block, with the tile's tracer count as a
-// constant (one body per T, chosen by a block-uniform switch): cotangent and
-// tracer-kernel arrays of the request's own size and no per-pair tests, at 2
-// waves per SIMD (one body for every T with per-pair tests needed 1).  The
-// transfer table and its theta derivatives are read through the L1/L2, since
-// one tile may span several requests.
-template <int T>
-__device__ __forceinline__ void ragged_adj_tile(const RaggedArgs& A, const int tile0, const int nsl, float* red) {
-  using Sf = typename Types<7>::F;
-  constexpr int W = 8;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int nwv = A.waves;
-  const RCol col = A.cols[tile0 + lane];
-  const int first = A.cols[tile0].job;  // a tile starts with a real column
-  const bool valid = col.job >= 0;
-  const RJob& jb = A.jobs[valid ? col.job : first];
-  const int c = jb.c;
-  const double ell = valid ? col.ell : A.cols[tile0].ell;
-  const EllC lc = ell_consts(ell);
-  const float lf = (float)(::sqrt((ell - 1.0) * ell * (ell + 1.0) * (ell + 2.0)) / ((ell + 0.5) * (ell + 0.5)));
-  float F[T];
-#pragma unroll
-  for (int i = 0; i < T; ++i) F[i] = ((jb.wl_mask >> i) & 1u) ? lf : 1.0f;
-  const float4* tab = A.ehtab + (size_t)c * NEHQ;
-  const float* dtab = A.ehtab7 + (size_t)c * (NEHQ + 1) * NEHD_ROW;
-  const float* cr = A.crec + (size_t)c * NCREC * W;
-  const double invh = (double)cr[CR_EHINVH * W];
-  const double lo_invh = (double)cr[CR_EHLO * W] * invh;  // exact in FP64
-  const int chunk = (A.Na + nsl * nwv - 1) / (nsl * nwv);
-  const int m0 = min(A.Na, ((int)blockIdx.y * nwv + wave) * chunk);
-  const int m1 = min(A.Na, m0 + chunk);
-
-  float acc[7];
-#pragma unroll
-  for (int q = 0; q < 7; ++q) acc[q] = 0.0f;
-  // symmetric cotangent matrix (diagonal doubled) times F_i F_j
-  float ct[T][T];
-  {
-    int p = 0;
-#pragma unroll
-    for (int i = 0; i < T; ++i) {
-#pragma unroll
-      for (int j = i; j < T; ++j) {
-        const float v = valid ? A.cbar[jb.cbar_off + (int64_t)p * jb.n_ell + col.l] * F[i] * F[j] : 0.0f;
-        ct[i][j] = (i == j) ? 2.0f * v : v;
-        ct[j][i] = ct[i][j];
-        ++p;
-      }
-    }
-  }
-  const float* cf = A.coef + ((size_t)c * A.Na + m0) * NCOEF * W;
-  const float* rr = A.R + ((size_t)c * A.Na + m0) * A.Tpad * W;
-  for (int m = m0; m < m1; ++m, cf += NCOEF * W, rr += A.Tpad * W) {
-    const PointCoefs<Sf, W> pc = load_coefs<Sf, W>(cf);
-    Sf Rv[T];
-#pragma unroll
-    for (int i = 0; i < T; ++i) Rv[i] = Mem<Sf>::ld(rr + i * W);
-    float Mv, Md[7];
-    limber_point_adj<W>(adj_tn_tab<W>(tab, dtab, invh, lo_invh, pc, lc), pc, lc, Mv, Md);
-    float V[T];
-    float G = 0.0f;
-#pragma unroll
-    for (int i = 0; i < T; ++i) {
-      float sv = 0.0f;
-#pragma unroll
-      for (int j = 0; j < T; ++j) sv += ct[i][j] * val(Rv[j]);
-      V[i] = sv;
-      G += 0.5f * val(Rv[i]) * sv;
-    }
-#pragma unroll
-    for (int d = 0; d < 7; ++d) {
-      float sd = 0.0f;
-#pragma unroll
-      for (int i = 0; i < T; ++i) sd += Rv[i].d[d] * V[i];
-      acc[d] += Mv * sd + G * Md[d];
-    }
-  }
-  if (nwv > 1) {
-    if (wave > 0) {
-#pragma unroll
-      for (int q = 0; q < 7; ++q) red[((wave - 1) * 7 + q) * 64 + lane] = acc[q];
-    }
-    __syncthreads();
-    if (wave == 0) {
-      for (int w = 1; w < nwv; ++w) {
-#pragma unroll
-        for (int q = 0; q < 7; ++q) acc[q] += red[((w - 1) * 7 + q) * 64 + lane];
-      }
-    }
-  }
-  if (wave != 0) return;
-  float* tc = A.theta_col + (size_t)blockIdx.y * A.part_stride;
-#pragma unroll
-  for (int d = 0; d < 7; ++d) tc[(size_t)(tile0 + lane) * 7 + d] = valid ? acc[d] : 0.0f;
-}
-
-__global__ __launch_bounds__(256, 2) void k_limber_ragged_adj(RaggedArgs A) {
-  extern __shared__ float red[];
-  const int ncols = *A.ncols;
-  // The grid is sized for capacity: the live tiles are dealt to the 8 XCDs
-  // (block b runs on XCD b % 8) in contiguous ranges, so neighbouring tiles
-  // (one request's columns) share an L2, and blocks past each XCD's range exit.
-  const int live = (ncols + 63) >> 6;
-  const int nsl = ragged_slices(live, A.waves, A.Na, A.max_slices);
-  if ((int)blockIdx.y >= nsl) return;
-  const int xq = live >> 3, xr = live & 7, xx = blockIdx.x & 7, xi = blockIdx.x >> 3;
-  if (xi >= xq + (xx < xr ? 1 : 0)) return;
-  const int tile0 = (xx * xq + min(xx, xr) + xi) * 64;
-  const int T = __builtin_amdgcn_readfirstlane(A.jobs[A.cols[tile0].job].T);
-  switch (T) {
-    case 1: ragged_adj_tile<1>(A, tile0, nsl, red); break;
-    case 2: ragged_adj_tile<2>(A, tile0, nsl, red); break;
-    case 3: ragged_adj_tile<3>(A, tile0, nsl, red); break;
-    case 4: ragged_adj_tile<4>(A, tile0, nsl, red); break;
-    case 5: ragged_adj_tile<5>(A, tile0, nsl, red); break;
-    case 6: ragged_adj_tile<6>(A, tile0, nsl, red); break;
-    case 7: ragged_adj_tile<7>(A, tile0, nsl, red); break;
-    case 8: ragged_adj_tile<8>(A, tile0, nsl, red); break;
-    case 9: ragged_adj_tile<9>(A, tile0, nsl, red); break;
-    default: ragged_adj_tile<10>(A, tile0, nsl, red); break;
-  }
-}
-
-hipError_t launch_limber_ragged(int nd, int max_cols, const RaggedArgs& a, hipStream_t s) {
+hipError_t launch_limber_ragged(int max_cols, const RaggedArgs& a, hipStream_t s) {
   if (a.waves < 1 || a.waves > 4 || max_cols < 64 || (max_cols % 64) != 0) return hipErrorInvalidValue;
-  if (a.max_slices < 1 || a.max_slices > 64 || !a.ehtab || (nd == 7 && !a.ehtab7)) return hipErrorInvalidValue;
-  if (nd == 0 && a.max_slices > 1 && !a.part) return hipErrorInvalidValue;
+  if (a.max_slices < 1 || a.max_slices > 64 || !a.ehtab) return hipErrorInvalidValue;
+  if (a.max_slices > 1 && !a.part) return hipErrorInvalidValue;
   const dim3 grid(max_cols / 64, a.max_slices);
-  if (nd == 0) {
-    // two transfer tables, or the reduction's [waves - 1][32][64] partials
-    const size_t sm = std::max((size_t)2 * NEHQ * sizeof(float4), (size_t)(a.waves - 1) * 32 * 64 * sizeof(float));
-    hipLaunchKernelGGL(k_limber_ragged_fwd, grid, dim3(64 * a.waves), sm, s, a);
-  } else if (nd == 7) {
-    const size_t sm = (size_t)(a.waves - 1) * 7 * 64 * sizeof(float);
-    hipLaunchKernelGGL(k_limber_ragged_adj, grid, dim3(64 * a.waves), sm, s, a);
-  } else {
-    return hipErrorInvalidValue;
-  }
+  // two transfer tables, or the reduction's [waves - 1][32][64] partials
+  const size_t sm = std::max((size_t)2 * NEHQ * sizeof(float4), (size_t)(a.waves - 1) * 32 * 64 * sizeof(float));
+  hipLaunchKernelGGL(k_limber_ragged_fwd, grid, dim3(64 * a.waves), sm, s, a);
   return hipGetLastError();
 }
 
@@ -1229,52 +1028,6 @@ hipError_t launch_ragged_slice_sum(const int* ncols, int waves, int Na, int max_
   if (max_out <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_ragged_slice_sum, dim3((unsigned)((max_out + 255) / 256)), dim3(256), 0, s, ncols, waves,
                      Na, max_slices, part, part_stride, range, out);
-  return hipGetLastError();
-}
-
-// theta[row(j)][d] = sum over the columns of request j and the adjoint
-// launch's live slices (FP64).  One 256-thread block per request (the grid
-// is sized for capacity): thread t adds the elements t, t + 256, ... of the
-// request's [n_ell][7] column partials over the slices (coalesced; element e
-// belongs to parameter e % 7, and 256 = 36 * 7 + 4 moves it by four), each
-// wave adds its lanes by a butterfly and thread q < 7 adds the four waves'
-// sums of parameter q in a fixed order.
-__global__ __launch_bounds__(256) void k_ragged_reduce(RReduceArgs A) {
-  __shared__ double wsum[4][8];
-  const int j = blockIdx.x;
-  if (j >= *A.njobs) return;  // uniform across the block
-  const int nsl = ragged_slices((*A.ncols + 63) >> 6, A.waves, A.Na, A.max_slices);
-  const RJob jb = A.jobs[j];
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int n = jb.n_ell * 7;
-  const float* p = A.theta_col + (size_t)jb.col0 * 7;
-  double acc[7];
-#pragma unroll
-  for (int q = 0; q < 7; ++q) acc[q] = 0.0;
-  int d = t % 7;
-  for (int e = t; e < n; e += 256) {
-    double v = 0.0;
-    for (int k = 0; k < nsl; ++k) v += (double)p[(size_t)k * A.part_stride + e];
-#pragma unroll
-    for (int q = 0; q < 7; ++q) acc[q] += (q == d) ? v : 0.0;
-    d = (d >= 3) ? d - 3 : d + 4;
-  }
-#pragma unroll
-  for (int q = 0; q < 7; ++q) {
-    double v = acc[q];
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    if (lane == q) wsum[wave][q] = v;
-  }
-  __syncthreads();
-  // out_off: the request's row in the batch
-  if (t < 7) A.theta[jb.out_off * 7 + t] = ((wsum[0][t] + wsum[1][t]) + wsum[2][t]) + wsum[3][t];
-}
-
-hipError_t launch_ragged_reduce(int max_jobs, const RReduceArgs& a, hipStream_t s) {
-  if (max_jobs <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_ragged_reduce, dim3(max_jobs), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

@@ -27,10 +27,12 @@ namespace {
 constexpr int MAXG = 4;         // served Simpson sizes
 constexpr int MAXSEC = 64;      // staging sections
 constexpr int TPAD_POOL = 12;   // pool of up to 10 tracers, padded
-// a-range slices of the ragged Limber kernels (the live count is chosen per
+// a-range slices of the ragged forward kernel (the live count is chosen per
 // batch on the device, ragged_slices)
 constexpr int SLICES_FWD = 8;
-constexpr int SLICES_ADJ = 16;
+// rows of 7 floats that a gradient request's column counts for in the memory
+// budget (its partials, adj_ragged_blocks() rows a group, need fewer)
+constexpr int ADJ_ROWS = 16;
 
 struct StageSec {
   int64_t dst, src, bytes;
@@ -99,7 +101,7 @@ struct GroupBufs {
   float4* ehtab = nullptr;     // [C][NEHQ] transfer tables of the forward rows
   float4* ehtab_d = nullptr;   // [Gd][NEHQ] ... of the gradient rows
   float* ehtab7 = nullptr;     // [Gd][NEHQ + 1][NEHD_ROW] their theta derivatives
-  float* theta_col = nullptr;  // [SLICES_ADJ][gcolcap][7]
+  float* theta_part = nullptr;  // the adjoint's block partials, rows of 7
 };
 
 struct Slot {
@@ -210,7 +212,7 @@ size_t req_footprint(const jc_server* S, const jc_request& r, int g) {
              (size_t)r.n_ell * sizeof(RCol) + sizeof(RJob) + (size_t)NEHQ * 16 + 64;
   if (r.want_grad)
     b += 8 * (Na * (NCOEF + TPAD_POOL) * 4 + NCHI * 2 * 4 + NCREC * 4) + (size_t)P * r.n_ell * 4 +
-         (size_t)r.n_ell * (sizeof(RCol) + 28 * SLICES_ADJ) + sizeof(RJob) + (size_t)NEHQ * 16 +
+         (size_t)r.n_ell * (sizeof(RCol) + 28 * ADJ_ROWS) + sizeof(RJob) + (size_t)NEHQ * 16 +
          (size_t)(NEHQ + 1) * NEHD_ROW * 4 + 64 + 7 * 8;
   return b;
 }
@@ -249,7 +251,8 @@ size_t layout_slot(jc_server* S, Slot* sl, unsigned char* base) {
     b.ehtab = (float4*)take((size_t)S->C * NEHQ * sizeof(float4));
     b.ehtab_d = (float4*)take((size_t)S->Gd * NEHQ * sizeof(float4));
     b.ehtab7 = (float*)take((size_t)S->Gd * (NEHQ + 1) * NEHD_ROW * 4);
-    b.theta_col = (float*)take((size_t)SLICES_ADJ * S->gcolcap * 7 * 4);
+    b.theta_part = (float*)take(
+        std::max((size_t)ADJ_ROWS * S->gcolcap, (size_t)adj_ragged_blocks(S->Gd, (int)Na)) * 7 * 4);
   }
   return off;
 }
@@ -350,27 +353,19 @@ hipError_t enqueue_pass(jc_server* S, Slot* sl, int pass, hipStream_t ps, const 
         ra.Tpad = TPAD_POOL;
         ra.out = sl->out;
         ra.cbar = sl->cbar;
-        ra.theta_col = b.theta_col;
+        ra.njobs = cnt + 2;
+        ra.theta_part = b.theta_part;
         ra.waves = S->waves;
         ra.ehtab = ta.ehtab;
         ra.ehtab7 = ta.ehtab7;
-        ra.max_slices = pass ? SLICES_ADJ : SLICES_FWD;
+        ra.max_slices = SLICES_FWD;
         ra.part = pass ? nullptr : sl->part;
-        ra.part_stride = pass ? (int64_t)S->gcolcap * 7 : S->outcap;
+        ra.part_stride = S->outcap;
         if (stage == 2) {
-          if ((e = launch_limber_ragged(nd, pass ? k.gcolcap : k.colcap, ra, st)) != hipSuccess) return e;
+          e = pass ? launch_ragged_adjoint(k.Gd, ra, st) : launch_limber_ragged(k.colcap, ra, st);
+          if (e != hipSuccess) return e;
         } else if (pass) {
-          RReduceArgs rr{};
-          rr.njobs = cnt + 2;
-          rr.jobs = b.gjobs;
-          rr.theta_col = b.theta_col;
-          rr.theta = sl->theta;
-          rr.ncols = ra.ncols;
-          rr.waves = ra.waves;
-          rr.Na = ra.Na;
-          rr.max_slices = ra.max_slices;
-          rr.part_stride = ra.part_stride;
-          if ((e = launch_ragged_reduce(k.Gd, rr, st)) != hipSuccess) return e;
+          if ((e = launch_ragged_reduce(k.Gd, ra, sl->theta, st)) != hipSuccess) return e;
         } else {
           // the group's output range [counts[4], counts[5]): add the slices
           if ((e = launch_ragged_slice_sum(ra.ncols, ra.waves, ra.Na, ra.max_slices, sl->part, S->outcap, cnt + 4,
