@@ -257,8 +257,10 @@ int jc_background_ex(jc_ctx* ctx, const double* cosmo, const double* a, int64_t 
  * context's transfer model. */
 int jc_sigma8_norm(jc_ctx* ctx, const double* cosmo, double* pknorm);
 
-/* Tile shape used by the Limber kernel for a batch shape (the autotuner
- * writes it; 0 = automatic).  waves_per_block in {1, 2, 4}. */
+/* Tile shapes for a batch shape (the autotuner writes them; 0 = automatic):
+ * waves_per_block of the Limber kernels without transfer tables, in {1, 2, 4},
+ * and cosmologies per block of the forward weak-lensing kernel, in {1, 4, 8,
+ * 16}. */
 int jc_set_tiles(jc_ctx* ctx, int32_t waves_per_block, int32_t wl_ctile);
 int jc_get_tiles(jc_ctx* ctx, int32_t* waves_per_block, int32_t* wl_ctile);
 /* Shape of the per-cosmology table kernel (autotuned): 0 = default,

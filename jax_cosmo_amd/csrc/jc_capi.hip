@@ -466,15 +466,6 @@ int adjoint_slices(const jc_ctx* ctx, int64_t B, int n_ell, int Na) {
   const int64_t units = B * adj_groups(Na);
   return (int)std::max<int64_t>(1, std::min<int64_t>(3 * (int64_t)ctx->num_cu / units, n_ell / 8));
 }
-int auto_ctile(jc_ctx* ctx, int64_t B, int nd) {
-  if (nd != 0) return 1;
-  if (ctx->wl_ctile > 0) return ctx->wl_ctile;
-  // measured on MI355X (N = 512, 10 tracers): one cosmology per block up to
-  // ~128 (more blocks), four from ~256 (table reuse); eight is slower
-  if (B >= 192) return 4;
-  return 1;
-}
-
 // Timing events only: jc_profile_read synchronizes the stream before reading
 // them, so they need no system-scope release (without it each record cost
 // the 1024-cosmology batch's stream ~1.5 us less).
@@ -656,8 +647,7 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
     wa.crec = w_crec;
     wa.R = w_R;
     wa.Tpad = ts->Tpad;
-    const int ct = auto_ctile(ctx, B, nd);
-    HIPCHK(timed(ctx, JC_KERNEL_WL, [&] { return launch_wl(nd, ct, wa, s); }));
+    HIPCHK(timed(ctx, JC_KERNEL_WL, [&] { return launch_wl(nd, ctx->wl_ctile, wa, ctx->num_cu, s); }));
   }
 
   LimberArgs la{};

@@ -301,7 +301,8 @@ __host__ __device__ inline int ragged_slices(int tiles, int waves, int Na, int m
 
 // launchers (defined next to their kernels)
 hipError_t launch_tables(int nd, const TablesArgs& a, hipStream_t s, int num_cu, int variant = 0);
-hipError_t launch_wl(int nd, int ctile, const WLArgs& a, hipStream_t s);
+// ctile: cosmologies per block of the forward kernel (1, 4, 8, 16; 0 = by rule)
+hipError_t launch_wl(int nd, int ctile, const WLArgs& a, int num_cu, hipStream_t s);
 // Gaussian likelihood on block-diagonal covariances (jc_likelihood.hip)
 hipError_t launch_block_inv(const double* cov, int P, int n_ell, double* inv, double* piv, hipStream_t s);
 hipError_t launch_loglike(const float* mu, int B, int P, int n_ell, const double* data, const double* prec,

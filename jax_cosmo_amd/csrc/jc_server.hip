@@ -339,7 +339,7 @@ hipError_t enqueue_pass(jc_server* S, Slot* sl, int pass, hipStream_t ps, const 
           wa.Tpad = TPAD_POOL;
           wa.dB = ta.dB;
           wa.rjobs = ta.rjobs;  // R rows in each request's tracer order
-          if ((e = launch_wl(nd, pass ? 1 : ctile, wa, st)) != hipSuccess) return e;
+          if ((e = launch_wl(nd, ctile, wa, S->ctx->num_cu, st)) != hipSuccess) return e;
         }
       } else {
         RaggedArgs ra{};

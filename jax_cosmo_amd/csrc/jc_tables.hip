@@ -141,15 +141,6 @@ JC_D void mat_mul(const Sd* a, const Sd* b, Sd* c) {  // c = a b
 // data unchanged, and uniform reads would go through the vector memory path).
 typedef const __attribute__((address_space(4))) double ConstD;
 
-// Raw buffer descriptor of `bytes` bytes at p (gfx9 word 3: 32-bit data,
-// no swizzle); a load whose offset lies past `bytes` returns zero.
-JC_D __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, bytes, 0x00020000);
-}
-JC_D float buf_f32(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-}
-
 // Cubic Hermite interpolant on [x_q, x_q + h] at fraction t, from the end
 // values f0, f1 and the end derivatives d0, d1 (per unit x).
 template <class Sd, class Tt>
@@ -1058,210 +1049,6 @@ hipError_t launch_kde(const double* z, int64_t n, const double* cz, const double
   if (n <= 0) return hipSuccess;
   const double scale = 1.0 / (sqrt(2.0 * PI) * bw) / wsum;
   hipLaunchKernelGGL(k_kde, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, z, n, cz, cw, ncat, bw, scale, out);
-  return hipGetLastError();
-}
-
-// ------------------------------------------------------------------ WL kernel
-// A block covers 64 consecutive outer nodes m (one per lane) for CT
-// cosmologies; its 4 waves split the 256 inner nodes j of the per-z Simpson
-// into contiguous quarters and their partial sums are added in LDS in a fixed
-// order (deterministic).  Every resident-table element loaded for (m, j)
-// serves CT cosmologies; NW = weak-lensing bins held in registers (>= the
-// set's count).  The last node (a = 1, z = 0) has chi = 0 and so a zero
-// kernel; the lane of the node before it writes that zero.
-constexpr int WL_M = 64;      // outer nodes per block
-constexpr int WL_SLICES = 4;  // waves per block, one quarter of j each
-
-template <int ND, int CT, int NW>
-__global__ __launch_bounds__(WL_M * WL_SLICES) void k_wl(WLArgs A) {
-  using Sf = typename Types<ND>::F;
-  constexpr int W = ND + 1;
-  extern __shared__ __align__(16) float wl_smem[];  // [CT][NCHI][2][W] tables, then [3][NACC][64] partial sums
-  float* s_tab = wl_smem;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int m = blockIdx.x * WL_M + lane;
-  const int c0 = blockIdx.y * CT;
-  const int B = A.dB ? min(*A.dB, A.B) : A.B;
-  if (c0 >= B) return;
-  for (int ct = 0; ct < CT; ++ct) {
-    const int c = c0 + ct < B ? c0 + ct : B - 1;
-    const float* src = A.chitab + (size_t)c * NCHI * 2 * W;
-    for (int e = tid; e < NCHI * 2 * W; e += WL_M * WL_SLICES) s_tab[ct * NCHI * 2 * W + e] = src[e];
-  }
-  __syncthreads();
-  const int N = A.Na - 1;  // nodes with a nonzero kernel
-  const bool active = m < N;
-  const int mm = active ? m : 0;
-  Sf chim[CT];
-  Sf acc[CT][NW];
-#pragma unroll
-  for (int ct = 0; ct < CT; ++ct) {
-    const int c = c0 + ct < B ? c0 + ct : B - 1;
-    chim[ct] = Mem<Sf>::ld(A.coef + (((size_t)c * A.Na + mm) * NCOEF + CF_CHI) * W);
-#pragma unroll
-    for (int i = 0; i < NW; ++i) acc[ct][i] = Make<Sf>::c(0.0);
-  }
-  if (active) {
-    // j = 0 is z' = z, where chi' == chi and the integrand is exactly zero
-    constexpr int JS = (NWL_J - 1) / WL_SLICES;
-    const int j0 = 1 + wave * JS;
-    // raw buffer loads: the table bases and the bin row offsets stay in
-    // SGPRs, so one 32-bit byte offset per lane advances per j (no 64-bit
-    // address arithmetic in the loop); loads past a table's end read zero
-    const int rs = NWL_J * A.Na;  // elements per table row block (and per bin of the weights)
-    const __amdgpu_buffer_rsrc_t rL = buf_rsrc(A.Lidx, rs);
-    const __amdgpu_buffer_rsrc_t rD = buf_rsrc(A.delta, rs * 4);
-    const __amdgpu_buffer_rsrc_t rN = buf_rsrc(A.Nw, rs * 4 * NW);
-    int oL = j0 * A.Na + m;
-    int o4 = 4 * oL;
-    for (int j = j0; j < j0 + JS; ++j, oL += A.Na, o4 += 4 * A.Na) {
-      const int L = __builtin_amdgcn_raw_buffer_load_b8(rL, oL, 0, 0);
-      const float dl = buf_f32(rD, o4, 0);
-      float nw[NW];
-#pragma unroll
-      for (int i = 0; i < NW; ++i) nw[i] = buf_f32(rN, o4, i * rs * 4);  // zero rows past nw
-      // cosmology-major tables: lanes (consecutive m, close segments L) read
-      // nearby words of one table
-      const float* tL = s_tab + L * 2 * W;
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        const float* t = tL + ct * NCHI * 2 * W;
-        Sf chi_l, sl;
-        if constexpr (W == 1) {  // one 8-byte read at a constant offset per cosmology
-          const float2 v = *reinterpret_cast<const float2*>(t);
-          chi_l = v.x;
-          sl = v.y;
-        } else {
-          chi_l = Mem<Sf>::ld(t);
-          sl = Mem<Sf>::ld(t + W);
-        }
-        // chi' = clip(interp, 0) (background.py:242): with chi >= 0 the clip
-        // cannot change clip(chi' - chi, 0) / clip(chi', 1) (probes.py:51),
-        // so it is left out
-        Sf chip = chi_l + sl * dl;
-        Sf num = maxc(chip - chim[ct], 0.0f);
-        Sf f = num * jm::rcp(maxc(chip, 1.0f));
-        // bins past the set's count carry nw = 0 and f is finite: no guard
-#pragma unroll
-        for (int i = 0; i < NW; ++i) acc[ct][i] = acc[ct][i] + nw[i] * f;
-      }
-    }
-    // single source planes (probes.py:53-64): clip(chi_s - chi, 0) / clip(chi_s, 1)
-    if (wave == 0) {
-#pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        if (i < A.nw) {
-          const WLSource sp = A.src[i];
-          if (sp.on) {
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-              const float* t = s_tab + ((ct * NCHI + sp.L) * 2) * W;
-              Sf chis = maxc(Mem<Sf>::ld(t) + Mem<Sf>::ld(t + W) * sp.off, 0.0f);
-              Sf f = maxc(chis - chim[ct], 0.0f) * jm::rcp(maxc(chis, 1.0f));
-              acc[ct][i] = acc[ct][i] + sp.fac * f;
-            }
-          }
-        }
-      }
-    }
-  }
-  __syncthreads();  // the tables are no longer read: reuse the space
-  float* red = wl_smem;
-  if (wave > 0) {
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int i = 0; i < NW; ++i)
-        Mem<Sf>::st(&red[(((wave - 1) * CT + ct) * NW + i) * W * 64 + lane], acc[ct][i], 64);
-  }
-  __syncthreads();
-  if (wave != 0 || m >= N) return;
-  // R columns of each bin and cosmology, taken before any store: the pool
-  // column, or (served batches) every position of the request that
-  // selects the bin; all MAXT positions are tested so that the loads issue
-  // together
-  uint32_t cm[CT][NW];
-#pragma unroll
-  for (int ct = 0; ct < CT; ++ct) {
-    const int c = c0 + ct < B ? c0 + ct : B - 1;
-    int T = 0;
-    int sel[MAXT];
-    if (A.rjobs) {
-      T = A.rjobs[c].T;
-#pragma unroll
-      for (int p = 0; p < MAXT; ++p) sel[p] = A.rjobs[c].sel[p];
-    }
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      uint32_t mk = 0;
-      if (i < A.nw) {
-        const int cl = A.col[i];
-        if (A.rjobs) {
-#pragma unroll
-          for (int p = 0; p < MAXT; ++p) mk |= (p < T && sel[p] == cl ? 1u : 0u) << p;
-        } else {
-          mk = 1u << cl;
-        }
-      }
-      cm[ct][i] = mk;
-    }
-  }
-#pragma unroll
-  for (int ct = 0; ct < CT; ++ct) {
-    const int c = c0 + ct;
-    if (c >= B) break;
-    Sf wl = Mem<Sf>::ld(A.crec + ((size_t)c * NCREC + CR_WLCONST) * W);
-    Sf pref = (A.zp1[m] * chim[ct]) * wl;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      if (i < A.nw) {
-        Sf r = acc[ct][i];
-        for (int w = 1; w < WL_SLICES; ++w)
-          r = r + Mem<Sf>::ld(&red[(((w - 1) * CT + ct) * NW + i) * W * 64 + lane], 64);
-        r = r * pref;
-        for (uint32_t mk = cm[ct][i]; mk; mk &= mk - 1) {
-          const int cl = __builtin_ctz(mk);
-          float* dst = A.R + (((size_t)c * A.Na + m) * A.Tpad + cl) * W;
-          Sf v = r;
-          if (A.ia) v = v + Mem<Sf>::ld(dst);  // the NLA term written by the table kernel
-          Mem<Sf>::st(dst, v);
-          // the a = 1 node: zero lensing kernel (chi = 0), the NLA term stays
-          if (m == N - 1 && !A.ia) Mem<Sf>::st(A.R + (((size_t)c * A.Na + N) * A.Tpad + cl) * W, Make<Sf>::c(0.0));
-        }
-      }
-    }
-  }
-}
-
-template <int ND, int CT, int NW>
-static void wl_launch_nw(const WLArgs& a, hipStream_t s) {
-  constexpr int W = ND + 1;
-  const size_t tab = (size_t)CT * NCHI * 2 * W;
-  const size_t red = (size_t)(WL_SLICES - 1) * CT * NW * W * 64;
-  const size_t sm = (tab > red ? tab : red) * sizeof(float);
-  const dim3 grid((a.Na - 1 + WL_M - 1) / WL_M, (a.B + CT - 1) / CT);
-  hipLaunchKernelGGL((k_wl<ND, CT, NW>), grid, dim3(WL_M * WL_SLICES), sm, s, a);
-}
-
-template <int ND, int CT>
-static void wl_launch_ct(const WLArgs& a, hipStream_t s) {
-  if (a.nw <= 5) wl_launch_nw<ND, CT, 5>(a, s);
-  else wl_launch_nw<ND, CT, NWL_MAX>(a, s);
-}
-
-hipError_t launch_wl(int nd, int ctile, const WLArgs& a, hipStream_t s) {
-  if (a.nw < 1 || a.nw > NWL_MAX) return hipErrorInvalidValue;
-  switch (nd * 32 + ctile) {
-    case 0 * 32 + 1: wl_launch_ct<0, 1>(a, s); break;
-    case 0 * 32 + 4: wl_launch_ct<0, 4>(a, s); break;
-    case 0 * 32 + 8: wl_launch_ct<0, 8>(a, s); break;
-    case 0 * 32 + 16: wl_launch_ct<0, 16>(a, s); break;
-    case 1 * 32 + 1: wl_launch_ct<1, 1>(a, s); break;
-    case 7 * 32 + 1: wl_launch_ct<7, 1>(a, s); break;
-    default: return hipErrorInvalidValue;
-  }
   return hipGetLastError();
 }
 
