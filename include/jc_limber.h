@@ -163,6 +163,12 @@ int jc_angular_cl_jvp(jc_ctx* ctx, const double* cosmo, const double* tangent, i
                       int64_t set_id, const double* ell, int64_t n_ell, int64_t n_z,
                       float* cl, float* cl_dot, int32_t flags);
 
+/* jac[B][P][n_ell][7] = dC/d(Omega_c, Omega_b, h, n_s, sigma8, w0, wa): the
+ * seven directional derivatives in one pass (jax.jacfwd of angular_cl).  Host
+ * pointers only (flags 0); returns after the copy. */
+int jc_angular_cl_jacobian(jc_ctx* ctx, const double* cosmo, int64_t B, int64_t set_id, const double* ell,
+                           int64_t n_ell, int64_t n_z, float* jac, int32_t flags);
+
 /* Adjoint: theta_bar[B][7] = sum_{p,l} cl_bar[b][p][l] dC[b][p][l]/dtheta.
  * Replaces jax.grad / jax.vjp of angular_cl (core.py:98-141 pytrees). */
 int jc_angular_cl_vjp(jc_ctx* ctx, const double* cosmo, int64_t B, int64_t set_id,

@@ -20,7 +20,7 @@ EXPORTS = (
     "jc_ctx_create", "jc_ctx_destroy", "jc_ctx_set_stream", "jc_ctx_reset_stream", "jc_synchronize",
     "jc_tracers_register", "jc_tracers_register_catalogs", "jc_tracers_register_host", "jc_tracers_release",
     "jc_angular_cl",
-    "jc_angular_cl_noalloc", "jc_angular_cl_jvp",
+    "jc_angular_cl_noalloc", "jc_angular_cl_jvp", "jc_angular_cl_jacobian",
     "jc_angular_cl_vjp", "jc_matter_power", "jc_background", "jc_background_ex", "jc_set_growth", "jc_set_tiles", "jc_get_tiles", "jc_set_tables_variant",
     "jc_set_forward_options", "jc_set_models", "jc_sparse_inv", "jc_gaussian_loglike", "jc_gaussian_loglike_grad",
     "jc_dense_cholesky", "jc_dense_solve", "jc_gaussian_loglike_dense", "jc_gaussian_loglike_grad_dense",
@@ -107,6 +107,7 @@ def load_library(path=LIB_PATH):
             "jc_angular_cl": [_P, _P, _I64, _I64, _P, _I64, _I64, _P, _I32],
             "jc_angular_cl_noalloc": [_P, _P, _I64, _I64, _P, _I64, _I64, _P, _I32],
             "jc_angular_cl_jvp": [_P, _P, _P, _I64, _I64, _P, _I64, _I64, _P, _P, _I32],
+            "jc_angular_cl_jacobian": [_P, _P, _I64, _I64, _P, _I64, _I64, _P, _I32],
             "jc_angular_cl_vjp": [_P, _P, _I64, _I64, _P, _I64, _I64, _P, _P, _I32],
             "jc_matter_power": [_P, _P, _P, _P, _I64, _P, _P],
             "jc_background": [_P, _P, _P, _I64, _P, _P],
@@ -290,6 +291,19 @@ class Context:
             check(self.lib.jc_angular_cl_jvp(self.handle, _ptr(cosmo), _ptr(tangent), B, set_id,
                                              _ptr(ell), ell.shape[0], n_z, _ptr(out), _ptr(dot), 0))
         return out, dot
+
+    def angular_cl_jacobian(self, cosmo, set_id, ell, n_z, n_pairs):
+        """dC/dtheta [B, P, n_ell, 7]."""
+        cosmo = np.ascontiguousarray(cosmo, dtype=np.float64).reshape(-1, 8)
+        ell = np.ascontiguousarray(ell, dtype=np.float64).reshape(-1)
+        B = cosmo.shape[0]
+        self._check_pairs(set_id, n_pairs)
+        jac = np.empty((B, n_pairs, ell.shape[0], 7), dtype=np.float32)
+        with self._lock:
+            self.reset_stream()
+            check(self.lib.jc_angular_cl_jacobian(self.handle, _ptr(cosmo), B, set_id, _ptr(ell),
+                                                  ell.shape[0], n_z, _ptr(jac), 0))
+        return jac
 
     def angular_cl_vjp(self, cosmo, set_id, ell, n_z, cl_bar):
         cosmo = np.ascontiguousarray(cosmo, dtype=np.float64).reshape(-1, 8)

@@ -89,8 +89,8 @@ def angular_cl_torch(params, ell, probes, n_z=512):
 
 
 def angular_cl_jacobian(cosmo_params, ell, probes, n_z=512, transfer_fn=None, nonlinear_fn=None, gamma=None):
-    """dC/dtheta [B, P, n_ell, 7] by seven device JVPs (forward mode), the
-    counterpart of jax.jacfwd of the mean (notebook jax-cosmo-intro, cell 46)."""
+    """dC/dtheta [B, P, n_ell, 7] by forward mode, all directions in one
+    pass, the counterpart of jax.jacfwd of the mean (notebook jax-cosmo-intro, cell 46)."""
     from . import power, transfer
     from .angular_cl import _check_fns, _n_cls, tracer_entries
 
@@ -99,14 +99,7 @@ def angular_cl_jacobian(cosmo_params, ell, probes, n_z=512, transfer_fn=None, no
     set_id = dctx.tracer_set(tracer_entries(probes))
     P = _n_cls(probes)
     cp = np.asarray(cosmo_params, dtype=np.float64).reshape(-1, 8)
-    B = cp.shape[0]
-    jac = np.empty((B, P, len(np.atleast_1d(ell)), 7), dtype=np.float32)
-    for d in range(7):
-        t = np.zeros((B, 7))
-        t[:, d] = 1.0
-        _, dot = dctx.angular_cl_jvp(cp, t, set_id, np.asarray(ell, dtype=np.float64), n_z, P)
-        jac[..., d] = dot
-    return jac
+    return dctx.angular_cl_jacobian(cp, set_id, np.asarray(ell, dtype=np.float64), n_z, P)
 
 
 def fisher_matrix(cosmo_params, ell, probes, C, n_z=512, transfer_fn=None, nonlinear_fn=None, gamma=None):
@@ -130,7 +123,7 @@ def log_likelihood_hessian(cosmo_params, ell, probes, data, C, n_z=512, transfer
     jax.hessian of the notebook's likelihood at its fiducial cosmology
     (jax-cosmo-intro cells 35-39, F = -H), where
 
-        H = -J^T C^-1 J,   J = dmu/dtheta (seven device JVPs).
+        H = -J^T C^-1 J,   J = dmu/dtheta (forward mode).
 
     Away from such a point the full Hessian adds sum_k (C^-1 r)_k d2mu_k,
     which this function leaves out (it then returns the Gauss-Newton

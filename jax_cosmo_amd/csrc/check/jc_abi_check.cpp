@@ -90,6 +90,10 @@ static void device_checks(jc_ctx* ctx) {
   std::vector<double> tan(B * 7, 0.5), th(B * 7);
   CHECK(jc_angular_cl_jvp(ctx, cosmo.data(), tan.data(), B, sid, ell.data(), L, 256, cl.data(), dot.data(), 0) ==
             JC_OK, "jvp");
+  std::vector<float> jac((size_t)B * P * L * 7);
+  CHECK(jc_angular_cl_jacobian(ctx, cosmo.data(), B, sid, ell.data(), L, 256, jac.data(), 0) == JC_OK, "jacobian");
+  for (float v : jac) CHECK(std::isfinite(v), "finite jacobian");
+  CHECK(jc_angular_cl_jacobian(ctx, cosmo.data(), B, sid, ell.data(), L, 255, jac.data(), 0) == JC_E_ARG, "odd n_z");
   CHECK(jc_angular_cl_vjp(ctx, cosmo.data(), B, sid, ell.data(), L, 256, cbar.data(), th.data(), 0) == JC_OK, "vjp");
   for (double v : th) CHECK(std::isfinite(v), "finite vjp");
   // likelihood algebra on the C_ell of cosmology 0

@@ -499,9 +499,13 @@ hipError_t timed(jc_ctx* ctx, int kind, F&& launch) {
 // sc != null (forward calls only): every per-call buffer comes from the
 // scratch regions of sc, and the tracer set's tables for n_z must already be
 // resident, so the call allocates nothing.
+// jac != null (nd = 1, device pointers): the cosmologies are B / 7 groups of
+// seven equal rows, jac_seeds their seeds on the device, one direction a row;
+// dC/dtheta goes to jac[B / 7][P][n_ell][7], and cl and cl_dot are workspaces.
 int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent, int64_t B,
                  int64_t set_id, const double* ell, int64_t n_ell, int64_t n_z, float* cl,
-                 float* cl_dot, const float* cl_bar, double* theta_bar, int32_t flags, Bump* sc = nullptr) {
+                 float* cl_dot, const float* cl_bar, double* theta_bar, int32_t flags, Bump* sc = nullptr,
+                 const double* jac_seeds = nullptr, float* jac = nullptr) {
   if (!ctx) return fail(JC_E_ARG, "null context");
   if (B < 1 || n_ell < 1) return fail(JC_E_ARG, "B and n_ell must be >= 1");
   if (n_z < 2 || (n_z % 2) != 0) return fail(JC_E_ARG, "N must be an even integer >= 2 (integrate.py:193)");
@@ -543,7 +547,9 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
   if (rc) return rc;
   const double* d_seeds = nullptr;
   std::vector<double> seeds;
-  if (nd > 0) {
+  if (jac) {
+    d_seeds = jac_seeds;
+  } else if (nd > 0) {
     // d param_i / d direction: the 7 differentiable parameters skip Omega_k
     static const int pidx[7] = {0, 1, 2, 3, 4, 6, 7};
     std::vector<double> tan_h;
@@ -695,6 +701,11 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
   la.out = d_out;
   la.out_t = d_out_t;
   HIPCHK(timed(ctx, JC_KERNEL_LIMBER, [&] { return launch_limber(nd, T, la, s); }));
+  if (jac) {
+    HIPCHK(launch_jac_sum(la.slices > 1 ? la.part + (size_t)la.slices * nout : d_out_t, la.slices, B / 7,
+                          (int64_t)P * n_ell, jac, s));
+    return JC_OK;
+  }
   if (la.slices > 1) {
     HIPCHK(launch_slice_sum(la.part, la.slices, (int64_t)nout, d_out, s));
     if (nd == 1) HIPCHK(launch_slice_sum(la.part + (size_t)la.slices * nout, la.slices, (int64_t)nout, d_out_t, s));
@@ -930,6 +941,59 @@ int jc_angular_cl_jvp(jc_ctx* ctx, const double* cosmo, const double* tangent, i
                       const double* ell, int64_t n_ell, int64_t n_z, float* cl, float* cl_dot, int32_t flags) {
   if (!cosmo || !tangent || !ell || !cl || !cl_dot) return fail(JC_E_ARG, "null array argument");
   return run_pipeline(ctx, 1, cosmo, tangent, B, set_id, ell, n_ell, n_z, cl, cl_dot, nullptr, nullptr, flags);
+}
+
+// The seven directions of a cosmology are seven rows of one directional
+// derivative: one launch of each kernel instead of seven of a seventh of the
+// blocks, which for a few cosmologies left the chip idle (one cosmology, 10 tracers,
+// 100 ell, n_z 512: 1198 -> 137 us a call).  At most JAC_ROWS rows
+// a launch (four table workgroups a compute unit) and JAC_COLS columns (where one
+// cosmology's seven rows fit them) bound the workspaces.
+int jc_angular_cl_jacobian(jc_ctx* ctx, const double* cosmo, int64_t B, int64_t set_id, const double* ell,
+                           int64_t n_ell, int64_t n_z, float* jac, int32_t flags) {
+  constexpr int64_t JAC_ROWS = 1024, JAC_COLS = 1 << 19;
+  if (!ctx || !cosmo || !ell || !jac) return fail(JC_E_ARG, "null argument");
+  if (flags & JC_DEVICE_PTRS) return fail(JC_E_UNSUPPORTED, "jc_angular_cl_jacobian takes host pointers");
+  if (B < 1 || n_ell < 1) return fail(JC_E_ARG, "B and n_ell must be >= 1");
+  if (B * n_ell > (int64_t)1 << 30) return fail(JC_E_ARG, "too many columns");
+  auto it = ctx->sets.find(set_id);
+  if (it == ctx->sets.end()) return fail(JC_E_ARG, "unknown tracer set %lld", (long long)set_id);
+  int rc = check_cosmo_host(cosmo, B);
+  if (rc) return rc;
+  HIPCHK(hipSetDevice(ctx->device));
+  hipStream_t s = ctx->stream;
+  const int T = it->second->T;
+  const size_t np = (size_t)(T * (T + 1) / 2) * n_ell;  // outputs per cosmology and direction
+  const int64_t fit = std::min(JAC_ROWS, JAC_COLS / n_ell) / 7;  // cosmologies a launch
+  const int64_t nb = std::min(B, std::max<int64_t>(1, fit));
+  static const int pidx[7] = {0, 1, 2, 3, 4, 6, 7};
+  // ell, and per chunk the parameter and seed rows, in one upload
+  std::vector<double> up((size_t)n_ell + (size_t)nb * 7 * 16);
+  memcpy(up.data(), ell, (size_t)n_ell * sizeof(double));
+  HIPCHK(ctx->params.reserve(up.size()));
+  HIPCHK(ctx->out.reserve((size_t)nb * 7 * np));
+  HIPCHK(ctx->out_t.reserve((size_t)nb * 7 * np));
+  HIPCHK(ctx->jac.reserve((size_t)nb * 7 * np));
+  for (int64_t b0 = 0; b0 < B; b0 += nb) {
+    const int64_t n = std::min(nb, B - b0);
+    double* pr = up.data() + n_ell;
+    double* sd = pr + n * 7 * 8;
+    std::fill(sd, sd + n * 7 * 8, 0.0);
+    for (int64_t r = 0; r < n * 7; ++r) {
+      memcpy(pr + r * 8, cosmo + (b0 + r / 7) * 8, 8 * sizeof(double));
+      sd[r * 8 + pidx[r % 7]] = 1.0;
+    }
+    const double* dp = ctx->params.p;
+    HIPCHK(hipMemcpyAsync(ctx->params.p, up.data(), ((size_t)n_ell + (size_t)n * 7 * 16) * sizeof(double),
+                          hipMemcpyHostToDevice, s));
+    rc = run_pipeline(ctx, 1, dp + n_ell, nullptr, n * 7, set_id, dp, n_ell, n_z, ctx->out.p, ctx->out_t.p, nullptr,
+                      nullptr, JC_DEVICE_PTRS, nullptr, dp + n_ell + n * 7 * 8, ctx->jac.p);
+    if (rc) return rc;
+    HIPCHK(hipMemcpyAsync(jac + (size_t)b0 * 7 * np, ctx->jac.p, (size_t)n * 7 * np * sizeof(float),
+                          hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));  // up and the device buffers are reused by the next chunk
+  }
+  return JC_OK;
 }
 
 int jc_angular_cl_vjp(jc_ctx* ctx, const double* cosmo, int64_t B, int64_t set_id, const double* ell,

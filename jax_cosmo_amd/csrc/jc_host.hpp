@@ -204,7 +204,7 @@ struct jc_ctx {
   // solves, inverses of the factor's diagonal blocks
   DevBuf<double> dn_mat, dn_dlog, dn_z, dn_x, dn_inv;
   DevBuf<int> dn_bad;
-  DevBuf<float> chitab, coef, crec, R, out, out_t, cbar, theta_col, part;
+  DevBuf<float> chitab, coef, crec, R, out, out_t, jac, cbar, theta_col, part;
   DevBuf<float4> ehtab;
   DevBuf<float> ehtab7;
   int waves = 0, wl_ctile = 0, tables_variant = 0;

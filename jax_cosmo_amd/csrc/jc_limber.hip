@@ -338,6 +338,32 @@ hipError_t launch_slice_sum(const float* part, int slices, int64_t n, float* out
   return hipGetLastError();
 }
 
+// Jacobian: jac[b][o][d] = part[b * 7 + d][o] added over the slices of
+// part[slices][B * 7][n], in order.  A thread takes one o of one cosmology: the
+// seven rows are read coalesced, its seven results lie together.
+__global__ void k_jac_sum(const float* __restrict__ part, int slices, int64_t B, int64_t n, float* __restrict__ jac) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= B * n) return;
+  const int64_t b = e / n, o = e - b * n;
+  const float* p = part + b * 7 * n + o;
+  float s[7];
+#pragma unroll
+  for (int d = 0; d < 7; ++d) s[d] = p[d * n];
+  for (int k = 1; k < slices; ++k) {
+    p += B * 7 * n;
+#pragma unroll
+    for (int d = 0; d < 7; ++d) s[d] += p[d * n];
+  }
+#pragma unroll
+  for (int d = 0; d < 7; ++d) jac[e * 7 + d] = s[d];
+}
+
+hipError_t launch_jac_sum(const float* part, int slices, int64_t B, int64_t n, float* jac, hipStream_t s) {
+  if (B <= 0 || n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_jac_sum, dim3((unsigned)((B * n + 255) / 256)), dim3(256), 0, s, part, slices, B, n, jac);
+  return hipGetLastError();
+}
+
 // ------------------------------------------------------------------ matrix-core contraction
 // Forward kernel with the pair contraction on the matrix cores: for one
 // cosmology C_p(ell) = sum_a K_p(a) M(a, ell) with K_p = R_i R_j is a GEMM
