@@ -198,6 +198,12 @@ int jc_sparse_inv(jc_ctx* ctx, const double* cov, int64_t P, int64_t n_ell, doub
 int jc_gaussian_loglike(jc_ctx* ctx, const float* mu, int64_t B, int64_t P, int64_t n_ell, const double* data,
                         const double* prec, double c0, double* loglike, float* dloglike_dmu, int32_t flags);
 
+/* The same from the covariance [P][P][n_ell] itself, include_logdet != 0 adding
+ * +1/2 log |det C|.  Host pointers only (flags 0); JC_E_ARG for a singular
+ * block. */
+int jc_gaussian_loglike_cov(jc_ctx* ctx, const float* mu, int64_t B, int64_t P, int64_t n_ell, const double* data,
+                            const double* cov, int32_t include_logdet, double* loglike, int32_t flags);
+
 /* The same for the means angular_cl(cosmo_b) of a registered tracer set,
  * with grad[b][7] = d loglike_b / d(Omega_c, Omega_b, h, n_s, sigma8, w0, wa):
  * jax.grad of a Gaussian likelihood through angular_cl (the likelihood of

@@ -22,7 +22,7 @@ EXPORTS = (
     "jc_angular_cl",
     "jc_angular_cl_noalloc", "jc_angular_cl_jvp", "jc_angular_cl_jacobian",
     "jc_angular_cl_vjp", "jc_matter_power", "jc_background", "jc_background_ex", "jc_set_growth", "jc_set_tiles", "jc_get_tiles", "jc_set_tables_variant",
-    "jc_set_forward_options", "jc_set_models", "jc_sparse_inv", "jc_gaussian_loglike", "jc_gaussian_loglike_grad",
+    "jc_set_forward_options", "jc_set_models", "jc_sparse_inv", "jc_gaussian_loglike", "jc_gaussian_loglike_cov", "jc_gaussian_loglike_grad",
     "jc_dense_cholesky", "jc_dense_solve", "jc_gaussian_loglike_dense", "jc_gaussian_loglike_grad_dense",
     "jc_sigma8_norm", "jc_debug_tables", "jc_profile_enable", "jc_profile_select", "jc_profile_read", "jc_last_error", "jc_version",
 )
@@ -120,6 +120,7 @@ def load_library(path=LIB_PATH):
             "jc_set_models": [_P, _I32, _I32],
             "jc_sparse_inv": [_P, _P, _I64, _I64, _P, _P, _I32],
             "jc_gaussian_loglike": [_P, _P, _I64, _I64, _I64, _P, _P, ctypes.c_double, _P, _P, _I32],
+            "jc_gaussian_loglike_cov": [_P, _P, _I64, _I64, _I64, _P, _P, _I32, _P, _I32],
             "jc_gaussian_loglike_grad": [_P, _P, _I64, _I64, _P, _I64, _I64, _P, _P, ctypes.c_double, _P, _P,
                                          _I32],
             "jc_dense_cholesky": [_P, _P, _I64, _P, _P, _I32],
@@ -518,6 +519,20 @@ class _Likelihood:
                                                float(c0), _ptr(ll), _ptr(dmu) if want_dmu else None, 0))
         return (ll, dmu) if want_dmu else ll
 
+    def gaussian_loglike_cov(self, mu, data, C, include_logdet=True):
+        """Log-likelihoods of B means [B][P][n_ell] under the block-diagonal
+        covariance C [P][P][n_ell]."""
+        C = _sparse_ok(C)
+        P, _, n_ell = C.shape
+        mu = np.ascontiguousarray(np.asarray(mu).reshape(-1, P, n_ell), dtype=np.float32)
+        data = _f64(data).reshape(P, n_ell)
+        ll = np.empty(mu.shape[0])
+        with self._lock:
+            self.reset_stream()
+            check(self.lib.jc_gaussian_loglike_cov(self.handle, _ptr(mu), mu.shape[0], P, n_ell, _ptr(data), _ptr(C),
+                                                   int(bool(include_logdet)), _ptr(ll), 0))
+        return ll
+
     def gaussian_loglike_grad(self, cosmo, set_id, ell, n_z, data, prec, c0=0.0):
         cosmo = _f64(cosmo).reshape(-1, 8)
         ell = _f64(ell).reshape(-1)
@@ -647,7 +662,7 @@ class _Likelihood:
         return ll.cpu().numpy(), g.cpu().numpy()
 
 
-for _name in ("sparse_inv", "gaussian_loglike", "gaussian_loglike_grad", "gaussian_loglike_grad_dev",
+for _name in ("sparse_inv", "gaussian_loglike", "gaussian_loglike_cov", "gaussian_loglike_grad", "gaussian_loglike_grad_dev",
               "dense_cholesky", "dense_solve", "gaussian_loglike_dense", "gaussian_loglike_grad_dense"):
     setattr(Context, _name, getattr(_Likelihood, _name))
 

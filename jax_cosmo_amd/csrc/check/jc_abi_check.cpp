@@ -106,6 +106,10 @@ static void device_checks(jc_ctx* ctx) {
   double logdet = 0.0, ll[B], g[B * 7];
   CHECK(jc_sparse_inv(ctx, cov.data(), P, L, inv.data(), &logdet, 0) == JC_OK, "sparse_inv");
   CHECK(jc_gaussian_loglike(ctx, cl.data(), B, P, L, data.data(), inv.data(), 0.0, ll, nullptr, 0) == JC_OK, "loglike");
+  double llc[B];
+  CHECK(jc_gaussian_loglike_cov(ctx, cl.data(), B, P, L, data.data(), cov.data(), 0, llc, 0) == JC_OK, "loglike_cov");
+  for (int b = 0; b < B; ++b) CHECK(fabs(llc[b] - ll[b]) <= 1e-9 * fabs(ll[b]), "loglike_cov equals loglike");
+  CHECK(jc_gaussian_loglike_cov(ctx, cl.data(), B, 65, L, data.data(), cov.data(), 0, llc, 0) == JC_E_ARG, "P of 65");
   CHECK(jc_gaussian_loglike_grad(ctx, cosmo.data(), B, sid, ell.data(), L, 256, data.data(), inv.data(), 0.0, ll, g,
                                  0) == JC_OK, "loglike_grad");
   // dense algebra on a small matrix

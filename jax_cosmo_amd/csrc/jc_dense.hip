@@ -23,24 +23,18 @@
 #include <algorithm>
 
 #include "jc_kernels.hpp"
+#include "jc_mma64.hpp"
 
 namespace jc {
 
 constexpr int DB = 64;              // panel width and tile size
 constexpr int SB = DENSE_SOLVE_BLOCK;  // rows a solve step takes
 
-typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
 // (Kernels here ask for 2 waves per SIMD: with a budget above 256 registers the
 // compiler keeps accumulators in the accumulation file and copies them in and
 // out of every product's loop.)
-// D[i][j] += sum_k A[i][k] B[k][j] over 4 k: lane l passes A[l % 16][l / 16]
-// and B[l / 16][l % 16] and holds D[l / 16 + 4 r][l % 16] in register r
-__device__ __forceinline__ d4 mfma64(double a, double b, d4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
 // Operands of 16 k: lane l takes k = 4 (l / 16) .. + 3 of row l % 16 (element q
 // of both operands in one instruction, so any assignment of k to lanes serves).
 // row: p[0 .. n) along k, n valid elements from the lane's first (n >= 4: all).
@@ -67,11 +61,6 @@ __device__ __forceinline__ d4 frag_col(const double* p, size_t ld, int n) {
     if (q < n) v[q] = p[q * ld];
   return v;
 }
-__device__ __forceinline__ void mma16(const d4& a, const d4& b, d4& c) {
-#pragma unroll
-  for (int q = 0; q < 4; ++q) c = mfma64(a[q], b[q], c);
-}
-
 // n steps of 16 k with the operands of the next D in flight (a load from L
 // outside the L2 takes longer than a step's products): load(s, q) fills slot q
 // with step s, use(q) consumes it.  n is uniform over the wave.

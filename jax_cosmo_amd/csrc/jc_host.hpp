@@ -198,7 +198,7 @@ struct jc_ctx {
   // workspace
   DevBuf<double> params, seeds, ell, theta, dbg, pk_k, pk_a, pk_out;
   // likelihood workspace: inputs staged from host, mean, cotangent, partials
-  DevBuf<double> lk_cosmo, lk_ell, lk_data, lk_prec, lk_part, lk_out, lk_grad, lk_piv;
+  DevBuf<double> lk_cosmo, lk_ell, lk_data, lk_prec, lk_part, lk_out, lk_grad, lk_inv;
   DevBuf<float> lk_mu, lk_s;
   // dense likelihood workspace: staged matrix, log L_ii, non-SPD flag, [B][N]
   // solves, inverses of the factor's diagonal blocks

@@ -304,9 +304,18 @@ hipError_t launch_tables(int nd, const TablesArgs& a, hipStream_t s, int num_cu,
 // ctile: cosmologies per block of the forward kernel (1, 4, 8, 16; 0 = by rule)
 hipError_t launch_wl(int nd, int ctile, const WLArgs& a, int num_cu, hipStream_t s);
 // Gaussian likelihood on block-diagonal covariances (jc_likelihood.hip)
-hipError_t launch_block_inv(const double* cov, int P, int n_ell, double* inv, double* piv, hipStream_t s);
+// (strides of element (p, q, l) of a precision array: (p P + q) pair + l ell)
+struct PrecLayout {
+  int64_t pair, ell;
+};
+// the reference's sparse format [P][P][n_ell], and one block after the other
+inline PrecLayout prec_sparse(int64_t n_ell) { return {n_ell, 1}; }
+inline PrecLayout prec_blocks(int64_t P) { return {1, P * P}; }
+// ld[n_ell][2]: |det| of block l = ld[l][0] 2^ld[l][1]
+hipError_t launch_block_inv(const double* cov, int P, int n_ell, double* inv, PrecLayout lay, double* ld,
+                            hipStream_t s);
 hipError_t launch_loglike(const float* mu, int B, int P, int n_ell, const double* data, const double* prec,
-                          double c0, float* s_out, double* part, double* loglike, hipStream_t s);
+                          PrecLayout lay, double c0, float* s_out, double* part, double* loglike, hipStream_t s);
 // Gaussian KDE n(z) (redshift.py:126-156) at n points from a catalog sorted
 // by redshift: out[p] = sum_k w_k N(z_p - z_k; bw) / sum_k w_k
 // growth rate and transverse distance of a background call (FP64 slots 6, 7)

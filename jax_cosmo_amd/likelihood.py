@@ -211,12 +211,8 @@ def log_likelihood_batch(data, mu, C, include_logdet=True):
         c0 = 0.5 * f.logdet if include_logdet else 0.0  # likelihood.py:61
         mu = np.asarray(mu).reshape(-1, f.N)
         return ctx.gaussian_loglike_dense(mu, data, f.L, c0)
-    prec, logdet = ctx.sparse_inv(C)
     # likelihood.py:61 returns -1/2 (r^T C^-1 r - log det C)
-    c0 = 0.5 * logdet if include_logdet else 0.0
-    P, _, n_ell = np.shape(C)
-    mu = np.asarray(mu).reshape(-1, P, n_ell)
-    return ctx.gaussian_loglike(mu, data, prec, c0)
+    return ctx.gaussian_loglike_cov(mu, data, C, include_logdet)
 
 
 def log_likelihood_and_grad(cosmo_params, ell, probes, data, C, include_logdet=True, n_z=512, transfer_fn=None,
