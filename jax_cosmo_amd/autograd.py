@@ -10,16 +10,19 @@ import numpy as np
 import torch
 
 from ._native import default_context
+from .angular_cl import _device_ell
 
 GRAD_INDEX = (0, 1, 2, 3, 4, 6, 7)  # positions of theta in the 8-parameter vector
 
 
 def _assemble(theta, omega_k):
-    B = theta.shape[0]
-    params = torch.empty((B, 8), dtype=torch.float64, device=theta.device)
-    params[:, list(GRAD_INDEX)] = theta.detach().to(torch.float64)
+    # slices, not an index list: the list would be uploaded on every call
+    theta = theta.detach().expand(theta.shape[0], 7)
+    params = torch.empty((theta.shape[0], 8), dtype=torch.float64, device=theta.device)
+    params[:, :5] = theta[:, :5]
     params[:, 5] = omega_k
-    return params.contiguous()
+    params[:, 6:] = theta[:, 5:]
+    return params
 
 
 class AngularClFunction(torch.autograd.Function):
@@ -31,7 +34,7 @@ class AngularClFunction(torch.autograd.Function):
         params = _assemble(theta, omega_k)
         ell64 = np.ascontiguousarray(np.asarray(ell, dtype=np.float64).reshape(-1))
         if theta.is_cuda:
-            el = torch.as_tensor(ell64, device=theta.device)
+            el = _device_ell(ell64, theta.device)
             out = torch.empty((params.shape[0], n_pairs, el.shape[0]), dtype=torch.float32,
                               device=theta.device)
             dctx.angular_cl_dev(params.data_ptr(), params.shape[0], set_id, el.data_ptr(),
@@ -53,7 +56,7 @@ class AngularClFunction(torch.autograd.Function):
         dctx.set_growth(models[2])
         g32 = grad.detach().to(torch.float32).contiguous()
         if params.is_cuda:
-            el = torch.as_tensor(ell64, device=params.device)
+            el = _device_ell(ell64, params.device)
             th = torch.empty((params.shape[0], 7), dtype=torch.float64, device=params.device)
             dctx.angular_cl_vjp_dev(params.data_ptr(), params.shape[0], set_id, el.data_ptr(),
                                     el.shape[0], n_z, g32.data_ptr(), th.data_ptr(),
@@ -69,17 +72,13 @@ def angular_cl_torch(params, ell, probes, n_z=512):
     Returns [B=1, n_cls, n_ell]; gradients reach the torch parameters."""
     from .angular_cl import _n_cls, tracer_entries
 
-    dev = None
-    for p in params:
-        if isinstance(p, torch.Tensor):
-            dev = p.device
-            break
-    vals = []
-    for i in GRAD_INDEX:
-        p = params[i]
-        vals.append(p.to(torch.float64).reshape(()) if isinstance(p, torch.Tensor)
-                    else torch.tensor(float(p), dtype=torch.float64, device=dev))
-    theta = torch.stack(vals).reshape(1, 7)
+    vals = [params[i] for i in GRAD_INDEX]
+    first = next(p for p in params if isinstance(p, torch.Tensor))
+    if not all(isinstance(p, torch.Tensor) and p.dtype == first.dtype and p.is_floating_point() for p in vals):
+        # numbers, or several types: one conversion (and its backward) each
+        vals = [p.to(torch.float64) if isinstance(p, torch.Tensor)
+                else torch.tensor(float(p), dtype=torch.float64, device=first.device) for p in vals]
+    theta = torch.stack([p.reshape(()) for p in vals]).reshape(1, 7)
     ok = params[5]
     omega_k = float(ok.detach().cpu()) if isinstance(ok, torch.Tensor) else float(ok)
     dctx = default_context()

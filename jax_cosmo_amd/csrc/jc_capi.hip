@@ -549,22 +549,16 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
   std::vector<double> seeds;
   if (jac) {
     d_seeds = jac_seeds;
-  } else if (nd > 0) {
+  } else if (nd == 1) {
     // d param_i / d direction: the 7 differentiable parameters skip Omega_k
     static const int pidx[7] = {0, 1, 2, 3, 4, 6, 7};
-    std::vector<double> tan_h;
-    if (nd == 1) {
-      tan_h.resize((size_t)B * 7);
-      if (dev) HIPCHK(hipMemcpyAsync(tan_h.data(), tangent, tan_h.size() * 8, hipMemcpyDeviceToHost, s));
-      else memcpy(tan_h.data(), tangent, tan_h.size() * 8);
-      HIPCHK(hipStreamSynchronize(s));
-    }
-    seeds.assign((size_t)B * 8 * nd, 0.0);
+    std::vector<double> tan_h((size_t)B * 7);
+    if (dev) HIPCHK(hipMemcpyAsync(tan_h.data(), tangent, tan_h.size() * 8, hipMemcpyDeviceToHost, s));
+    else memcpy(tan_h.data(), tangent, tan_h.size() * 8);
+    HIPCHK(hipStreamSynchronize(s));
+    seeds.assign((size_t)B * 8, 0.0);
     for (int64_t b = 0; b < B; ++b)
-      for (int q = 0; q < 7; ++q) {
-        if (nd == 7) seeds[((size_t)b * 8 + pidx[q]) * 7 + q] = 1.0;
-        else seeds[((size_t)b * 8 + pidx[q])] = tan_h[(size_t)b * 7 + q];
-      }
+      for (int q = 0; q < 7; ++q) seeds[(size_t)b * 8 + pidx[q]] = tan_h[(size_t)b * 7 + q];
     HIPCHK(ctx->seeds.reserve(seeds.size()));
     HIPCHK(hipMemcpyAsync(ctx->seeds.p, seeds.data(), seeds.size() * 8, hipMemcpyHostToDevice, s));
     d_seeds = ctx->seeds.p;

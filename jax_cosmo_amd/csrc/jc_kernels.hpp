@@ -101,7 +101,7 @@ struct ASeg {
 
 struct TablesArgs {
   const double* params;   // [B][8] Cosmology(...) parameters
-  const double* seeds;    // [B][8][ND] d param / d direction (ND > 0)
+  const double* seeds;    // [B][8] d param / d direction (ND = 1; the 7 directions of ND = 7 are the parameters)
   int B, Na;
   const double* a_list;   // [Na] scale factors
   const double* a_wgt;    // [Na] quadrature weight of each node (0 = evaluation only)

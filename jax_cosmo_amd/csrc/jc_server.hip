@@ -91,7 +91,6 @@ struct Req {
 struct GroupBufs {
   double* params = nullptr;   // [C][8]
   double* gparams = nullptr;  // [Gd][8]
-  double* gseeds = nullptr;   // [Gd][8][7]
   RJob* jobs = nullptr;       // [C]
   RJob* gjobs = nullptr;      // [Gd]
   RCol* cols = nullptr;       // [colcap]
@@ -235,7 +234,6 @@ size_t layout_slot(jc_server* S, Slot* sl, unsigned char* base) {
     const size_t Na = S->Na[g];
     b.params = (double*)take((size_t)S->C * 8 * 8);
     b.gparams = (double*)take((size_t)S->Gd * 8 * 8);
-    b.gseeds = (double*)take((size_t)S->Gd * 8 * 7 * 8);
     b.jobs = (RJob*)take((size_t)S->C * sizeof(RJob));
     b.gjobs = (RJob*)take((size_t)S->Gd * sizeof(RJob));
     b.cols = (RCol*)take((size_t)S->colcap * sizeof(RCol));
@@ -262,7 +260,6 @@ TablesArgs tables_args(jc_server* S, int g, const GroupBufs& b, int nd, const in
   GridTables* gt = S->grid[g];
   TablesArgs ta{};
   ta.params = nd ? b.gparams : b.params;
-  ta.seeds = nd ? b.gseeds : nullptr;
   ta.B = nd ? k.Gd : k.C;  // grid bound (the live count is *dcount)
   ta.Na = S->Na[g];
   ta.a_list = gt->a_list.p;
@@ -420,13 +417,6 @@ int slot_init(jc_server* S, Slot* sl) {
   }
   sl->h_out = sl->h_outb[0];
   sl->h_theta = sl->h_thetab[0];
-  // constant seeds of the adjoint (identity over the 7 parameters, Omega_k skipped)
-  std::vector<double> seeds((size_t)S->Gd * 8 * 7, 0.0);
-  static const int pidx[7] = {0, 1, 2, 3, 4, 6, 7};
-  for (int c = 0; c < S->Gd; ++c)
-    for (int q = 0; q < 7; ++q) seeds[((size_t)c * 8 + pidx[q]) * 7 + q] = 1.0;
-  for (int g = 0; g < S->ng; ++g)
-    HIPCHK(hipMemcpy(sl->g[g].gseeds, seeds.data(), seeds.size() * 8, hipMemcpyHostToDevice));
   // zero counts and an empty staging header so a replay before any batch is a no-op
   std::vector<int> z(MAXG * 8, 0);
   HIPCHK(hipMemcpy(sl->counts, z.data(), z.size() * 4, hipMemcpyHostToDevice));

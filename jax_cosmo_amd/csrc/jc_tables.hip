@@ -47,6 +47,19 @@ struct Seed {
     return r;
   }
 };
+// The adjoint's seven directions are the seven parameters themselves (Omega_k,
+// parameter 5, has none): constants, which fold into the first operations.
+JC_D int param_dir(int i) { return i < 5 ? i : (i == 5 ? -1 : i - 1); }
+template <>
+struct Seed<7> {
+  static JC_D Types<7>::D load(const double* params, const double*, int c, int i) {
+    Types<7>::D r;
+    r.v = params[c * 8 + i];
+#pragma unroll
+    for (int d = 0; d < 7; ++d) r.d[d] = d == param_dir(i) ? 1.0 : 0.0;
+    return r;
+  }
+};
 template <>
 struct Seed<0> {
   static JC_D double load(const double* params, const double*, int c, int i) { return params[c * 8 + i]; }
@@ -297,7 +310,7 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         q[i].v = p[i].v;
-        q[i].d[0] = A.seeds[((size_t)c * 8 + i) * ND + lane];
+        q[i].d[0] = ND == 7 ? (lane == param_dir(i) ? 1.0 : 0.0) : A.seeds[((size_t)c * 8 + i) * ND + lane];
       }
       const EHc<D1> eh = eh_setup(make_cosmo(q));
       const D1 vals[15] = {eh.fb, eh.fc, eh.inv13keq, eh.ln_inv13keq, eh.beta_c18, eh.c14a, eh.sh_d,
