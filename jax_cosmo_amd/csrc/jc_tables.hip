@@ -250,12 +250,18 @@ struct TabLds {
 // tables.  The per-a nodes and the nodes of the transfer table are one list of
 // 64-node tasks that the waves draw from, so the a-grid's odd node (n_z + 1)
 // costs one wave a pass, not all of them.
-template <int ND, int NT, int MINW>
+// WO: floats of a stored scalar.  With ND = 1 and WO = 8 the seven directions
+// of a cosmology are seven workgroups, which write one derivative each into the
+// records of the adjoint (direction 0 the values too): a few cosmologies leave
+// the chip idle, and a workgroup of one direction takes half the time of one of
+// seven.
+template <int ND, int NT, int MINW, int WO = ND + 1>
 __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
   using Sd = typename Types<ND>::D;
   using Sf = typename Types<ND>::F;
   using L = TabLds<ND>;
   constexpr int W = ND + 1, NW = NT / 64;
+  constexpr bool SPLIT = WO != W;
   extern __shared__ __align__(16) unsigned char smem[];
   Sd* const lds = reinterpret_cast<Sd*>(smem);
   Sd* const s_chi = lds + L::CHI;
@@ -270,15 +276,32 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
   float* const s_k32 = reinterpret_cast<float*>(s_p1f + NHF_K);
   int* const s_next = reinterpret_cast<int*>(s_k32 + NHF_K);
 
-  const int c = blockIdx.x;
+  const int dir = SPLIT ? blockIdx.x % (WO - 1) : 0;
+  const int c = SPLIT ? blockIdx.x / (WO - 1) : blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // a scalar of the records: its value, and the derivatives
+  auto put = [&](float* o, const Sd& v) {
+    if constexpr (SPLIT) {
+      if (dir == 0) o[0] = (float)v.v;
+      o[1 + dir] = (float)v.d[0];
+    } else {
+      Mem<Sf>::st(o, conv<Sf>(v));
+    }
+  };
   if (c >= A.B) return;
   if (A.dB && c >= *A.dB) return;  // served batches: grid sized for capacity
 
   Sd p[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) p[i] = Seed<ND>::load(A.params, A.seeds, c, i);
+  for (int i = 0; i < 8; ++i) {
+    if constexpr (SPLIT) {
+      p[i].v = A.params[c * 8 + i];
+      p[i].d[0] = dir == param_dir(i) ? 1.0 : 0.0;
+    } else {
+      p[i] = Seed<ND>::load(A.params, A.seeds, c, i);
+    }
+  }
   const CosmoP<Sd> cp = make_cosmo(p);
   for (int i = tid; i < NHF_K; i += NT) s_k32[i] = A.hf_k32[i];
   if (tid == 0) *s_next = 0;
@@ -310,7 +333,7 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         q[i].v = p[i].v;
-        q[i].d[0] = ND == 7 ? (lane == param_dir(i) ? 1.0 : 0.0) : A.seeds[((size_t)c * 8 + i) * ND + lane];
+        q[i].d[0] = ND == 7 ? (lane == param_dir(i) ? 1.0 : 0.0) : p[i].d[0];
       }
       const EHc<D1> eh = eh_setup(make_cosmo(q));
       const D1 vals[15] = {eh.fb, eh.fc, eh.inv13keq, eh.ln_inv13keq, eh.beta_c18, eh.c14a, eh.sh_d,
@@ -467,9 +490,9 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
     constexpr int slot[18] = {CR_FB, CR_FC, CR_INV13KEQ, CR_BETAC18, CR_C14A, CR_SHD, CR_ALPHAB, CR_BETAB,
                               CR_BETANODE, CR_LNKSILK, CR_NS, CR_WLCONST, CR_LNINV13, CR_BNODE_SHD, CR_BB_SHD,
                               CR_ALPHAG, CR_TQ, CR_NW};
-    float* cr = A.crec + (size_t)c * NCREC * W;
+    float* cr = A.crec + (size_t)c * NCREC * WO;
 #pragma unroll
-    for (int i = 0; i < 18; ++i) Mem<Sf>::st(cr + slot[i] * W, conv<Sf>(vals[i]));
+    for (int i = 0; i < 18; ++i) put(cr + slot[i] * WO, vals[i]);
   }
   // T^2 k^n_s times the resident weights: of the sigma_8 Romberg table
   // (power.py:56-78, integrate.py:67-159: its extrapolation is a fixed linear
@@ -506,11 +529,11 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
     const Sd chi_i = s_chi[tid];
     Sd slope = zero<Sd>();
     if (tid < NCHI - 1) slope = (s_chi[tid + 1] - chi_i) / (A.atab_chi[tid + 1] - A.atab_chi[tid]);
-    float* ct = A.chitab + ((size_t)c * NCHI + tid) * 2 * W;
-    Mem<Sf>::st(ct, conv<Sf>(chi_i));
-    Mem<Sf>::st(ct + W, conv<Sf>(slope));
+    float* ct = A.chitab + ((size_t)c * NCHI + tid) * 2 * WO;
+    put(ct, chi_i);
+    put(ct + WO, slope);
   }
-  if (tid == 0) Mem<Sf>::st(A.crec + ((size_t)c * NCREC + CR_PKNORM) * W, conv<Sf>(pknorm));
+  if (tid == 0) put(A.crec + ((size_t)c * NCREC + CR_PKNORM) * WO, pknorm);
 
   // ------------------------------------------- Gaussian moments
   // of the a = 1 power (without D^2) on the 256 R nodes:
@@ -698,7 +721,7 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
     g = s_g[sg.gi] + (s_g[sg.gj] - s_g[sg.gi]) * sg.tg;
     g = minc(maxc(g, 0.0), 1.0);                                            // background.py:488
   };
-  const bool tab = (ND == 0 || ND == 7) && A.ehtab;
+  const bool tab = (ND == 0 || WO == 8) && A.ehtab;
   float lo = 0.0f, invh = 0.0f;
   double h = 0.0;
   if (tab) {
@@ -735,16 +758,19 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
     invh = (float)(NEHQ / span);
     if ((double)invh * span > (double)NEHQ) invh = nextafterf(invh, 0.0f);
     h = 1.0 / (double)invh;
-    if (tid == 0) {
-      A.crec[((size_t)c * NCREC + CR_EHLO) * W] = lo;
-      A.crec[((size_t)c * NCREC + CR_EHINVH) * W] = invh;
+    if (tid == 0 && dir == 0) {
+      A.crec[((size_t)c * NCREC + CR_EHLO) * WO] = lo;
+      A.crec[((size_t)c * NCREC + CR_EHINVH) * WO] = invh;
     }
   }
   // T(k) k^(n_s/2) (transfer.py:119-149, power.py:14-18) and its ln k
   // derivative at the table's nodes, in float with forward-mode duals; each
   // value is moved from the float-rounded node to the exact one with its
   // derivative
-  float2* s_nd = reinterpret_cast<float2*>(ND == 0 ? s_x : s_smp);  // [NEHQ + 1]
+  // (one direction a workgroup: the samples are too few, the moments' k rows are free)
+  float2* s_nd = SPLIT ? reinterpret_cast<float2*>(reinterpret_cast<double*>(smem) + L::KP)
+                       : reinterpret_cast<float2*>(ND == 0 ? s_x : s_smp);  // [NEHQ + 1]
+  static_assert(!SPLIT || 4 * NHF_K >= NEHQ + 1, "the nodes fit the k rows");
   const float hns = 0.5f * (float)val(cp.n_s);
   auto table_node = [&](int q) {
     using D1 = Dual<float, 1>;
@@ -854,7 +880,7 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
     // max(chi^2, 1) = max(chi, 1)^2 (angular_cl.py:91,96)
     const Sd wgt = (A.a_wgt[m] / c2) * dchida * (invchi * invchi);
 
-    float* cf = A.coef + ((size_t)c * A.Na + m) * NCOEF * W;
+    float* cf = A.coef + ((size_t)c * A.Na + m) * NCOEF * WO;
     if (ND == 0 && A.ehtab) {  // forward record (FwdSlot)
       if constexpr (ND == 0) {
         const double iRnl = 1.0 / Rnl, yc = Rnl * invchi, iyc = chi1 * iRnl, c3 = chi1 * chi1 * chi1;
@@ -870,27 +896,27 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
         cf[FT_CHI] = (float)chi;
       }
     } else {
-      Mem<Sf>::st(cf + CF_INV_CHI * W, conv<Sf>(invchi));
-      Mem<Sf>::st(cf + CF_CHI1 * W, conv<Sf>(chi1));
+      put(cf + CF_INV_CHI * WO, invchi);
+      put(cf + CF_CHI1 * WO, chi1);
       // the logarithms stored as floats are taken to float accuracy
-      Mem<Sf>::st(cf + CF_LNINVCHI * W, conv<Sf>(-jm::logf_acc(chi1)));
-      Mem<Sf>::st(cf + CF_KNL * W, conv<Sf>(1.0 / Rnl));
-      Mem<Sf>::st(cf + CF_MU * W, conv<Sf>(hf.mu_n));
-      Mem<Sf>::st(cf + CF_WGT * W, conv<Sf>(wgt));
-      Mem<Sf>::st(cf + CF_G2P * W, conv<Sf>(g2 * pknorm));
-      Mem<Sf>::st(cf + CF_LGRNL * W, conv<Sf>(maxc(root, LN_RMIN) * 1.4426950408889634));
-      Mem<Sf>::st(cf + CF_RNL * W, conv<Sf>(Rnl));
-      Mem<Sf>::st(cf + CF_AN * W, conv<Sf>(hf.a_n));
-      Mem<Sf>::st(cf + CF_BN * W, conv<Sf>(hf.b_n));
-      Mem<Sf>::st(cf + CF_LGCF3 * W, conv<Sf>(hf.lg_cf3));
-      Mem<Sf>::st(cf + CF_GAM3 * W, conv<Sf>(hf.gam3));
-      Mem<Sf>::st(cf + CF_ALPHA * W, conv<Sf>(hf.alpha_n));
-      Mem<Sf>::st(cf + CF_BETA * W, conv<Sf>(hf.beta_n));
-      Mem<Sf>::st(cf + CF_NU * W, conv<Sf>(hf.nu_n));
-      Mem<Sf>::st(cf + CF_F1X3 * W, conv<Sf>(hf.f1x3));
-      Mem<Sf>::st(cf + CF_F2 * W, conv<Sf>(hf.f2));
-      Mem<Sf>::st(cf + CF_CHI * W, conv<Sf>(chi));
-      Mem<Sf>::st(cf + CF_GROWTH * W, conv<Sf>(g));
+      put(cf + CF_LNINVCHI * WO, -jm::logf_acc(chi1));
+      put(cf + CF_KNL * WO, 1.0 / Rnl);
+      put(cf + CF_MU * WO, hf.mu_n);
+      put(cf + CF_WGT * WO, wgt);
+      put(cf + CF_G2P * WO, g2 * pknorm);
+      put(cf + CF_LGRNL * WO, maxc(root, LN_RMIN) * 1.4426950408889634);
+      put(cf + CF_RNL * WO, Rnl);
+      put(cf + CF_AN * WO, hf.a_n);
+      put(cf + CF_BN * WO, hf.b_n);
+      put(cf + CF_LGCF3 * WO, hf.lg_cf3);
+      put(cf + CF_GAM3 * WO, hf.gam3);
+      put(cf + CF_ALPHA * WO, hf.alpha_n);
+      put(cf + CF_BETA * WO, hf.beta_n);
+      put(cf + CF_NU * WO, hf.nu_n);
+      put(cf + CF_F1X3 * WO, hf.f1x3);
+      put(cf + CF_F2 * WO, hf.f2);
+      put(cf + CF_CHI * WO, chi);
+      put(cf + CF_GROWTH * WO, g);
     }
 
     // z-local kernels, H = H0 sqrt(E^2) (background.py:129-148): number
@@ -912,7 +938,7 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
         for (int i = 0; i < MAXT; ++i) cmask |= (i < T && jb.sel[i] == lc ? 1u : 0u) << i;
       }
       const size_t rb = ((size_t)c * A.Na + m) * A.Tpad;
-      for (uint32_t mk = cmask; mk; mk &= mk - 1) Mem<Sf>::st(A.R + (rb + __builtin_ctz(mk)) * W, conv<Sf>(r));
+      for (uint32_t mk = cmask; mk; mk &= mk - 1) put(A.R + (rb + __builtin_ctz(mk)) * WO, r);
     }
     if (A.dbg) {
       double* d = A.dbg + (size_t)c * A.dbg_stride + 1024 + (size_t)m * 8;
@@ -931,8 +957,16 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
     } else {
       const int q = 64 * (t - na_tasks) + lane;
       if (q <= NEHQ) {
-        table_node(q);
+        if (dir == 0) table_node(q);
         if constexpr (ND == 7) eh_dtab_node<W>(c, q, (double)lo, h, A.crec, A.ehtab7);
+        if constexpr (SPLIT) {
+          const EHc<Sf> e1 = eh_from<Sf>([&](int i) { return conv<Sf>(s_eh[i]); }, A.transfer_model);
+          const float x = (float)((double)lo + (double)q * h), k = jm::exp(x), ik = jm::exp(-x);
+          const Sf tn = eh_transfer(e1, k, ik, x) * jm::exp(conv<Sf>(cp.n_s) * (0.5f * x));
+          float* o = A.ehtab7 + ((size_t)c * (NEHQ + 1) + q) * NEHD_ROW;
+          o[dir] = tn.d[0];
+          if (dir == 0) o[7] = 0.0f;
+        }
       }
     }
   }
@@ -943,7 +977,7 @@ __global__ __launch_bounds__(NT, MINW) void k_tables(TablesArgs A) {
     d[384 + tid] = val(s_sig[tid]);
     if (tid == 0) d[640] = val(pknorm);
   }
-  if (!tab) return;
+  if (!tab || dir != 0) return;  // uniform over the workgroup
   __syncthreads();
   // cubic Hermite pieces of T(k) k^(n_s/2) between the nodes
   const float hf = (float)h;
@@ -996,6 +1030,12 @@ hipError_t launch_background_ex(const double* params, const double* a, int n, co
 // while there is at most one for each, two share it (2) up to two each, and
 // four (1) beyond.  Measured on 256 CUs, n_z 512, for 3 / 2 / 1 in us: 31 / 36 / 40
 // at 1 cosmology, 45 / 52 / 54 at 256, 79 / 58 / 63 at 512, 136 / 105 / 92 at 1024.
+// Dual tables: while there is at most one workgroup per CU, one of 512 threads
+// per cosmology and direction (the adjoint's seven directions apart); beyond, 256
+// threads, and the adjoint's directions together.  Measured, n_z 512: directions
+// apart 85 -> 49 us at 1 cosmology, 106 -> 82 at 36, but 105 -> 119 at 73; 512
+// threads against 256 for one direction 43 / 51 us at 7 rows, 54 / 64 at 210, 96 / 78
+// at 420.
 hipError_t launch_tables(int nd, const TablesArgs& a, hipStream_t s, int num_cu, int variant) {
   const size_t sm = nd == 0 ? TabLds<0>::bytes() : (nd == 1 ? TabLds<1>::bytes() : TabLds<7>::bytes());
   if (nd == 0) {
@@ -1006,7 +1046,10 @@ hipError_t launch_tables(int nd, const TablesArgs& a, hipStream_t s, int num_cu,
       default: hipLaunchKernelGGL((k_tables<0, 256, 2>), dim3(a.B), dim3(256), sm, s, a); break;
     }
   } else if (nd == 1) {
-    hipLaunchKernelGGL((k_tables<1, 256, 2>), dim3(a.B), dim3(256), sm, s, a);
+    if (a.B <= num_cu) hipLaunchKernelGGL((k_tables<1, 512, 2>), dim3(a.B), dim3(512), sm, s, a);
+    else hipLaunchKernelGGL((k_tables<1, 256, 2>), dim3(a.B), dim3(256), sm, s, a);
+  } else if (nd == 7 && 7 * (int64_t)a.B <= num_cu && !a.dB) {  // (a.dB: the live count is on the device)
+    hipLaunchKernelGGL((k_tables<1, 512, 2, 8>), dim3(7 * a.B), dim3(512), TabLds<1>::bytes(), s, a);
   } else if (nd == 7) {
     hipLaunchKernelGGL((k_tables<7, 256, 1>), dim3(a.B), dim3(256), sm, s, a);
   } else {
