@@ -541,10 +541,21 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
 
   const double* d_cosmo = nullptr;
   const double* d_ell = nullptr;
-  rc = to_device(ctx, ctx->params, cosmo, (size_t)B * 8, dev, &d_cosmo, sc);
-  if (rc) return rc;
-  rc = to_device(ctx, ctx->ell, ell, (size_t)n_ell, dev, &d_ell, sc);
-  if (rc) return rc;
+  const size_t n_in = (size_t)B * 8 + (size_t)n_ell;
+  if (!dev && !sc && n_in * sizeof(double) <= PIN_IN) {
+    double* h = reinterpret_cast<double*>(ctx->pin_in);
+    memcpy(h, cosmo, (size_t)B * 64);
+    memcpy(h + B * 8, ell, (size_t)n_ell * 8);
+    HIPCHK(ctx->params.reserve(n_in));
+    HIPCHK(launch_stage(h, ctx->params.p, n_in * sizeof(double), s));
+    d_cosmo = ctx->params.p;
+    d_ell = ctx->params.p + B * 8;
+  } else {
+    rc = to_device(ctx, ctx->params, cosmo, (size_t)B * 8, dev, &d_cosmo, sc);
+    if (rc) return rc;
+    rc = to_device(ctx, ctx->ell, ell, (size_t)n_ell, dev, &d_ell, sc);
+    if (rc) return rc;
+  }
   const double* d_seeds = nullptr;
   std::vector<double> seeds;
   if (jac) {
@@ -621,7 +632,12 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
   if (l_slices > 1 && !adj_tab && (rc = workspace(ctx->part, (size_t)l_slices * nslice, sc, &w_part))) return rc;
   float* d_out = cl;
   float* d_out_t = cl_dot;
-  if (!dev && nd != 7) {
+  const size_t res_bytes = nd == 7 ? (size_t)B * 7 * sizeof(double) : nout * sizeof(float);
+  const bool pinned = !dev && !sc && res_bytes * (nd == 1 ? 2 : 1) <= PIN_OUT;
+  if (pinned) {
+    d_out = reinterpret_cast<float*>(ctx->pin_out);
+    d_out_t = d_out + nout;
+  } else if (!dev && nd != 7) {
     if ((rc = workspace(ctx->out, nout, sc, &d_out))) return rc;
     if (nd == 1) {
       HIPCHK(ctx->out_t.reserve(nout));
@@ -678,7 +694,9 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
     HIPCHK(timed(ctx, JC_KERNEL_LIMBER,
                  [&] { return adj_tab ? launch_adjoint(T, la, s) : launch_limber(nd, T, la, s); }));
     double* d_th = theta_bar;
-    if (!dev) {
+    if (pinned) {
+      d_th = reinterpret_cast<double*>(ctx->pin_out);
+    } else if (!dev) {
       HIPCHK(ctx->theta.reserve((size_t)B * 7));
       d_th = ctx->theta.p;
     }
@@ -687,8 +705,9 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
                    : launch_theta_reduce(la.slices > 1 ? la.part : ctx->theta_col.p, la.slices, (int)B, (int)n_ell,
                                          d_th, s));
     if (!dev) {
-      HIPCHK(hipMemcpyAsync(theta_bar, d_th, (size_t)B * 7 * sizeof(double), hipMemcpyDeviceToHost, s));
+      if (!pinned) HIPCHK(hipMemcpyAsync(theta_bar, d_th, res_bytes, hipMemcpyDeviceToHost, s));
       HIPCHK(hipStreamSynchronize(s));
+      if (pinned) memcpy(theta_bar, d_th, res_bytes);
     }
     return JC_OK;
   }
@@ -705,9 +724,15 @@ int run_pipeline(jc_ctx* ctx, int nd, const double* cosmo, const double* tangent
     if (nd == 1) HIPCHK(launch_slice_sum(la.part + (size_t)la.slices * nout, la.slices, (int64_t)nout, d_out_t, s));
   }
   if (!dev) {
-    HIPCHK(hipMemcpyAsync(cl, d_out, nout * sizeof(float), hipMemcpyDeviceToHost, s));
-    if (nd == 1) HIPCHK(hipMemcpyAsync(cl_dot, d_out_t, nout * sizeof(float), hipMemcpyDeviceToHost, s));
+    if (!pinned) {
+      HIPCHK(hipMemcpyAsync(cl, d_out, res_bytes, hipMemcpyDeviceToHost, s));
+      if (nd == 1) HIPCHK(hipMemcpyAsync(cl_dot, d_out_t, res_bytes, hipMemcpyDeviceToHost, s));
+    }
     HIPCHK(hipStreamSynchronize(s));
+    if (pinned) {
+      memcpy(cl, d_out, res_bytes);
+      if (nd == 1) memcpy(cl_dot, d_out_t, res_bytes);
+    }
   }
   return JC_OK;
 }
@@ -789,8 +814,13 @@ int jc_ctx_create(int device, jc_ctx** out) {
   HIPCHK(hipStreamCreateWithFlags(&ctx->own, hipStreamNonBlocking));
   ctx->stream = ctx->own;
   int rc = scratch_address(device, &ctx->scratch);
+  if (rc == JC_OK && (hipHostMalloc((void**)&ctx->pin_in, PIN_IN, hipHostMallocMapped) != hipSuccess ||
+                      hipHostMalloc((void**)&ctx->pin_out, PIN_OUT, hipHostMallocMapped) != hipSuccess))
+    rc = fail(JC_E_NOMEM, "no pinned host memory");
   if (rc == JC_OK) rc = ctx_init_tables(ctx.get());
   if (rc) {
+    if (ctx->pin_in) (void)hipHostFree(ctx->pin_in);
+    if (ctx->pin_out) (void)hipHostFree(ctx->pin_out);
     (void)hipStreamDestroy(ctx->own);
     return rc;
   }
@@ -808,6 +838,8 @@ int jc_ctx_destroy(jc_ctx* ctx) {
     (void)hipEventDestroy(r.b);
   }
   for (auto e : ctx->ev_pool) (void)hipEventDestroy(e);
+  (void)hipHostFree(ctx->pin_in);
+  (void)hipHostFree(ctx->pin_out);
   delete ctx;
   if (own) (void)hipStreamDestroy(own);
   return JC_OK;
@@ -976,15 +1008,19 @@ int jc_angular_cl_jacobian(jc_ctx* ctx, const double* cosmo, int64_t B, int64_t 
   const int64_t nb = std::min(B, std::max<int64_t>(1, fit));
   static const int pidx[7] = {0, 1, 2, 3, 4, 6, 7};
   // ell, and per chunk the parameter and seed rows, in one upload
-  std::vector<double> up((size_t)n_ell + (size_t)nb * 7 * 16);
-  memcpy(up.data(), ell, (size_t)n_ell * sizeof(double));
-  HIPCHK(ctx->params.reserve(up.size()));
+  const size_t n_up = (size_t)n_ell + (size_t)nb * 7 * 16;
+  const bool pin_in = n_up * sizeof(double) <= PIN_IN, pin_out = (size_t)nb * 7 * np * sizeof(float) <= PIN_OUT;
+  std::vector<double> pageable(pin_in ? 0 : n_up);
+  double* up = pin_in ? reinterpret_cast<double*>(ctx->pin_in) : pageable.data();
+  memcpy(up, ell, (size_t)n_ell * sizeof(double));
+  HIPCHK(ctx->params.reserve(n_up));
   HIPCHK(ctx->out.reserve((size_t)nb * 7 * np));
   HIPCHK(ctx->out_t.reserve((size_t)nb * 7 * np));
-  HIPCHK(ctx->jac.reserve((size_t)nb * 7 * np));
+  if (!pin_out) HIPCHK(ctx->jac.reserve((size_t)nb * 7 * np));
+  float* d_jac = pin_out ? reinterpret_cast<float*>(ctx->pin_out) : ctx->jac.p;
   for (int64_t b0 = 0; b0 < B; b0 += nb) {
     const int64_t n = std::min(nb, B - b0);
-    double* pr = up.data() + n_ell;
+    double* pr = up + n_ell;
     double* sd = pr + n * 7 * 8;
     std::fill(sd, sd + n * 7 * 8, 0.0);
     for (int64_t r = 0; r < n * 7; ++r) {
@@ -992,14 +1028,16 @@ int jc_angular_cl_jacobian(jc_ctx* ctx, const double* cosmo, int64_t B, int64_t 
       sd[r * 8 + pidx[r % 7]] = 1.0;
     }
     const double* dp = ctx->params.p;
-    HIPCHK(hipMemcpyAsync(ctx->params.p, up.data(), ((size_t)n_ell + (size_t)n * 7 * 16) * sizeof(double),
-                          hipMemcpyHostToDevice, s));
+    const size_t bytes = ((size_t)n_ell + (size_t)n * 7 * 16) * sizeof(double);
+    if (pin_in) HIPCHK(launch_stage(up, ctx->params.p, bytes, s));
+    else HIPCHK(hipMemcpyAsync(ctx->params.p, up, bytes, hipMemcpyHostToDevice, s));
     rc = run_pipeline(ctx, 1, dp + n_ell, nullptr, n * 7, set_id, dp, n_ell, n_z, ctx->out.p, ctx->out_t.p, nullptr,
-                      nullptr, JC_DEVICE_PTRS, nullptr, dp + n_ell + n * 7 * 8, ctx->jac.p);
+                      nullptr, JC_DEVICE_PTRS, nullptr, dp + n_ell + n * 7 * 8, d_jac);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(jac + (size_t)b0 * 7 * np, ctx->jac.p, (size_t)n * 7 * np * sizeof(float),
-                          hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));  // up and the device buffers are reused by the next chunk
+    const size_t res = (size_t)n * 7 * np * sizeof(float);
+    if (!pin_out) HIPCHK(hipMemcpyAsync(jac + (size_t)b0 * 7 * np, d_jac, res, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));  // the buffers are reused by the next chunk
+    if (pin_out) memcpy(jac + (size_t)b0 * 7 * np, d_jac, res);
   }
   return JC_OK;
 }
@@ -1055,19 +1093,23 @@ int jc_gaussian_loglike_cov(jc_ctx* ctx, const float* mu, int64_t B, int64_t P, 
   int rc = to_device(ctx, ctx->lk_prec, cov, (size_t)P * P * n_ell, false, &d_cov);
   if (rc) return rc;
   HIPCHK(ctx->lk_inv.reserve((size_t)P * P * n_ell));
-  std::vector<double> res((size_t)B + 2 * n_ell);  // the results, then ld
-  HIPCHK(ctx->lk_out.reserve(res.size()));
+  const size_t n_res = (size_t)B + 2 * n_ell;  // the results, then ld
+  const bool pinned = n_res * sizeof(double) <= PIN_OUT;
+  std::vector<double> pageable(pinned ? 0 : n_res);
+  const double* res = pinned ? reinterpret_cast<double*>(ctx->pin_out) : pageable.data();
+  if (!pinned) HIPCHK(ctx->lk_out.reserve(n_res));
+  double* d_res = pinned ? reinterpret_cast<double*>(ctx->pin_out) : ctx->lk_out.p;
   const PrecLayout lay = prec_blocks(P);
-  HIPCHK(launch_block_inv(d_cov, (int)P, (int)n_ell, ctx->lk_inv.p, lay, ctx->lk_out.p + B, s));
+  HIPCHK(launch_block_inv(d_cov, (int)P, (int)n_ell, ctx->lk_inv.p, lay, d_res + B, s));
   if ((rc = to_device(ctx, ctx->lk_data, data, (size_t)P * n_ell, false, &d_data))) return rc;
   if ((rc = to_device(ctx, ctx->lk_mu, mu, (size_t)B * P * n_ell, false, &d_mu))) return rc;
   HIPCHK(ctx->lk_part.reserve((size_t)B * n_ell));
   HIPCHK(launch_loglike(d_mu, (int)B, (int)P, (int)n_ell, d_data, ctx->lk_inv.p, lay, 0.0, nullptr, ctx->lk_part.p,
-                        ctx->lk_out.p, s));
-  HIPCHK(hipMemcpyAsync(res.data(), ctx->lk_out.p, res.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+                        d_res, s));
+  if (!pinned) HIPCHK(hipMemcpyAsync(pageable.data(), d_res, n_res * sizeof(double), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   double logdet = 0.0;
-  if ((rc = block_logdet(res.data() + B, n_ell, &logdet))) return rc;
+  if ((rc = block_logdet(res + B, n_ell, &logdet))) return rc;
   const double c0 = include_logdet ? 0.5 * logdet : 0.0;  // likelihood.py:61
   for (int64_t b = 0; b < B; ++b) loglike[b] = res[b] + c0;
   return JC_OK;

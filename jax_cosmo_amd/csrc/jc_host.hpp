@@ -181,10 +181,20 @@ int eval_pz(jc_ctx* ctx, TracerSet* ts, int i, const std::vector<double>& z, std
 
 }  // namespace jch
 
+// Bytes of a context's pinned host buffers (allocated with it).  Host-pointer
+// calls whose parameters and multipoles, or whose results, fit them pass through
+// them: one copy kernel brings the inputs in, and the last kernel writes its
+// results straight to host memory, instead of a copy command per array (5-10 us
+// each for small pageable arrays in, 25 us and more out; a call of one cosmology,
+// 10 tracers, 100 ell, n_z 512: 103 -> 92 us).  The call's final
+// synchronisation hands the buffers back.
+constexpr size_t PIN_IN = 128u << 10, PIN_OUT = 512u << 10;
+
 struct jc_ctx {
   using TracerSet = jch::TracerSet;
   template <class T> using DevBuf = jch::DevBuf<T>;
   int device = 0;
+  unsigned char *pin_in = nullptr, *pin_out = nullptr;  // PIN_IN and PIN_OUT bytes, read and written by the device in place
   unsigned char* scratch = nullptr;  // this device's scratch array (jc_angular_cl_noalloc)
   hipStream_t own = nullptr;
   hipStream_t stream = nullptr;

@@ -323,6 +323,8 @@ hipError_t launch_background_ex(const double* params, const double* a, int n, co
                                 int growth_model, double gamma, double* dbg, hipStream_t s);
 // out[o] = sum over s of part[s * n + o], s = 0..slices-1 in order
 hipError_t launch_slice_sum(const float* part, int slices, int64_t n, float* out, hipStream_t s);
+// dst = src, whole 8-byte words (src may be pinned host memory)
+hipError_t launch_stage(const void* src, void* dst, size_t bytes, hipStream_t s);
 // jac[b][o][d] = sum over s of part[s][b * 7 + d][o], for B cosmologies and n outputs
 hipError_t launch_jac_sum(const float* part, int slices, int64_t B, int64_t n, float* jac, hipStream_t s);
 hipError_t launch_kde(const double* z, int64_t n, const double* cz, const double* cw, int64_t ncat, double bw,

@@ -339,28 +339,34 @@ hipError_t launch_slice_sum(const float* part, int slices, int64_t n, float* out
 }
 
 // Jacobian: jac[b][o][d] = part[b * 7 + d][o] added over the slices of
-// part[slices][B * 7][n], in order.  A thread takes one o of one cosmology: the
-// seven rows are read coalesced, its seven results lie together.
+// part[slices][B * 7][n], in order.  A thread takes one entry, so that jac, which
+// may lie in host memory, is written in whole lines.
 __global__ void k_jac_sum(const float* __restrict__ part, int slices, int64_t B, int64_t n, float* __restrict__ jac) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= B * n) return;
-  const int64_t b = e / n, o = e - b * n;
-  const float* p = part + b * 7 * n + o;
-  float s[7];
-#pragma unroll
-  for (int d = 0; d < 7; ++d) s[d] = p[d * n];
-  for (int k = 1; k < slices; ++k) {
-    p += B * 7 * n;
-#pragma unroll
-    for (int d = 0; d < 7; ++d) s[d] += p[d * n];
-  }
-#pragma unroll
-  for (int d = 0; d < 7; ++d) jac[e * 7 + d] = s[d];
+  if (e >= B * n * 7) return;
+  const int64_t q = e / 7, b = q / n, o = q - b * n;
+  const float* p = part + (b * 7 + (e - q * 7)) * n + o;
+  float s = p[0];
+  for (int k = 1; k < slices; ++k) s += p[k * B * 7 * n];
+  jac[e] = s;
 }
 
 hipError_t launch_jac_sum(const float* part, int slices, int64_t B, int64_t n, float* jac, hipStream_t s) {
   if (B <= 0 || n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_jac_sum, dim3((unsigned)((B * n + 255) / 256)), dim3(256), 0, s, part, slices, B, n, jac);
+  hipLaunchKernelGGL(k_jac_sum, dim3((unsigned)((B * n * 7 + 255) / 256)), dim3(256), 0, s, part, slices, B, n, jac);
+  return hipGetLastError();
+}
+
+__global__ void k_stage(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst, size_t n) {
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < n) dst[e] = src[e];
+}
+
+hipError_t launch_stage(const void* src, void* dst, size_t bytes, hipStream_t s) {
+  const size_t n = bytes / 8;
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_stage, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const uint64_t*)src, (uint64_t*)dst,
+                     n);
   return hipGetLastError();
 }
 
