@@ -13,6 +13,7 @@ import numpy as np
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libjc_limber.so")
 
 JC_DEVICE_PTRS = 1
+JC_DEVICE_FACTOR = 2
 
 ERRORS = {-1: ValueError, -2: MemoryError, -3: NotImplementedError, -4: RuntimeError}
 
@@ -608,22 +609,20 @@ class _Likelihood:
         import torch
 
         N = L.shape[0]
-        dev = L.device
-        mu_t = torch.as_tensor(np.asarray(mu, dtype=np.float32).reshape(-1, N)).to(dev)
-        B = mu_t.shape[0]
-        data_t = torch.as_tensor(_f64(data).reshape(N)).to(dev)
-        ll = torch.empty(B, dtype=torch.float64, device=dev)
-        dmu = torch.empty((B, N), dtype=torch.float32, device=dev) if want_dmu else None
+        mu = np.ascontiguousarray(np.asarray(mu, dtype=np.float32).reshape(-1, N))
+        B = mu.shape[0]
+        data = _f64(data).reshape(N)
+        ll = np.empty(B)
+        dmu = np.empty((B, N), dtype=np.float32) if want_dmu else None
         with self._lock:
-            self.set_stream(torch.cuda.current_stream().cuda_stream)
+            self.set_stream(torch.cuda.current_stream().cuda_stream)  # after the factor's
             try:
-                check(self.lib.jc_gaussian_loglike_dense(self.handle, _P(mu_t.data_ptr()), B, N, _P(data_t.data_ptr()),
-                                                         _P(L.data_ptr()), float(c0), _P(ll.data_ptr()),
-                                                         _P(dmu.data_ptr()) if want_dmu else None, JC_DEVICE_PTRS))
+                check(self.lib.jc_gaussian_loglike_dense(self.handle, _ptr(mu), B, N, _ptr(data), _P(L.data_ptr()),
+                                                         float(c0), _ptr(ll), _ptr(dmu) if want_dmu else None,
+                                                         JC_DEVICE_FACTOR))
             finally:
                 self.reset_stream()
-        ll = ll.cpu().numpy()
-        return (ll, dmu.cpu().numpy()) if want_dmu else ll
+        return (ll, dmu) if want_dmu else ll
 
     def gaussian_loglike_grad_dense(self, cosmo, set_id, ell, n_z, data, L, c0=0.0):
         """(log-likelihood [B], its gradient [B][7]) of the means

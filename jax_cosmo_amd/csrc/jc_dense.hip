@@ -13,7 +13,7 @@
 //                 its first block then factors and inverts the next panel's
 //                 diagonal block (chol64) beside the other tiles.
 // Triangular solves for B right-hand sides stored as rows ([B][N]), in
-// 256-row blocks whose triangles are inverted first, all at once
+// 512-row blocks whose triangles are inverted first, all at once
 // (k_tri_inv64, k_tri_merge): per block one product with its inverse
 // (k_solve_diag) and one that removes it from the remaining rows
 // (k_solve_update).
@@ -359,140 +359,156 @@ __global__ __launch_bounds__(256, 2) void k_tri_inv64(const double* __restrict__
 }
 
 // k_tri_merge: two inverted neighbours of H rows to one of 2 H:
-// inv21 = -inv22 (L21 inv11), 32 columns per block (grid y), 16 rows a wave.
-constexpr int MS = 34;  // LDS row stride of the [H][32] product
-
-template <int H>
-__global__ __launch_bounds__(4 * H, 2) void k_tri_merge(const double* __restrict__ L, int64_t N, double* __restrict__ inv) {
+// inv21 = -inv22 (L21 inv11), 16 NC columns per block (grid y), 16 rows a wave.
+template <int H, int NC>
+__global__ __launch_bounds__(4 * H, H < 256 ? 2 : 4) void k_tri_merge(const double* __restrict__ L, int64_t N,
+                                                                      double* __restrict__ inv) {
+  constexpr int MS = 16 * NC + 2;  // LDS row stride of the product
   __shared__ double tm[H * MS];
   constexpr int per = SB / (2 * H);
   const int64_t k0 = (int64_t)blockIdx.x * 2 * H;
   double* V = inv + (size_t)(blockIdx.x / per) * SB * SB + (size_t)(blockIdx.x % per) * 2 * H * (SB + 1);
-  const int j0 = blockIdx.y * 32;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, g = lane >> 4;
-  const int w0 = wave * 16;
+  const int j0 = blockIdx.y * 16 * NC;
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int w0 = 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t lrow = k0 + H + w0 + i;  // rows past N: zero (their columns lie below N)
-  d4 c0 = {0.0, 0.0, 0.0, 0.0}, c1 = c0;
-  for (int k = j0; k < H; k += 16) {  // inv11 has no rows above its column
-    const double* v = V + (size_t)(k + 4 * g) * SB + j0 + i;
-    const d4 x = lrow < N ? frag_row(L + (size_t)lrow * N + k0 + k + 4 * g, 4) : d4{0.0, 0.0, 0.0, 0.0};
-    mma16(x, frag_col(v, SB, 4), c0);
-    mma16(x, frag_col(v + 16, SB, 4), c1);
-  }
+  d4 acc[NC];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    tm[(w0 + g + 4 * r) * MS + i] = c0[r];
-    tm[(w0 + g + 4 * r) * MS + 16 + i] = c1[r];
-  }
+  for (int c = 0; c < NC; ++c) acc[c] = d4{0.0, 0.0, 0.0, 0.0};
+  constexpr int D = 4;
+  d4 x[D], v[D][NC];
+  pipelined<D>((H - j0) / 16, [&](int s, int q) {  // inv11 has no rows above its column
+    const int k = j0 + 16 * s + 4 * g;
+    x[q] = lrow < N ? frag_row(L + (size_t)lrow * N + k0 + k, 4) : d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[q][c] = frag_col(V + (size_t)k * SB + j0 + 16 * c + i, SB, 4);
+  }, [&](int q) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) mma16(x[q], v[q][c], acc[c]);
+  });
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) tm[(w0 + g + 4 * r) * MS + 16 * c + i] = acc[c][r];
   __syncthreads();
-  c0 = c1 = d4{0.0, 0.0, 0.0, 0.0};
-  for (int k = 0; k <= w0; k += 16) {
-    const d4 x = frag_row(V + (size_t)(H + w0 + i) * SB + H + k + 4 * g, 4);
-    const double* t = tm + (k + 4 * g) * MS + i;
-    mma16(x, frag_col(t, MS, 4), c0);
-    mma16(x, frag_col(t + 16, MS, 4), c1);
-  }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    double* o = V + (size_t)(H + w0 + g + 4 * r) * SB + j0 + i;
-    o[0] = -c0[r];
-    o[16] = -c1[r];
-  }
+  for (int c = 0; c < NC; ++c) acc[c] = d4{0.0, 0.0, 0.0, 0.0};
+  pipelined<D>(w0 / 16 + 1, [&](int s, int q) {
+    x[q] = frag_row(V + (size_t)(H + w0 + i) * SB + H + 16 * s + 4 * g, 4);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[q][c] = frag_col(tm + (16 * s + 4 * g) * MS + 16 * c + i, MS, 4);
+  }, [&](int q) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) mma16(x[q], v[q][c], acc[c]);
+  });
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) V[(size_t)(H + w0 + g + 4 * r) * SB + j0 + 16 * c + i] = -acc[c][r];
 }
 
+// The solves' steps are a chain, so each has to be short: a workgroup takes a
+// small tile of the result, its 4 waves every 4th step of 16 k of the same tile,
+// and their sums are added through LDS in order.  (A v_mfma_f64_16x16x4 holds its
+// SIMD for 75 cycles: one wave per tile chained 32 steps of 300 cycles and more, and
+// tiles large enough for that left many SIMDs with none.)  N = 5500, inverses
+// included: 256 right-hand sides 657 -> 400 us, one 289 -> 178; 512-row blocks
+// against 256 save 90 of that.  256 right-hand sides cost the matrix cores 115 us.
+
 // k_solve_diag: x_k = inv_k r_k (TR: with inv_k's transpose) for the block's
-// rows, 64 rows (grid y) of 16 right-hand sides per workgroup, 16 rows a wave;
-// R [B][N] what is left of the right-hand sides, X [B][N] the solution.
+// rows, 16 rows (grid y) of 16 right-hand sides per workgroup; R [B][N] what is
+// left of the right-hand sides, X [B][N] the solution.
 template <bool TR>
 __global__ __launch_bounds__(256, 2) void k_solve_diag(const double* __restrict__ inv, int64_t N, int64_t k0, int64_t B,
                                                      const double* __restrict__ R, double* __restrict__ X) {
+  __shared__ double red[4][4][64];
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-  const int w0 = 64 * blockIdx.y + 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nb = (int)min((int64_t)SB, N - k0);
-  if (w0 >= nb) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w0 = 16 * blockIdx.y, nb = (int)min((int64_t)SB, N - k0);
   const int64_t b0 = (int64_t)blockIdx.x * 16;
   const double* V = inv + (size_t)(k0 / SB) * SB * SB;
   const double* r = R + (size_t)min(b0 + i, B - 1) * N + k0 + 4 * g;
   const int row = w0 + i;
-  const int kb = TR ? w0 : 0;
+  const int kb = (TR ? w0 : 0) + 16 * wave;
   const int ke = min((nb + 15) & ~15, TR ? SB : w0 + 16);
-  constexpr int D = 4;
+  constexpr int D = 8;  // a wave's steps, all in flight
   d4 acc = {0.0, 0.0, 0.0, 0.0}, x[D], v[D];
-  auto load = [&](int s, int q, int left) {  // left: columns from the lane's first on (4: all)
-    const int k = kb + 16 * s;
-    x[q] = frag_row(r + k, left);
+  pipelined<D>((ke - kb + 63) / 64, [&](int s, int q) {
+    const int k = kb + 64 * s;
+    x[q] = frag_row(r + k, nb - k - 4 * g);  // (what is left of the block from the lane's first column on)
     v[q] = TR ? frag_col(V + (size_t)(k + 4 * g) * SB + row, SB, 4) : frag_row(V + (size_t)row * SB + k + 4 * g, 4);
-  };
-  auto use = [&](int q) { mma16(x[q], v[q], acc); };
-  const int n = (ke - kb) / 16;
-  if (nb == SB) pipelined<D>(n, [&](int s, int q) { load(s, q, 4); }, use);
-  else pipelined<D>(n, [&](int s, int q) { load(s, q, nb - (kb + 16 * s) - 4 * g); }, use);
-  if (row >= nb) return;
+  }, [&](int q) { mma16(x[q], v[q], acc); });
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
-    if (b0 + g + 4 * q < B) X[(size_t)(b0 + g + 4 * q) * N + k0 + row] = acc[q];
+  for (int q = 0; q < 4; ++q) red[wave][q][lane] = acc[q];
+  __syncthreads();
+  const int64_t b = b0 + g + 4 * wave;  // wave w adds and writes register w
+  if (row < nb && b < B)
+    X[(size_t)b * N + k0 + row] = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
 }
 
 // k_solve_update: removes the solved block from the rows still to come
 // (forward: after it, r_i -= sum_t L[i][k0+t] x_{k0+t}; TR: before it,
-// r_i -= sum_t L[k0+t][i] x_{k0+t}).  A workgroup takes WR x 32 rows x 64
-// right-hand sides, a wave 16 WR x 32 right-hand sides.  What bounds it is the
-// L2: L and x cross it once per 64 right-hand sides and once per WR x 32 rows,
-// so the wide tile is used while there are enough of them to fill the chip, and
-// workgroups are numbered so that one XCD's L2 holds the same rows of L for all
-// right-hand sides.
-template <bool TR, int WR>
+// r_i -= sum_t L[k0+t][i] x_{k0+t}), 32 rows x 16 WB right-hand sides a
+// workgroup.  Workgroups are numbered so that one XCD's L2 holds the same rows of
+// L for all right-hand sides.
+template <bool TR, int WB>
 __global__ __launch_bounds__(256, 2) void k_solve_update(const double* __restrict__ L, int64_t N, int64_t k0, int64_t B,
                                                       int gy, const double* __restrict__ X, double* __restrict__ R) {
+  __shared__ double red[4][2 * WB][4][64];
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nb = (int)min((int64_t)SB, N - k0);
   const int n = gridDim.x, q8 = n >> 3, r8 = n & 7, xc = blockIdx.x & 7;  // block b runs on XCD b % 8
   const int id = xc * q8 + min(xc, r8) + (blockIdx.x >> 3);
-  const int64_t row0 = (TR ? 0 : k0 + SB) + (int64_t)(id / gy) * (32 * WR) + 16 * WR * (wave & 1);
-  const int64_t row_end = TR ? k0 : N;
-  const int64_t b0 = (int64_t)(id % gy) * 64 + 32 * (wave >> 1);
-  if (b0 >= B || row0 >= row_end) return;
-  const double* x[2];
-  int64_t rw[WR];
+  const int64_t row0 = (TR ? 0 : k0 + SB) + (int64_t)(id / gy) * 32, row_end = TR ? k0 : N;
+  const int64_t b0 = (int64_t)(id % gy) * (16 * WB);
+  const double* x[WB];
+  int64_t rw[2];
 #pragma unroll
-  for (int a = 0; a < 2; ++a) x[a] = X + (size_t)min(b0 + 16 * a + i, B - 1) * N + k0;
+  for (int a = 0; a < WB; ++a) x[a] = X + (size_t)min(b0 + 16 * a + i, B - 1) * N + k0;
 #pragma unroll
-  for (int c = 0; c < WR; ++c) rw[c] = min(row0 + 16 * c + i, row_end - 1);
-  d4 acc[2][WR];
+  for (int c = 0; c < 2; ++c) rw[c] = min(row0 + 16 * c + i, row_end - 1);
+  d4 acc[WB][2];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < WB; ++a)
 #pragma unroll
-    for (int c = 0; c < WR; ++c) acc[a][c] = d4{0.0, 0.0, 0.0, 0.0};
-  constexpr int D = 3;
-  d4 xv[D][2], lv[D][WR];
+    for (int c = 0; c < 2; ++c) acc[a][c] = d4{0.0, 0.0, 0.0, 0.0};
+  constexpr int D = 4;
+  d4 xv[D][WB], lv[D][2];
   auto load = [&](int s, int q, int left) {  // left: columns from the lane's first on (4: all)
-    const int kk = 16 * s + 4 * g;
+    const int kk = 64 * s + 16 * wave + 4 * g;
 #pragma unroll
-    for (int a = 0; a < 2; ++a) xv[q][a] = frag_row(x[a] + kk, left);
+    for (int a = 0; a < WB; ++a) xv[q][a] = frag_row(x[a] + kk, left);
 #pragma unroll
-    for (int c = 0; c < WR; ++c)
+    for (int c = 0; c < 2; ++c)
       lv[q][c] = TR ? frag_col(L + (size_t)(k0 + kk) * N + rw[c], N, left)
                     : frag_row(L + (size_t)rw[c] * N + k0 + kk, left);
   };
   auto use = [&](int q) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < WB; ++a)
 #pragma unroll
-      for (int c = 0; c < WR; ++c) mma16(xv[q][a], lv[q][c], acc[a][c]);
+      for (int c = 0; c < 2; ++c) mma16(xv[q][a], lv[q][c], acc[a][c]);
   };
-  if (nb == SB) pipelined<D>(SB / 16, [&](int s, int q) { load(s, q, 4); }, use);
-  else pipelined<D>((nb + 15) / 16, [&](int s, int q) { load(s, q, nb - 16 * s - 4 * g); }, use);
+  if (nb == SB)
+    pipelined<D>(SB / 64, [&](int s, int q) { load(s, q, 4); }, use);
+  else
+    pipelined<D>((nb - 16 * wave + 63) / 64,
+                 [&](int s, int q) { load(s, q, nb - (64 * s + 16 * wave) - 4 * g); }, use);
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < WB; ++a)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int64_t b = b0 + 16 * a + g + 4 * q;
-      if (b >= B) continue;
+    for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int c = 0; c < WR; ++c)
-        if (row0 + 16 * c + i < row_end) R[(size_t)b * N + row0 + 16 * c + i] -= acc[a][c][q];
-    }
+      for (int q = 0; q < 4; ++q) red[wave][2 * a + c][q][lane] = acc[a][c][q];
+  __syncthreads();
+  // the 2 WB tiles of 4 registers, in turn to the waves
+  for (int e = wave; e < 8 * WB; e += 4) {
+    const int t = e >> 2, q = e & 3;
+    const int64_t b = b0 + 16 * (t >> 1) + g + 4 * q, row = row0 + 16 * (t & 1) + i;
+    if (b < B && row < row_end)
+      R[(size_t)b * N + row] -= ((red[0][t][q][lane] + red[1][t][q][lane]) + red[2][t][q][lane]) + red[3][t][q][lane];
+  }
 }
 
 // r = data - mu (FP64), [B][N]
@@ -542,27 +558,27 @@ hipError_t launch_tri_inverse(const double* L, int64_t N, double* inv, hipStream
   // whole SB blocks: the merges of a partial last block read identity rows
   const int64_t ns = (N + SB - 1) / SB;
   hipLaunchKernelGGL(k_tri_inv64, dim3((unsigned)(ns * (SB / DB))), dim3(256), 0, s, L, N, inv);
-  static_assert(SB == 256, "the merges go 64 -> 128 -> 256");
-  if (N > 64) hipLaunchKernelGGL((k_tri_merge<64>), dim3((unsigned)(ns * 2), 2), dim3(256), 0, s, L, N, inv);
-  if (N > 128) hipLaunchKernelGGL((k_tri_merge<128>), dim3((unsigned)ns, 4), dim3(512), 0, s, L, N, inv);
+  static_assert(SB == 512, "the merges go 64 -> 128 -> 256 -> 512");
+  if (N > 64) hipLaunchKernelGGL((k_tri_merge<64, 2>), dim3((unsigned)(ns * 4), 2), dim3(256), 0, s, L, N, inv);
+  if (N > 128) hipLaunchKernelGGL((k_tri_merge<128, 2>), dim3((unsigned)(ns * 2), 4), dim3(512), 0, s, L, N, inv);
+  if (N > 256) hipLaunchKernelGGL((k_tri_merge<256, 1>), dim3((unsigned)ns, 16), dim3(1024), 0, s, L, N, inv);
   return hipGetLastError();
 }
 
 template <bool TR>
 static void solve_pass(const double* L, int64_t N, const double* inv, double* R, double* X, int64_t B, hipStream_t s) {
-  const int gy = (int)((B + 63) / 64);
   const int64_t last = (N - 1) / SB * SB;
   for (int64_t step = 0; step <= last; step += SB) {
     const int64_t k0 = TR ? last - step : step;
     const int64_t nb = std::min<int64_t>(SB, N - k0), rows = TR ? k0 : N - k0 - SB;
-    const dim3 gd((unsigned)((B + 15) / 16), (unsigned)((nb + 63) / 64));
+    const dim3 gd((unsigned)((B + 15) / 16), (unsigned)((nb + 15) / 16));
     hipLaunchKernelGGL((k_solve_diag<TR>), gd, dim3(256), 0, s, inv, N, k0, B, R, X);
     if (rows <= 0) continue;
-    const int64_t wide = (rows + 63) / 64 * gy, narrow = (rows + 31) / 32 * gy;
-    if (wide >= 256)
-      hipLaunchKernelGGL((k_solve_update<TR, 2>), dim3((unsigned)wide), dim3(256), 0, s, L, N, k0, B, gy, X, R);
-    else
-      hipLaunchKernelGGL((k_solve_update<TR, 1>), dim3((unsigned)narrow), dim3(256), 0, s, L, N, k0, B, gy, X, R);
+    // (16 right-hand sides at most: half the products)
+    const int gy = (int)(B <= 16 ? 1 : (B + 31) / 32);
+    const dim3 gu((unsigned)((rows + 31) / 32 * gy));
+    if (B <= 16) hipLaunchKernelGGL((k_solve_update<TR, 1>), gu, dim3(256), 0, s, L, N, k0, B, gy, X, R);
+    else hipLaunchKernelGGL((k_solve_update<TR, 2>), gu, dim3(256), 0, s, L, N, k0, B, gy, X, R);
   }
 }
 
@@ -575,10 +591,9 @@ hipError_t launch_dense_solve(const double* L, int64_t N, const double* inv, dou
 }
 
 hipError_t launch_dense_loglike(const float* mu, int64_t B, int64_t N, const double* data, const double* L, double c0,
-                                double* inv, double* Z, double* X, double* loglike, float* dmu, hipStream_t s) {
+                                const double* inv, double* Z, double* X, double* loglike, float* dmu, hipStream_t s) {
   const int64_t n = B * N;
-  hipError_t e = launch_tri_inverse(L, N, inv, s);
-  if (e != hipSuccess) return e;
+  hipError_t e;
   hipLaunchKernelGGL(k_resid, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, mu, data, N, B, Z);
   if ((e = launch_dense_solve(L, N, inv, Z, X, B, 0, s)) != hipSuccess) return e;
   hipLaunchKernelGGL(k_sq_sum, dim3((unsigned)B), dim3(256), 0, s, X, N, c0, loglike);

@@ -351,7 +351,7 @@ hipError_t launch_ragged_reduce(int max_jobs, const RaggedArgs& a, double* theta
 // B means, with Z and X as [B][N] workspaces and dmu (may be null) =
 // C^-1 (data - mu_b) as float
 constexpr int DENSE_PANEL = 64;
-constexpr int DENSE_SOLVE_BLOCK = 256;
+constexpr int DENSE_SOLVE_BLOCK = 512;
 inline size_t tri_inverse_size(int64_t N) {
   return (size_t)((N + DENSE_SOLVE_BLOCK - 1) / DENSE_SOLVE_BLOCK) * DENSE_SOLVE_BLOCK * DENSE_SOLVE_BLOCK;
 }
@@ -360,7 +360,7 @@ hipError_t launch_tri_inverse(const double* L, int64_t N, double* inv, hipStream
 hipError_t launch_dense_solve(const double* L, int64_t N, const double* inv, double* R, double* X, int64_t B,
                               int transpose, hipStream_t s);
 hipError_t launch_dense_loglike(const float* mu, int64_t B, int64_t N, const double* data, const double* L, double c0,
-                                double* inv, double* Z, double* X, double* loglike, float* dmu, hipStream_t s);
+                                const double* inv, double* Z, double* X, double* loglike, float* dmu, hipStream_t s);
 // out[o] = sum of the forward partials of the launch's live slices, for o in
 // [range[0], range[1]) (device values), grid sized for max_out floats
 hipError_t launch_ragged_slice_sum(const int* ncols, int waves, int Na, int max_slices, const float* part,
