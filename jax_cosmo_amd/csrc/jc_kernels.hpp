@@ -299,6 +299,19 @@ __host__ __device__ inline int ragged_slices(int tiles, int waves, int Na, int m
   return s < 1 ? 1 : s;
 }
 
+// Blocks that hold every unit of `tiles` live tiles or fewer: ragged_slices
+// rounds 2048 / (tiles x waves) up, so tiles x slices <= 2048 / waves + tiles; an XCD
+// holds up to one tile more than an eighth.
+inline int ragged_fwd_blocks(int tiles, int waves, int max_slices) {
+  const int per_xcd = (tiles + 7) / 8;
+  int most = 0;  // units of the fullest XCD
+  for (int t = 1; t <= tiles; ++t) {
+    const int s = (2048 + t * waves - 1) / (t * waves), n = (t + 7) / 8 * (s < max_slices ? s : max_slices);
+    most = n > most ? n : most;
+  }
+  return 8 * (most > per_xcd ? most : per_xcd);
+}
+
 // launchers (defined next to their kernels)
 hipError_t launch_tables(int nd, const TablesArgs& a, hipStream_t s, int num_cu, int variant = 0);
 // ctile: cosmologies per block of the forward kernel (1, 4, 8, 16; 0 = by rule)
@@ -337,7 +350,7 @@ hipError_t launch_adjoint(int T, const LimberArgs& a, hipStream_t s);
 // [nsl][B][n_ell][7] (nsl = 1: the partials of an unsliced launch)
 hipError_t launch_theta_reduce(const float* theta_col, int nsl, int B, int n_ell, double* theta, hipStream_t s);
 hipError_t launch_pk_eval(const PkArgs& a, hipStream_t s);
-// grid sized for max_cols columns; blocks beyond *ncols exit at once
+// for up to max_cols columns
 hipError_t launch_limber_ragged(int max_cols, const RaggedArgs& a, hipStream_t s);
 hipError_t launch_ragged_adjoint(int max_jobs, const RaggedArgs& a, hipStream_t s);
 hipError_t launch_ragged_reduce(int max_jobs, const RaggedArgs& a, double* theta, hipStream_t s);

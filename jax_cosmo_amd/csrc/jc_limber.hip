@@ -867,8 +867,8 @@ hipError_t launch_pk_eval(const PkArgs& a, hipStream_t s) {
 // ahead, and, when the tile's columns belong to at most two requests, their
 // transfer tables staged into LDS (otherwise read through the L1/L2).
 template <int T, bool STAGED>
-__device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int tile0, const int nsl, float4* lds4,
-                                                const uint64_t starts) {
+__device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int tile0, const int nsl,
+                                                const int slice, float4* lds4, const uint64_t starts) {
   constexpr int P = T * (T + 1) / 2;
   constexpr int RCH = RedChunk<P>::value;
   float* red = reinterpret_cast<float*>(lds4);
@@ -898,7 +898,7 @@ __device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int t
   const EllT lt = ell_tab(ell, (double)A.crec[(size_t)c * NCREC + CR_EHINVH]);
   // this wave's share of the a range
   const int chunk = (A.Na + nsl * nwv - 1) / (nsl * nwv);
-  const int m0 = min(A.Na, ((int)blockIdx.y * nwv + wave) * chunk);
+  const int m0 = min(A.Na, (slice * nwv + wave) * chunk);
   const int m1 = min(A.Na, m0 + chunk);
 
   float acc[P];
@@ -965,7 +965,7 @@ __device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int t
   }
   if (wave != 0 || !valid) return;
   const float lf = (float)(::sqrt((ell - 1.0) * ell * (ell + 1.0) * (ell + 2.0)) / ((ell + 0.5) * (ell + 0.5)));
-  float* out = nsl > 1 ? A.part + (size_t)blockIdx.y * A.part_stride : A.out;
+  float* out = nsl > 1 ? A.part + (size_t)slice * A.part_stride : A.out;
   const float lm3 = ell_m3(ell);
   int p = 0;
 #pragma unroll
@@ -980,16 +980,21 @@ __device__ __forceinline__ void ragged_fwd_tile(const RaggedArgs& A, const int t
   }
 }
 
+// One block per live (tile, slice) unit, within a grid of ragged_fwd_blocks: with
+// one per tile and slice of the batch's capacity, a tenth of a full batch was 13 000
+// workgroups, nearly all empty (34 -> 31 us; the slice sum's 22 000, 12 -> 5).  (A
+// loop over units in fewer blocks spilled 166 registers.)
 __global__ __launch_bounds__(256, 4) void k_limber_ragged_fwd(RaggedArgs A) {
   extern __shared__ float4 lds4[];
   const int ncols = *A.ncols;
-  // live tiles dealt to the 8 XCDs in contiguous ranges, as k_limber_ragged_adj
+  // live tiles dealt to the 8 XCDs in contiguous ranges (the grid is a multiple of 8)
   const int live = (ncols + 63) >> 6;
   const int nsl = ragged_slices(live, A.waves, A.Na, A.max_slices);
-  if ((int)blockIdx.y >= nsl) return;
-  const int xq = live >> 3, xr = live & 7, xx = blockIdx.x & 7, xi = blockIdx.x >> 3;
-  if (xi >= xq + (xx < xr ? 1 : 0)) return;
-  const int tile0 = (xx * xq + min(xx, xr) + xi) * 64;
+  const int xq = live >> 3, xr = live & 7, xx = blockIdx.x & 7, u = blockIdx.x >> 3;
+  const int mine = xq + (xx < xr ? 1 : 0);  // this XCD's tiles
+  if (u >= mine * nsl) return;
+  const int slice = u / mine;
+  const int tile0 = (xx * xq + min(xx, xr) + u - slice * mine) * 64;
   const int first = A.cols[tile0].job;
   const int T = __builtin_amdgcn_readfirstlane(A.jobs[first].T);
   // the requests of the tile: a new one starts at each lane whose job
@@ -1001,29 +1006,29 @@ __global__ __launch_bounds__(256, 4) void k_limber_ragged_fwd(RaggedArgs A) {
   const uint64_t starts = __ballot(lane > 0 && job != prev);
   if (__popcll(starts) <= 1) {
     switch (T) {
-      case 1: ragged_fwd_tile<1, true>(A, tile0, nsl, lds4, starts); break;
-      case 2: ragged_fwd_tile<2, true>(A, tile0, nsl, lds4, starts); break;
-      case 3: ragged_fwd_tile<3, true>(A, tile0, nsl, lds4, starts); break;
-      case 4: ragged_fwd_tile<4, true>(A, tile0, nsl, lds4, starts); break;
-      case 5: ragged_fwd_tile<5, true>(A, tile0, nsl, lds4, starts); break;
-      case 6: ragged_fwd_tile<6, true>(A, tile0, nsl, lds4, starts); break;
-      case 7: ragged_fwd_tile<7, true>(A, tile0, nsl, lds4, starts); break;
-      case 8: ragged_fwd_tile<8, true>(A, tile0, nsl, lds4, starts); break;
-      case 9: ragged_fwd_tile<9, true>(A, tile0, nsl, lds4, starts); break;
-      default: ragged_fwd_tile<10, true>(A, tile0, nsl, lds4, starts); break;
+      case 1: ragged_fwd_tile<1, true>(A, tile0, nsl, slice, lds4, starts); break;
+      case 2: ragged_fwd_tile<2, true>(A, tile0, nsl, slice, lds4, starts); break;
+      case 3: ragged_fwd_tile<3, true>(A, tile0, nsl, slice, lds4, starts); break;
+      case 4: ragged_fwd_tile<4, true>(A, tile0, nsl, slice, lds4, starts); break;
+      case 5: ragged_fwd_tile<5, true>(A, tile0, nsl, slice, lds4, starts); break;
+      case 6: ragged_fwd_tile<6, true>(A, tile0, nsl, slice, lds4, starts); break;
+      case 7: ragged_fwd_tile<7, true>(A, tile0, nsl, slice, lds4, starts); break;
+      case 8: ragged_fwd_tile<8, true>(A, tile0, nsl, slice, lds4, starts); break;
+      case 9: ragged_fwd_tile<9, true>(A, tile0, nsl, slice, lds4, starts); break;
+      default: ragged_fwd_tile<10, true>(A, tile0, nsl, slice, lds4, starts); break;
     }
   } else {
     switch (T) {
-      case 1: ragged_fwd_tile<1, false>(A, tile0, nsl, lds4, starts); break;
-      case 2: ragged_fwd_tile<2, false>(A, tile0, nsl, lds4, starts); break;
-      case 3: ragged_fwd_tile<3, false>(A, tile0, nsl, lds4, starts); break;
-      case 4: ragged_fwd_tile<4, false>(A, tile0, nsl, lds4, starts); break;
-      case 5: ragged_fwd_tile<5, false>(A, tile0, nsl, lds4, starts); break;
-      case 6: ragged_fwd_tile<6, false>(A, tile0, nsl, lds4, starts); break;
-      case 7: ragged_fwd_tile<7, false>(A, tile0, nsl, lds4, starts); break;
-      case 8: ragged_fwd_tile<8, false>(A, tile0, nsl, lds4, starts); break;
-      case 9: ragged_fwd_tile<9, false>(A, tile0, nsl, lds4, starts); break;
-      default: ragged_fwd_tile<10, false>(A, tile0, nsl, lds4, starts); break;
+      case 1: ragged_fwd_tile<1, false>(A, tile0, nsl, slice, lds4, starts); break;
+      case 2: ragged_fwd_tile<2, false>(A, tile0, nsl, slice, lds4, starts); break;
+      case 3: ragged_fwd_tile<3, false>(A, tile0, nsl, slice, lds4, starts); break;
+      case 4: ragged_fwd_tile<4, false>(A, tile0, nsl, slice, lds4, starts); break;
+      case 5: ragged_fwd_tile<5, false>(A, tile0, nsl, slice, lds4, starts); break;
+      case 6: ragged_fwd_tile<6, false>(A, tile0, nsl, slice, lds4, starts); break;
+      case 7: ragged_fwd_tile<7, false>(A, tile0, nsl, slice, lds4, starts); break;
+      case 8: ragged_fwd_tile<8, false>(A, tile0, nsl, slice, lds4, starts); break;
+      case 9: ragged_fwd_tile<9, false>(A, tile0, nsl, slice, lds4, starts); break;
+      default: ragged_fwd_tile<10, false>(A, tile0, nsl, slice, lds4, starts); break;
     }
   }
 }
@@ -1032,7 +1037,7 @@ hipError_t launch_limber_ragged(int max_cols, const RaggedArgs& a, hipStream_t s
   if (a.waves < 1 || a.waves > 4 || max_cols < 64 || (max_cols % 64) != 0) return hipErrorInvalidValue;
   if (a.max_slices < 1 || a.max_slices > 64 || !a.ehtab) return hipErrorInvalidValue;
   if (a.max_slices > 1 && !a.part) return hipErrorInvalidValue;
-  const dim3 grid(max_cols / 64, a.max_slices);
+  const dim3 grid(ragged_fwd_blocks(max_cols / 64, a.waves, a.max_slices));
   // two transfer tables, or the reduction's [waves - 1][32][64] partials
   const size_t sm = std::max((size_t)2 * NEHQ * sizeof(float4), (size_t)(a.waves - 1) * 32 * 64 * sizeof(float));
   hipLaunchKernelGGL(k_limber_ragged_fwd, grid, dim3(64 * a.waves), sm, s, a);
@@ -1041,24 +1046,26 @@ hipError_t launch_limber_ragged(int max_cols, const RaggedArgs& a, hipStream_t s
 
 // out[o] = part[0][o] + part[1][o] + ... over the forward launch's live
 // slices (in order), for o in [range[0], range[1]); nothing with one slice
-// (the Limber kernel then wrote out itself)
+// (the Limber kernel then wrote out itself); blocks walk the live range
 __global__ void k_ragged_slice_sum(const int* __restrict__ ncols, int waves, int Na, int max_slices,
                                    const float* __restrict__ part, int64_t stride, const int* __restrict__ range,
                                    float* __restrict__ out) {
   const int nsl = ragged_slices((*ncols + 63) >> 6, waves, Na, max_slices);
   if (nsl <= 1) return;
-  const int64_t o = range[0] + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= range[1]) return;
-  float v = part[o];
-  for (int k = 1; k < nsl; ++k) v += part[(size_t)k * stride + o];
-  out[o] = v;
+  const int64_t end = range[1];
+  for (int64_t o = range[0] + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; o < end;
+       o += (int64_t)gridDim.x * blockDim.x) {
+    float v = part[o];
+    for (int k = 1; k < nsl; ++k) v += part[(size_t)k * stride + o];
+    out[o] = v;
+  }
 }
 
 hipError_t launch_ragged_slice_sum(const int* ncols, int waves, int Na, int max_slices, const float* part,
                                    int64_t part_stride, const int* range, int64_t max_out, float* out,
                                    hipStream_t s) {
   if (max_out <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_ragged_slice_sum, dim3((unsigned)((max_out + 255) / 256)), dim3(256), 0, s, ncols, waves,
+  hipLaunchKernelGGL(k_ragged_slice_sum, dim3((unsigned)std::min<int64_t>((max_out + 255) / 256, 1024)), dim3(256), 0, s, ncols, waves,
                      Na, max_slices, part, part_stride, range, out);
   return hipGetLastError();
 }

@@ -73,7 +73,7 @@ JC_D void load_seg(const float* tab, int L, float* chi, float* sl) {
 }  // namespace
 
 template <int ND, int CT, int NW, int SL>
-__global__ __launch_bounds__(WL_M * SL) void k_wl(WLArgs A) {
+__device__ __forceinline__ void wl_block(const WLArgs& A) {
   using Sf = typename Types<ND>::F;
   constexpr int W = ND + 1;
   constexpr int TS = NCHI * 2 * W;                  // floats of a cosmology's table
@@ -241,11 +241,37 @@ __global__ __launch_bounds__(WL_M * SL) void k_wl(WLArgs A) {
 }
 
 template <int ND, int CT, int NW, int SL>
-static hipError_t wl_launch(const WLArgs& a, hipStream_t s) {
+__global__ __launch_bounds__(WL_M * SL) void k_wl(WLArgs A) {
+  wl_block<ND, CT, NW, SL>(A);
+}
+
+// Served batches: the grid is made for a full batch, the number of cosmologies
+// is on the device.  CT of them share a block in a full batch; below `few` of
+// them, which would leave most of the chip idle, two do, and 8 waves
+// split the inner nodes (three branches of 50 cosmologies side by side: 40 -> 21 us
+// each).
+template <int CT, int NW, int SL>
+__global__ __launch_bounds__(WL_M * SL) void k_wl_live(WLArgs A, int few) {
+  if (*A.dB <= few) wl_block<0, 2, NW, SL>(A);
+  else wl_block<0, CT, NW, SL>(A);
+}
+
+template <int ND, int CT, int NW, int SL>
+static hipError_t wl_launch(const WLArgs& a, int num_cu, hipStream_t s) {
   constexpr int W = ND + 1;
   constexpr size_t sm = std::max((size_t)CT * NCHI * 2 * W, (size_t)SL * NW * W * 64) * sizeof(float);
   static_assert(sm <= 160 * 1024, "LDS of a block");
-  const dim3 grid((a.Na - 1 + WL_M - 1) / WL_M, (a.B + CT - 1) / CT);
+  const int nb = (a.Na - 1 + WL_M - 1) / WL_M;
+  if constexpr (ND == 0 && CT > 2) {
+    if (a.dB) {
+      // two a block up to 4 blocks of one cosmology per CU (the rule below)
+      const int few = std::min(4 * num_cu / nb, a.B);
+      const dim3 grid(nb, std::max((few + 1) / 2, (a.B + CT - 1) / CT));
+      hipLaunchKernelGGL((k_wl_live<CT, NW, SL>), grid, dim3(WL_M * SL), sm, s, a, few);
+      return hipGetLastError();
+    }
+  }
+  const dim3 grid(nb, (a.B + CT - 1) / CT);
   hipLaunchKernelGGL((k_wl<ND, CT, NW, SL>), grid, dim3(WL_M * SL), sm, s, a);
   return hipGetLastError();
 }
@@ -265,20 +291,20 @@ static hipError_t wl_launch_nw(int nd, int ctile, const WLArgs& a, int num_cu, h
   if (nd == 0) {
     if (ctile == 0) ctile = blocks <= num_cu ? 1 : (blocks <= 2 * num_cu ? 2 : (blocks <= 16 * num_cu ? 4 : 8));
     switch (ctile) {
-      case 1: return wl_launch<0, 1, NW, 8>(a, s);
-      case 2: return wl_launch<0, 2, NW, 8>(a, s);
-      case 4: return wl_launch<0, 4, NW, 8>(a, s);
-      case 8: return wl_launch<0, 8, NW, 4>(a, s);
-      case 16: return wl_launch<0, 16, NW, 4>(a, s);
+      case 1: return wl_launch<0, 1, NW, 8>(a, num_cu, s);
+      case 2: return wl_launch<0, 2, NW, 8>(a, num_cu, s);
+      case 4: return wl_launch<0, 4, NW, 8>(a, num_cu, s);
+      case 8: return a.dB ? wl_launch<0, 8, NW, 8>(a, num_cu, s) : wl_launch<0, 8, NW, 4>(a, num_cu, s);
+      case 16: return wl_launch<0, 16, NW, 4>(a, num_cu, s);
       default: return hipErrorInvalidValue;
     }
   }
-  if (nd == 1) return blocks <= num_cu ? wl_launch<1, 1, NW, 8>(a, s) : wl_launch<1, 1, NW, 4>(a, s);
+  if (nd == 1) return blocks <= num_cu ? wl_launch<1, 1, NW, 8>(a, num_cu, s) : wl_launch<1, 1, NW, 4>(a, num_cu, s);
   if (nd != 7) return hipErrorInvalidValue;
   if constexpr (NW <= 5) {  // (with 10 bins the partial sums of 8 waves would not fit the LDS)
-    if (blocks <= 2 * num_cu) return wl_launch<7, 1, NW, 8>(a, s);
+    if (blocks <= 2 * num_cu) return wl_launch<7, 1, NW, 8>(a, num_cu, s);
   }
-  return blocks <= 4 * num_cu ? wl_launch<7, 1, NW, 4>(a, s) : wl_launch<7, 2, NW, 4>(a, s);
+  return blocks <= 4 * num_cu ? wl_launch<7, 1, NW, 4>(a, num_cu, s) : wl_launch<7, 2, NW, 4>(a, num_cu, s);
 }
 
 hipError_t launch_wl(int nd, int ctile, const WLArgs& a, int num_cu, hipStream_t s) {
