@@ -60,8 +60,8 @@ extern "C" {
 /* flags */
 #define JC_DEVICE_PTRS 1 /* array arguments are device pointers; the call is
                             asynchronous on the context stream */
-#define JC_DEVICE_FACTOR 2 /* jc_gaussian_loglike_dense: L is a device pointer and
-                            * the other arrays are host pointers */
+#define JC_DEVICE_FACTOR 2 /* jc_dense_cholesky, jc_gaussian_loglike_dense: L is a
+                            * device pointer, the other arrays are host pointers */
 
 typedef struct jc_ctx jc_ctx;
 

@@ -572,13 +572,13 @@ class _Likelihood:
             raise ValueError("expected a square dense covariance, got shape %s" % (C.shape,))
         N = C.shape[0]
         stream = torch.cuda.current_stream()
-        L = torch.from_numpy(C).to("cuda")
+        L = torch.empty((N, N), dtype=torch.float64, device="cuda")
         ld = ctypes.c_double()
         with self._lock:
             self.set_stream(stream.cuda_stream)
             try:
-                check(self.lib.jc_dense_cholesky(self.handle, _P(L.data_ptr()), N, _P(L.data_ptr()),
-                                                 ctypes.byref(ld), JC_DEVICE_PTRS))
+                check(self.lib.jc_dense_cholesky(self.handle, _ptr(C), N, _P(L.data_ptr()), ctypes.byref(ld),
+                                                 JC_DEVICE_FACTOR))
             finally:
                 self.reset_stream()
         return L, ld.value

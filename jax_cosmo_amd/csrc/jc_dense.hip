@@ -241,6 +241,7 @@ __global__ __launch_bounds__(256, 2) void k_chol_first(double* __restrict__ A, i
                                                      double* __restrict__ dlog, int* __restrict__ bad) {
   __shared__ double S[DB * LS], V[DB * LS];
   const int nb = (int)min((int64_t)DB, N);
+  if (threadIdx.x == 0) *bad = 0;  // (the thread that sets it)
   for (int e = threadIdx.x; e < DB * DB; e += 256) {
     const int i = e / DB, j = e - i * DB;
     S[i * LS + j] = i < nb && j <= i ? A[(size_t)i * N + j] : (i == j ? 1.0 : 0.0);
@@ -537,6 +538,22 @@ __global__ __launch_bounds__(256) void k_sq_sum(const double* __restrict__ Z, in
 __global__ void k_to_float(const double* __restrict__ x, int64_t n, float* __restrict__ y) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e < n) y[e] = (float)x[e];
+}
+
+// one row a block
+__global__ __launch_bounds__(256) void k_unpack_lower(const double* __restrict__ src, double* __restrict__ A, int64_t N,
+                                                      int64_t r0) {
+  const int64_t r = r0 + blockIdx.x;
+  const double* in = src + (tri_row(r) - tri_row(r0));
+  double* out = A + (size_t)r * N;
+#pragma unroll 4
+  for (int64_t c = threadIdx.x; c <= r; c += 256) out[c] = in[c];
+}
+
+hipError_t launch_unpack_lower(const double* src, double* A, int64_t N, int64_t r0, int64_t r1, hipStream_t s) {
+  if (r1 <= r0) return hipSuccess;
+  hipLaunchKernelGGL(k_unpack_lower, dim3((unsigned)(r1 - r0)), dim3(256), 0, s, src, A, N, r0);
+  return hipGetLastError();
 }
 
 hipError_t launch_dense_cholesky(double* A, int64_t N, double* inv, double* dlog, int* bad, hipStream_t s) {

@@ -189,12 +189,18 @@ int eval_pz(jc_ctx* ctx, TracerSet* ts, int i, const std::vector<double>& z, std
 // 10 tracers, 100 ell, n_z 512: 103 -> 92 us).  The call's final
 // synchronisation hands the buffers back.
 constexpr size_t PIN_IN = 128u << 10, PIN_OUT = 512u << 10;
+// Pinned pieces that a host covariance's lower triangle passes through
+// (allocated by a context's first such call).
+constexpr int TRI_PIECES = 4;
+constexpr size_t TRI_PIECE = 2u << 20;
 
 struct jc_ctx {
   using TracerSet = jch::TracerSet;
   template <class T> using DevBuf = jch::DevBuf<T>;
   int device = 0;
   unsigned char *pin_in = nullptr, *pin_out = nullptr;  // PIN_IN and PIN_OUT bytes, read and written by the device in place
+  unsigned char* tri_stage = nullptr;       // [TRI_PIECES][TRI_PIECE]
+  hipEvent_t tri_free[TRI_PIECES] = {};     // recorded after a piece has been read
   unsigned char* scratch = nullptr;  // this device's scratch array (jc_angular_cl_noalloc)
   hipStream_t own = nullptr;
   hipStream_t stream = nullptr;
@@ -210,10 +216,9 @@ struct jc_ctx {
   // likelihood workspace: inputs staged from host, mean, cotangent, partials
   DevBuf<double> lk_cosmo, lk_ell, lk_data, lk_prec, lk_part, lk_out, lk_grad, lk_inv;
   DevBuf<float> lk_mu, lk_s;
-  // dense likelihood workspace: staged matrix, log L_ii, non-SPD flag, [B][N]
+  // dense likelihood workspace: staged matrix, log L_ii and non-SPD flag, [B][N]
   // solves, inverses of the factor's diagonal blocks
   DevBuf<double> dn_mat, dn_dlog, dn_z, dn_x, dn_inv;
-  DevBuf<int> dn_bad;
   DevBuf<float> chitab, coef, crec, R, out, out_t, jac, cbar, theta_col, part;
   DevBuf<float4> ehtab;
   DevBuf<float> ehtab7;

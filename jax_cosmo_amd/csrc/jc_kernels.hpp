@@ -368,6 +368,13 @@ constexpr int DENSE_SOLVE_BLOCK = 512;
 inline size_t tri_inverse_size(int64_t N) {
   return (size_t)((N + DENSE_SOLVE_BLOCK - 1) / DENSE_SOLVE_BLOCK) * DENSE_SOLVE_BLOCK * DENSE_SOLVE_BLOCK;
 }
+// packed lower triangle: row r starts at tri_row(r) doubles and is padded to whole
+// 64-byte lines; rows [r0, r1) at src (pinned host memory) into the rows of A
+__host__ __device__ inline int64_t tri_row(int64_t r) {
+  const int64_t g = r >> 3;
+  return 32 * g * (g + 1) + (r & 7) * 8 * (g + 1);
+}
+hipError_t launch_unpack_lower(const double* src, double* A, int64_t N, int64_t r0, int64_t r1, hipStream_t s);
 hipError_t launch_dense_cholesky(double* A, int64_t N, double* inv, double* dlog, int* bad, hipStream_t s);
 hipError_t launch_tri_inverse(const double* L, int64_t N, double* inv, hipStream_t s);
 hipError_t launch_dense_solve(const double* L, int64_t N, const double* inv, double* R, double* X, int64_t B,
