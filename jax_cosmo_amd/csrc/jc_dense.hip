@@ -116,32 +116,12 @@ __device__ __forceinline__ double sqrt_rsqrt(double d, double& r) {
 }
 
 // V (lower triangle by 16 x 16 blocks) = the inverse of the lower triangular
-// 64 x 64 block in S, by the 256 threads of a block: wave w substitutes its
-// 16 x 16 diagonal block (column i in lane i), then
+// 64 x 64 block in S, by the 256 threads of a block, from the inverses of its
+// 16 x 16 diagonal blocks, which the caller has put into V:
 // V21 = -V22 (S21 V11), 16 and 32 wide.
-__device__ void tri64_inverse(const double* S, double* V) {
+__device__ void tri64_merge(const double* S, double* V) {
   double* Tm = V + 32;  // rows 0-31, columns 32-63: above the inverse's diagonal, not part of it
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  {
-    const int o = 16 * wave, i = lane & 15;
-    const double* L = S + o * LS + o;
-    double x[16];
-    const double rd = 1.0 / L[i * LS + i];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      double s0 = i == r ? 1.0 : 0.0, s1 = 0.0;
-#pragma unroll
-      for (int t = 0; t < r; ++t) {
-        if (t & 1) s1 -= L[r * LS + t] * x[t];
-        else s0 -= L[r * LS + t] * x[t];
-      }
-      x[r] = (s0 + s1) * lane_d(rd, r);
-    }
-    if (lane < 16) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) V[(o + r) * LS + o + i] = x[r];
-    }
-  }
   __syncthreads();
   const d4 zero = {0.0, 0.0, 0.0, 0.0};
   if (wave < 2) {
@@ -171,24 +151,57 @@ __device__ void tri64_inverse(const double* S, double* V) {
   __syncthreads();
 }
 
+// The same with nothing in V: wave w substitutes its 16 x 16 diagonal block
+// (column i in lane i) first.
+__device__ void tri64_inverse(const double* S, double* V) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  {
+    const int o = 16 * wave, i = lane & 15;
+    const double* L = S + o * LS + o;
+    double x[16];
+    const double rd = 1.0 / L[i * LS + i];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      double s0 = i == r ? 1.0 : 0.0, s1 = 0.0;
+#pragma unroll
+      for (int t = 0; t < r; ++t) {
+        if (t & 1) s1 -= L[r * LS + t] * x[t];
+        else s0 -= L[r * LS + t] * x[t];
+      }
+      x[r] = (s0 + s1) * lane_d(rd, r);
+    }
+    if (lane < 16) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) V[(o + r) * LS + o + i] = x[r];
+    }
+  }
+  tri64_merge(S, V);
+}
+
 // Factors the 64 x 64 block in S (lower triangle; identity past nb) in place
 // and leaves the inverse of its factor in the lower triangle (by 16 x 16
-// blocks) of V, by the 256 threads of a block.  16 columns at a time: one wave
+// blocks) of V, by the 256 threads of a block.  16 columns at a time: wave 0
 // factors them down all rows of the block (row o + i in lane i, so the rows
 // below the diagonal come with it; pivots and multipliers by readlane, no
-// barrier), then all waves update the rest as 16 x 16 products.
-// A chain of 64 pivots with barriers between them took 97 us.
+// barrier), then all waves update the rest as 16 x 16 products.  Beside it wave 1
+// does the same with 16 rows of the identity below the diagonal block, which
+// become its inverse (by substitution afterwards: 3 us more).  One block in LDS 16
+// us, 2.4 of them a panel (2.7 as L D L^T with the square roots at the end); with
+// barriers between 64 pivots 97 us.
 __device__ void chol64(double* S, double* V, int nb, double* dlog, int* bad) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __syncthreads();  // the caller has written S
   for (int jb = 0; jb < 4; ++jb) {
     const int o = 16 * jb;
-    if (wave == 0) {
-      double* row = S + min(o + lane, DB - 1) * LS + o;
-      double a[16];
+    const int r0 = wave == 0 ? min(o + lane, DB - 1) : o + (lane & 15);
+    double* row = S + r0 * LS + o;
+    double a[16];
+    if (wave < 2) {
 #pragma unroll
-      for (int c = 0; c < 16; ++c) a[c] = row[c];
-      double dg = 1.0;
+      for (int c = 0; c < 16; ++c) a[c] = wave == 1 && lane >= 16 ? (lane - 16 == c ? 1.0 : 0.0) : row[c];
+    }
+    __syncthreads();  // wave 1 has read the block that wave 0 will overwrite
+    if (wave < 2) {
       bool ok = true;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
@@ -196,18 +209,21 @@ __device__ void chol64(double* S, double* V, int nb, double* dlog, int* bad) {
         ok = ok && p > 0.0;
         const double d = p > 0.0 ? p : 1.0;  // keeps the rest finite; the caller reports the failure
         double r;
-        const double s = sqrt_rsqrt(d, r);
-        dg = lane == j ? s : dg;
-        a[j] = lane == j ? s : a[j] * r;
+        const double q = sqrt_rsqrt(d, r);
+        a[j] = lane == j ? q : a[j] * r;
 #pragma unroll
         for (int c = j + 1; c < 16; ++c) a[c] -= a[j] * lane_d(a[j], c);
       }
-      if (o + lane < DB) {
+      if (wave == 0) {
+        if (o + lane < DB) {
 #pragma unroll
-        for (int c = 0; c < 16; ++c) row[c] = lane >= c ? a[c] : 0.0;
+          for (int c = 0; c < 16; ++c) row[c] = lane >= c ? a[c] : 0.0;
+        }
+        if (!ok && lane == 0) *bad = 1;
+      } else if (lane >= 16 && lane < 32) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) V[(o + j) * LS + o + lane - 16] = a[j];
       }
-      if (lane < 16 && o + lane < nb) dlog[o + lane] = ::log(dg);
-      if (!ok && lane == 0) *bad = 1;
     }
     __syncthreads();
     int t = 0;
@@ -222,7 +238,8 @@ __device__ void chol64(double* S, double* V, int nb, double* dlog, int* bad) {
       }
     __syncthreads();
   }
-  tri64_inverse(S, V);
+  if (wave == 3 && lane < nb) dlog[lane] = ::log(S[lane * LS + lane]);
+  tri64_merge(S, V);
 }
 
 // the diagonal block in S (written by the caller) -> factor in A, inverse in inv
