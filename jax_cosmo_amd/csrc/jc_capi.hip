@@ -1285,20 +1285,28 @@ int jc_dense_solve(jc_ctx* ctx, const double* L, int64_t N, const double* R, int
   const double* d_L = nullptr;
   int rc = to_device(ctx, ctx->dn_mat, L, (size_t)N * N, dev, &d_L);
   if (rc) return rc;
-  // the solves are out of place: from a copy of R into the result, and, for
-  // C^-1 R, through a second workspace
-  HIPCHK(ctx->dn_z.reserve(n));
-  HIPCHK(ctx->dn_inv.reserve(tri_inverse_size(N)));
-  if (!dev || mode == 2) HIPCHK(ctx->dn_x.reserve(n));
-  double* res = dev ? X : ctx->dn_x.p;
-  HIPCHK(hipMemcpyAsync(ctx->dn_z.p, R, n * sizeof(double), dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-  HIPCHK(launch_tri_inverse(d_L, N, ctx->dn_inv.p, s));
-  if (mode == 2) {
-    HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_z.p, ctx->dn_x.p, nrhs, 0, s));
-    res = dev ? X : ctx->dn_z.p;
-    HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_x.p, res, nrhs, 1, s));
+  double* res = X;
+  if (N <= DENSE_PANEL) {
+    const double* d_R = nullptr;
+    if ((rc = to_device(ctx, ctx->dn_z, R, n, dev, &d_R))) return rc;
+    if (!dev) res = ctx->dn_z.p;
+    HIPCHK(launch_small_solve(d_L, (int)N, d_R, res, nrhs, mode, s));
   } else {
-    HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_z.p, res, nrhs, mode, s));
+    // the solves are out of place: from a copy of R into the result, and, for
+    // C^-1 R, through a second workspace
+    HIPCHK(ctx->dn_z.reserve(n));
+    HIPCHK(ctx->dn_inv.reserve(tri_inverse_size(N)));
+    if (!dev || mode == 2) HIPCHK(ctx->dn_x.reserve(n));
+    if (!dev) res = ctx->dn_x.p;
+    HIPCHK(hipMemcpyAsync(ctx->dn_z.p, R, n * sizeof(double), dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
+    HIPCHK(launch_tri_inverse(d_L, N, ctx->dn_inv.p, s));
+    if (mode == 2) {
+      HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_z.p, ctx->dn_x.p, nrhs, 0, s));
+      res = dev ? X : ctx->dn_z.p;
+      HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_x.p, res, nrhs, 1, s));
+    } else {
+      HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_z.p, res, nrhs, mode, s));
+    }
   }
   if (!dev) {
     HIPCHK(hipMemcpyAsync(X, res, n * sizeof(double), hipMemcpyDeviceToHost, s));

@@ -151,29 +151,26 @@ __device__ void tri64_merge(const double* S, double* V) {
   __syncthreads();
 }
 
-// The same with nothing in V: wave w substitutes its 16 x 16 diagonal block
-// (column i in lane i) first.
+// The same with nothing in V: wave w inverts its 16 x 16 diagonal block first,
+// lane i solving x L^T = e_i by columns: a step chains a product and an FMA (by
+// rows it was a dot product, 2.9 us a block).
 __device__ void tri64_inverse(const double* S, double* V) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  {
-    const int o = 16 * wave, i = lane & 15;
-    const double* L = S + o * LS + o;
-    double x[16];
-    const double rd = 1.0 / L[i * LS + i];
+  const int o = 16 * wave, i = lane & 15;
+  const double* L = S + o * LS + o;
+  const double rd = 1.0 / L[i * LS + i];
+  double a[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      double s0 = i == r ? 1.0 : 0.0, s1 = 0.0;
+  for (int c = 0; c < 16; ++c) a[c] = i == c ? 1.0 : 0.0;
 #pragma unroll
-      for (int t = 0; t < r; ++t) {
-        if (t & 1) s1 -= L[r * LS + t] * x[t];
-        else s0 -= L[r * LS + t] * x[t];
-      }
-      x[r] = (s0 + s1) * lane_d(rd, r);
-    }
-    if (lane < 16) {
+  for (int j = 0; j < 16; ++j) {
+    a[j] *= lane_d(rd, j);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) V[(o + r) * LS + o + i] = x[r];
-    }
+    for (int c = j + 1; c < 16; ++c) a[c] -= a[j] * L[c * LS + j];
+  }
+  if (lane < 16) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) V[(o + j) * LS + o + i] = a[j];
   }
   tri64_merge(S, V);
 }
@@ -529,6 +526,39 @@ __global__ __launch_bounds__(256, 2) void k_solve_update(const double* __restric
   }
 }
 
+// Solves with at most 64 rows, all modes in one launch: a wave takes a
+// right-hand side, lane i row i, by substitution (10 rows, L^-T L^-1: 64 us a call with
+// three launches, 56 with one).  X may be R.
+__global__ __launch_bounds__(256) void k_solve_small(const double* __restrict__ L, int N, const double* R, double* X,
+                                                     int64_t B, int mode) {
+  __shared__ double S[DB * LS];
+  const int lane = threadIdx.x & 63;
+  for (int e = threadIdx.x; e < DB * DB; e += 256) {
+    const int r = e / DB, c = e - r * DB;
+    if (r < N && c <= r) S[r * LS + c] = L[(size_t)r * N + c];
+  }
+  __syncthreads();
+  const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (b >= B) return;
+  const double rd = lane < N ? 1.0 / S[lane * LS + lane] : 0.0;
+  double r = lane < N ? R[(size_t)b * N + lane] : 0.0;
+  if (mode != 1) {
+    for (int k = 0; k < N; ++k) {
+      const double x = lane_d(r, k) * lane_d(rd, k);
+      if (lane > k && lane < N) r -= S[lane * LS + k] * x;
+      else if (lane == k) r = x;
+    }
+  }
+  if (mode != 0) {
+    for (int k = N - 1; k >= 0; --k) {
+      const double x = lane_d(r, k) * lane_d(rd, k);
+      if (lane < k) r -= S[k * LS + lane] * x;
+      else if (lane == k) r = x;
+    }
+  }
+  if (lane < N) X[(size_t)b * N + lane] = r;
+}
+
 // r = data - mu (FP64), [B][N]
 __global__ void k_resid(const float* __restrict__ mu, const double* __restrict__ data, int64_t N, int64_t B,
                         double* __restrict__ r) {
@@ -591,7 +621,7 @@ hipError_t launch_tri_inverse(const double* L, int64_t N, double* inv, hipStream
   if (N < 1) return hipErrorInvalidValue;
   // whole SB blocks: the merges of a partial last block read identity rows
   const int64_t ns = (N + SB - 1) / SB;
-  hipLaunchKernelGGL(k_tri_inv64, dim3((unsigned)(ns * (SB / DB))), dim3(256), 0, s, L, N, inv);
+  hipLaunchKernelGGL(k_tri_inv64, dim3((unsigned)(N <= DB ? 1 : ns * (SB / DB))), dim3(256), 0, s, L, N, inv);
   static_assert(SB == 512, "the merges go 64 -> 128 -> 256 -> 512");
   if (N > 64) hipLaunchKernelGGL((k_tri_merge<64, 2>), dim3((unsigned)(ns * 4), 2), dim3(256), 0, s, L, N, inv);
   if (N > 128) hipLaunchKernelGGL((k_tri_merge<128, 2>), dim3((unsigned)(ns * 2), 4), dim3(512), 0, s, L, N, inv);
@@ -621,6 +651,12 @@ hipError_t launch_dense_solve(const double* L, int64_t N, const double* inv, dou
   if (N < 1 || B < 1 || R == X) return hipErrorInvalidValue;
   if (transpose) solve_pass<true>(L, N, inv, R, X, B, s);
   else solve_pass<false>(L, N, inv, R, X, B, s);
+  return hipGetLastError();
+}
+
+hipError_t launch_small_solve(const double* L, int N, const double* R, double* X, int64_t B, int mode, hipStream_t s) {
+  if (N < 1 || N > DB || B < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_solve_small, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, L, N, R, X, B, mode);
   return hipGetLastError();
 }
 

@@ -379,6 +379,8 @@ hipError_t launch_dense_cholesky(double* A, int64_t N, double* inv, double* dlog
 hipError_t launch_tri_inverse(const double* L, int64_t N, double* inv, hipStream_t s);
 hipError_t launch_dense_solve(const double* L, int64_t N, const double* inv, double* R, double* X, int64_t B,
                               int transpose, hipStream_t s);
+// N <= DENSE_PANEL: X = L^-1 R (mode 0), L^-T R (1) or L^-T L^-1 R (2)
+hipError_t launch_small_solve(const double* L, int N, const double* R, double* X, int64_t B, int mode, hipStream_t s);
 hipError_t launch_dense_loglike(const float* mu, int64_t B, int64_t N, const double* data, const double* L, double c0,
                                 const double* inv, double* Z, double* X, double* loglike, float* dmu, hipStream_t s);
 // out[o] = sum of the forward partials of the launch's live slices, for o in

@@ -32,3 +32,18 @@ def test_solves_around_blocks(n):
         np.testing.assert_allclose(ll, -0.5 * (d ** 2).sum(0), rtol=1e-10)
         x = np.linalg.solve(ref.T, d).T
         np.testing.assert_allclose(dmu, x, rtol=0, atol=2.0 ** -23 * np.abs(x).max())
+
+
+@pytest.mark.parametrize("n", [1, 2, 33, 63, 64, 65])
+@pytest.mark.parametrize("nrhs", [1, 4, 5, 130])
+def test_solves_of_few_rows(n, nrhs):
+    ctx = default_context()
+    ref = np.linalg.cholesky(spd(n, n))
+    Lr = torch.as_tensor(ref, device="cuda")
+    R = np.random.default_rng(n).normal(size=(nrhs, n))
+    z = np.linalg.solve(ref, R.T)
+    for mode, want in ((0, z.T), (1, np.linalg.solve(ref.T, R.T).T), (2, np.linalg.solve(ref.T, z).T)):
+        atol = 1e-10 * max(1.0, np.abs(want).max())
+        np.testing.assert_allclose(ctx.dense_solve(Lr, R, mode=mode), want, rtol=0, atol=atol)
+        Rd = torch.as_tensor(R, device="cuda")  # solved in place
+        np.testing.assert_allclose(ctx.dense_solve(Lr, Rd, mode=mode).cpu().numpy(), want, rtol=0, atol=atol)
