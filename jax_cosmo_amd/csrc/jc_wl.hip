@@ -282,14 +282,15 @@ static hipError_t wl_launch(const WLArgs& a, int num_cu, hipStream_t s) {
 // split the inner nodes.  Measured on 256 CUs, n_z 512 (8 node blocks), 5 bins,
 // us for 1 / 2 / 4 / 8 cosmologies a block: 8.3 / 8.8 / 10.5 / 17 at 1
 // cosmology, 17 / 11.3 / 13.5 / 22 at 64, 50 / 31 / 22 / 26 at 256, 93 / 55 / 37 /
-// 38 at 512, 177 / 100 / 66 / 59 at 1024.  Seven directions, (1, 8 waves) / (1, 4)
+// 38 at 512, 177 / 100 / 66 / 59 at 1024.  A batch of 520 takes 204 us
+// with 4 and 208 with 8, one of 700 235 and 232.  Seven directions, (1, 8 waves) / (1, 4)
 // / (2, 4): 14 / 23 / 30 at 1, 26 / 31 / 35 at 64, 44 / 44 / 45 at 128, 80 / 78 / 75
 // at 256, 312 / 289 / 258 at 1024.  ctile (ND = 0): 0 = by this rule.
 template <int NW>
 static hipError_t wl_launch_nw(int nd, int ctile, const WLArgs& a, int num_cu, hipStream_t s) {
   const int64_t blocks = (int64_t)((a.Na - 1 + WL_M - 1) / WL_M) * a.B;  // at one cosmology each
   if (nd == 0) {
-    if (ctile == 0) ctile = blocks <= num_cu ? 1 : (blocks <= 2 * num_cu ? 2 : (blocks <= 16 * num_cu ? 4 : 8));
+    if (ctile == 0) ctile = blocks <= num_cu ? 1 : (blocks <= 2 * num_cu ? 2 : (blocks <= 20 * num_cu ? 4 : 8));
     switch (ctile) {
       case 1: return wl_launch<0, 1, NW, 8>(a, num_cu, s);
       case 2: return wl_launch<0, 2, NW, 8>(a, num_cu, s);
