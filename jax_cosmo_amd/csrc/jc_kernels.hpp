@@ -299,17 +299,12 @@ __host__ __device__ inline int ragged_slices(int tiles, int waves, int Na, int m
   return s < 1 ? 1 : s;
 }
 
-// Blocks that hold every unit of `tiles` live tiles or fewer: ragged_slices
-// rounds 2048 / (tiles x waves) up, so tiles x slices <= 2048 / waves + tiles; an XCD
-// holds up to one tile more than an eighth.
+// Blocks that hold every unit of `tiles` live tiles or fewer.  An XCD has at most
+// t / 8 + 1 of t tiles and ragged_slices gives each at most 2048 / (t waves) + 1
+// slices and at most max_slices, so its units are at most 256 / waves + t / 8 +
+// max_slices + 1.
 inline int ragged_fwd_blocks(int tiles, int waves, int max_slices) {
-  const int per_xcd = (tiles + 7) / 8;
-  int most = 0;  // units of the fullest XCD
-  for (int t = 1; t <= tiles; ++t) {
-    const int s = (2048 + t * waves - 1) / (t * waves), n = (t + 7) / 8 * (s < max_slices ? s : max_slices);
-    most = n > most ? n : most;
-  }
-  return 8 * (most > per_xcd ? most : per_xcd);
+  return 8 * ((256 + waves - 1) / waves + (tiles + 7) / 8 + max_slices + 1);
 }
 
 // launchers (defined next to their kernels)
