@@ -12,6 +12,7 @@ import torch
 from ._native import default_context
 from .angular_cl import _device_ell
 
+MAX_COLUMNS = 1 << 30  # (cosmology, ell) columns of a launch
 GRAD_INDEX = (0, 1, 2, 3, 4, 6, 7)  # positions of theta in the 8-parameter vector
 
 
@@ -98,7 +99,11 @@ def angular_cl_jacobian(cosmo_params, ell, probes, n_z=512, transfer_fn=None, no
     set_id = dctx.tracer_set(tracer_entries(probes))
     P = _n_cls(probes)
     cp = np.asarray(cosmo_params, dtype=np.float64).reshape(-1, 8)
-    return dctx.angular_cl_jacobian(cp, set_id, np.asarray(ell, dtype=np.float64), n_z, P)
+    ell = np.asarray(ell, dtype=np.float64)
+    if 7 * ell.size > MAX_COLUMNS:  # one cosmology's seven rows exceed a launch: a direction at a time
+        return np.stack([dctx.angular_cl_jvp(cp, np.broadcast_to(e, (len(cp), 7)), set_id, ell, n_z, P)[1]
+                         for e in np.eye(7)], axis=-1)
+    return dctx.angular_cl_jacobian(cp, set_id, ell, n_z, P)
 
 
 def fisher_matrix(cosmo_params, ell, probes, C, n_z=512, transfer_fn=None, nonlinear_fn=None, gamma=None):

@@ -35,3 +35,15 @@ def test_jacobian_against_directional_derivatives(B, wl, nc, n_ell, n_z):
         dot = ctx.angular_cl_jvp(params, t, sid, ell, n_z, P)[1]
         scale = np.abs(dot).max(axis=2, keepdims=True)
         assert (np.abs(jac[..., d] - dot) <= 1e-5 * scale).all()
+
+
+def test_a_direction_at_a_time(monkeypatch):
+    """More multipoles than seven rows of a launch hold: the same Jacobian by
+    single directions."""
+    ell = np.geomspace(20.0, 2000.0, 9)
+    probes = [jc.probes.WeakLensing([jc.redshift.smail_nz(1.0, 2.0, 0.7)])]
+    ref = jag.angular_cl_jacobian(PARAMS, ell, probes, n_z=62)
+    monkeypatch.setattr(jag, "MAX_COLUMNS", 62)
+    jac = jag.angular_cl_jacobian(PARAMS, ell, probes, n_z=62)
+    assert jac.shape == ref.shape and jac.dtype == ref.dtype
+    assert (np.abs(jac - ref) <= 1e-5 * np.abs(ref).max(axis=2, keepdims=True)).all()
