@@ -733,7 +733,7 @@ def main():
         "host_buffers": host_batch,
         "rel_err_vs_fp64_oracle": {"max": max(errs) if errs else None, "samples": len(errs)},
         "tiles": {"waves_per_block": tiles_c3[0], "wl_ctile": tiles_c3[1], "tuned_now": tuned is not None,
-                  "note": "0 = library default (waves 2 if >= 2048 blocks else 4; wl_ctile 4 if B >= 192 else 1)"},
+                  "note": "0 = the library's launch rules"},
         "served": served,
         "batch_vs_served_batch_shaped": (value / served["batch_shaped"]["C_ell_per_s"]) if served else None,
         "likelihood_gradient": grad,
