@@ -332,10 +332,16 @@ int build_grid(jc_ctx* ctx, TracerSet* ts, int N, GridTables** out) {
     // rows padded with zeros to the kernel's bin count (5 or NWL_MAX)
     const int nw_rows = wg->nw <= 5 ? 5 : NWL_MAX;
     std::vector<float> Nw((size_t)nw_rows * NWL_J * Na, 0.0f);
-    // n(z') of every bin at every inner node, [j][m]
-    std::vector<double> zin((size_t)NWL_J * Na);
-    for (int m = 0; m < Na; ++m)
-      for (int j = 0; j < NWL_J; ++j) zin[(size_t)j * Na + m] = linspace_at(z[m], zmax, NWL_J, j);
+    // n(z') of every bin at every inner node, [j][m].  The a-grid reaches the
+    // largest zmax of all tracers; past the probe's own, where the inner grid would
+    // run backwards and the clip of chi' - chi makes the integrand zero
+    // (probes.py:51), it is the point z itself with zero weights: the kernel's
+    // unclipped loop takes chi' >= chi for granted.
+    std::vector<double> zin((size_t)NWL_J * Na), zend(Na);
+    for (int m = 0; m < Na; ++m) {
+      zend[m] = std::max(zmax, z[m]);
+      for (int j = 0; j < NWL_J; ++j) zin[(size_t)j * Na + m] = linspace_at(z[m], zend[m], NWL_J, j);
+    }
     std::vector<std::vector<double>> pzin(wg->nw);
     for (int q = 0; q < wg->nw; ++q) {
       if (ts->tr[idx[q]].nz_kind == JC_NZ_DELTA) continue;
@@ -343,9 +349,9 @@ int build_grid(jc_ctx* ctx, TracerSet* ts, int N, GridTables** out) {
       if (rc) return rc;
     }
     for (int m = 0; m < Na; ++m) {
-      const double dxm = (zmax - z[m]) / (NWL_J - 1);
+      const double dxm = (zend[m] - z[m]) / (NWL_J - 1);  // 0 past zmax
       for (int j = 0; j < NWL_J; ++j) {
-        const double zp = linspace_at(z[m], zmax, NWL_J, j);
+        const double zp = zin[(size_t)j * Na + m];
         const double ap = 1.0 / (1.0 + zp);  // z2a, utils.py:2-4
         const int seg = interp_segment(ap, ctx->atab_chi_h);
         L[(size_t)j * Na + m] = (uint8_t)seg;

@@ -13,7 +13,9 @@
 // node before it writes that zero.
 //
 // Nodes with chi_m >= 1 (all but the last ones of a fine grid; wave-uniform)
-// have chi' >= chi_m >= 1, so neither clip acts: f = (chi' - chi_m) / chi', and
+// have chi' >= chi_m >= 1 (the resident tables put no inner node nearer than its
+// outer one: past the probe's zmax all of them are the outer node, with zero
+// weights), so neither clip acts: f = (chi' - chi_m) / chi', and
 // its derivatives are ((chi_m / chi') dchi' - dchi_m) / chi', two FMAs a
 // direction, with the 1 / chi' moved to the weights.  ND = 0: 8 instructions and
 // a reciprocal a point with 5 bins; bound by the resident tables' path through
