@@ -8,7 +8,7 @@
 //
 // Cholesky C = L L^T, right-looking in 64-column panels, two launches a panel:
 //   k_chol_panel  the panel below its 64 x 64 diagonal block, L21 = A21 L11^-T,
-//                 as a product with the block's inverse;
+//                 as a product with the block's inverse and one correction;
 //   k_chol_syrk   the trailing lower triangle, A22 -= L21 L21^T, 64 x 64 tiles;
 //                 its first block then factors and inverts the next panel's
 //                 diagonal block (chol64) beside the other tiles.
@@ -264,27 +264,52 @@ __global__ __launch_bounds__(256, 2) void k_chol_first(double* __restrict__ A, i
 }
 
 // rows i >= k0 + 64: x = a L11^-T, 16 rows a wave (which reads its rows' 64
-// columns before it writes them)
+// columns before it writes them).  The product with the block's inverse alone has a
+// residual that grows with the block's condition number and goes into every
+// later panel (covariances of condition 1e12 met non-positive pivots); one
+// correction, x += (a - x L11^T) L11^-T, brings it back to that of a substitution.
+// Products are taken transposed, with the rows of L11 dealt to the operand's lanes
+// so that a result comes back as the 4 consecutive columns per lane in which it is
+// used and stored.
 __global__ __launch_bounds__(256, 2) void k_chol_panel(double* __restrict__ A, int64_t N, int64_t k0,
                                                      const double* __restrict__ inv) {
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int64_t r0 = k0 + DB + ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
   if (r0 >= N) return;
-  const double* row = A + (size_t)min(r0 + i, N - 1) * N + k0 + 4 * g;
-  d4 a[4], acc[4];
+  const int p = 4 * (i & 3) + (i >> 2);  // result (g, r) is then row 4 g + r of a 16 x 16 block
+  double* const row = A + (size_t)min(r0 + i, N - 1) * N + k0 + 4 * g;
+  d4 a[4], x[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) a[s] = frag_row(row + 16 * s, 4);
+  auto inverse = [&](const d4* v, int c) {
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    acc[c] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int s = 0; s <= c; ++s) mma16(frag_row(inv + (16 * c + p) * DB + 16 * s + 4 * g, 4), v[s], acc);
+    return acc;
+  };
 #pragma unroll
-    for (int s = 0; s <= c; ++s) mma16(a[s], frag_row(inv + (16 * c + i) * DB + 16 * s + 4 * g, 4), acc[c]);
+  for (int c = 0; c < 4; ++c) x[c] = inverse(a, c);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {  // the residual, in place of a
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s <= c; ++s) {
+      d4 l = frag_row(A + (size_t)(k0 + 16 * c + p) * N + k0 + 16 * s + 4 * g, 4);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (s == c && 4 * g + q > p) l[q] = 0.0;  // above L11's diagonal lies whatever the caller had
+      mma16(l, x[s], acc);
+    }
+    a[c] -= acc;
   }
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < 4; ++c) x[c] += inverse(a, c);
+  if (r0 + i >= N) return;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (r0 + g + 4 * r < N) A[(size_t)(r0 + g + 4 * r) * N + k0 + 16 * c + i] = acc[c][r];
+  for (int c = 0; c < 4; ++c) {
+    *reinterpret_cast<d2u*>(row + 16 * c) = d2u{x[c][0], x[c][1]};
+    *reinterpret_cast<d2u*>(row + 16 * c + 2) = d2u{x[c][2], x[c][3]};
+  }
 }
 
 // trailing update of the lower triangle from row/column r0 = k0 + 64: tile
