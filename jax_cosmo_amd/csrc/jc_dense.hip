@@ -539,8 +539,14 @@ __global__ __launch_bounds__(256, 2) void k_solve_diag(const double* __restrict_
   for (int q = 0; q < 4; ++q) red[wave][q][lane] = acc[q];
   __syncthreads();
   const int64_t b = b0 + g + 4 * wave;  // wave w adds and writes register w
-  if (row < nb && b < B)
-    X[(size_t)b * N + k0 + row] = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
+  if (row >= nb || b >= B) return;
+  double s = ((red[0][wave][lane] + red[1][wave][lane]) + red[2][wave][lane]) + red[3][wave][lane];
+  if (s != s) {  // something not finite, perhaps only against a zero on the triangle's other side
+    const double* rb = R + (size_t)b * N + k0;
+    s = 0.0;
+    for (int k = TR ? row : 0; k < (TR ? nb : row + 1); ++k) s += rb[k] * V[TR ? (size_t)k * SB + row : (size_t)row * SB + k];
+  }
+  X[(size_t)b * N + k0 + row] = s;
 }
 
 // k_solve_update: removes the solved block from the rows still to come
