@@ -229,6 +229,14 @@ int jc_dense_cholesky(jc_ctx* ctx, const double* cov, int64_t N, double* L, doub
 int jc_dense_solve(jc_ctx* ctx, const double* L, int64_t N, const double* R, int64_t nrhs, int32_t mode,
                    double* X, int32_t flags);
 
+/* The same on device pointers, asynchronous, with n_work doubles of device memory
+ * of the caller's (at least jc_dense_solve_workspace's answer; may be NULL where
+ * that is 0): larger blocks, fewer launches.  Neither call uses memory of the
+ * context for device pointers. */
+int jc_dense_solve_workspace(int64_t N, int64_t nrhs, int32_t mode, int64_t* doubles);
+int jc_dense_solve_work(jc_ctx* ctx, const double* L, int64_t N, const double* R, int64_t nrhs, int32_t mode,
+                        double* X, double* work, int64_t n_work);
+
 /* loglike[b] = -1/2 (data - mu_b)^T C^-1 (data - mu_b) + c0 for B means
  * mu [B][N] float32, with C given by its factor L (jc_dense_cholesky): the
  * quadratic form as |L^-1 (data - mu_b)|^2 (the value of both inverse

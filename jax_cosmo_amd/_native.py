@@ -24,7 +24,7 @@ EXPORTS = (
     "jc_angular_cl_noalloc", "jc_angular_cl_jvp", "jc_angular_cl_jacobian",
     "jc_angular_cl_vjp", "jc_matter_power", "jc_background", "jc_background_ex", "jc_set_growth", "jc_set_tiles", "jc_get_tiles", "jc_set_tables_variant",
     "jc_set_forward_options", "jc_set_models", "jc_sparse_inv", "jc_gaussian_loglike", "jc_gaussian_loglike_cov", "jc_gaussian_loglike_grad",
-    "jc_dense_cholesky", "jc_dense_solve", "jc_gaussian_loglike_dense", "jc_gaussian_loglike_grad_dense",
+    "jc_dense_cholesky", "jc_dense_solve", "jc_dense_solve_workspace", "jc_dense_solve_work", "jc_gaussian_loglike_dense", "jc_gaussian_loglike_grad_dense",
     "jc_sigma8_norm", "jc_debug_tables", "jc_profile_enable", "jc_profile_select", "jc_profile_read", "jc_last_error", "jc_version",
 )
 KERNELS = ("tables", "wl", "limber", "ehtab")
@@ -126,6 +126,8 @@ def load_library(path=LIB_PATH):
                                          _I32],
             "jc_dense_cholesky": [_P, _P, _I64, _P, _P, _I32],
             "jc_dense_solve": [_P, _P, _I64, _P, _I64, _I32, _P, _I32],
+            "jc_dense_solve_workspace": [_I64, _I64, _I32, _P],
+            "jc_dense_solve_work": [_P, _P, _I64, _P, _I64, _I32, _P, _P, _I64],
             "jc_gaussian_loglike_dense": [_P, _P, _I64, _I64, _P, _P, ctypes.c_double, _P, _P, _I32],
             "jc_gaussian_loglike_grad_dense": [_P, _P, _I64, _I64, _P, _I64, _I64, _P, _P, ctypes.c_double, _P, _P,
                                                _I32],
@@ -594,11 +596,15 @@ class _Likelihood:
         X = R.to(device=L.device, dtype=torch.float64).contiguous() if on_dev else \
             torch.as_tensor(_f64(R).reshape(-1, N)).to(L.device)
         X = X.reshape(-1, N)
+        # the workspace belongs to this call and its stream: solves on other streams have their own
+        n_work = ctypes.c_int64()
+        check(self.lib.jc_dense_solve_workspace(N, X.shape[0], int(mode), ctypes.byref(n_work)))
+        work = torch.empty(n_work.value, dtype=torch.float64, device=L.device)
         with self._lock:
             self.set_stream(torch.cuda.current_stream().cuda_stream)
             try:
-                check(self.lib.jc_dense_solve(self.handle, _P(L.data_ptr()), N, _P(X.data_ptr()), X.shape[0], int(mode),
-                                              _P(X.data_ptr()), JC_DEVICE_PTRS))
+                check(self.lib.jc_dense_solve_work(self.handle, _P(L.data_ptr()), N, _P(X.data_ptr()), X.shape[0],
+                                                   int(mode), _P(X.data_ptr()), _P(work.data_ptr()), n_work.value))
             finally:
                 self.reset_stream()
         return X if on_dev else X.cpu().numpy()

@@ -119,6 +119,9 @@ static void device_checks(jc_ctx* ctx) {
     for (int j = 0; j < N; ++j) C[(size_t)i * N + j] = (i == j ? N : 0.0) + 1.0 / (1.0 + i + j);
   CHECK(jc_dense_cholesky(ctx, C.data(), N, Lf.data(), &logdet, 0) == JC_OK, "cholesky");
   CHECK(jc_dense_solve(ctx, Lf.data(), N, R.data(), 2, 2, X.data(), 0) == JC_OK, "dense solve");
+  int64_t nw = -1;
+  CHECK(jc_dense_solve_workspace(N, 2, 2, &nw) == JC_OK && nw >= 0, "dense solve workspace");
+  CHECK(jc_dense_solve_workspace(0, 2, 2, &nw) == JC_E_ARG, "workspace of no rows");
   // background and power
   std::vector<double> a(40), k(40), chi(40), gr(40), rate(40), fk(40), pl(40), pn(40);
   for (int i = 0; i < 40; ++i) {

@@ -1279,45 +1279,84 @@ int jc_dense_cholesky(jc_ctx* ctx, const double* cov, int64_t N, double* L, doub
   return JC_OK;
 }
 
+static int check_dense_solve(int64_t N, int64_t nrhs, int32_t mode) {
+  if (N < 1 || N > 65535 || nrhs < 1) return fail(JC_E_ARG, "N in 1..65535 and nrhs >= 1 required");
+  if (mode < 0 || mode > 2) return fail(JC_E_ARG, "mode must be 0 (L^-1), 1 (L^-T) or 2 (C^-1)");
+  return JC_OK;
+}
+
+// N > DENSE_PANEL, on the device: inv as of launch_tri_inverse; z holds R and is
+// overwritten; x (C^-1 R only) is a second workspace; the result goes to res, which
+// may be z for C^-1 R
+static hipError_t dense_solve_blocks(const double* L, int64_t N, int32_t mode, double* inv, double* z, double* x,
+                                     double* res, int64_t nrhs, hipStream_t s) {
+  hipError_t e = launch_tri_inverse(L, N, inv, s);
+  if (e != hipSuccess) return e;
+  if (mode != 2) return launch_dense_solve(L, N, inv, z, res, nrhs, mode, s);
+  if ((e = launch_dense_solve(L, N, inv, z, x, nrhs, 0, s)) != hipSuccess) return e;
+  return launch_dense_solve(L, N, inv, x, res, nrhs, 1, s);
+}
+
+// Device pointers: the call is asynchronous and takes no memory of the context, so
+// that solves on several streams do not meet and the call can be captured.  It works
+// in X then, by blocks of 64 rows; with the caller's workspace (jc_dense_solve_work)
+// by blocks of 512.
 int jc_dense_solve(jc_ctx* ctx, const double* L, int64_t N, const double* R, int64_t nrhs, int32_t mode,
                    double* X, int32_t flags) {
   if (!ctx || !L || !R || !X) return fail(JC_E_ARG, "null argument");
-  if (N < 1 || N > 65535 || nrhs < 1) return fail(JC_E_ARG, "N in 1..65535 and nrhs >= 1 required");
-  if (mode < 0 || mode > 2) return fail(JC_E_ARG, "mode must be 0 (L^-1), 1 (L^-T) or 2 (C^-1)");
+  int rc = check_dense_solve(N, nrhs, mode);
+  if (rc) return rc;
   HIPCHK(hipSetDevice(ctx->device));
-  const bool dev = (flags & JC_DEVICE_PTRS) != 0;
   hipStream_t s = ctx->stream;
   const size_t n = (size_t)nrhs * N;
-  const double* d_L = nullptr;
-  int rc = to_device(ctx, ctx->dn_mat, L, (size_t)N * N, dev, &d_L);
-  if (rc) return rc;
-  double* res = X;
+  if (flags & JC_DEVICE_PTRS) {
+    if (N <= DENSE_PANEL) {
+      HIPCHK(launch_small_solve(L, (int)N, R, X, nrhs, mode, s));
+    } else {
+      if (X != R) HIPCHK(hipMemcpyAsync(X, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+      HIPCHK(launch_dense_solve_in_place(L, N, X, nrhs, mode, s));
+    }
+    return JC_OK;
+  }
+  const double *d_L = nullptr, *d_R = nullptr;
+  if ((rc = to_device(ctx, ctx->dn_mat, L, (size_t)N * N, false, &d_L))) return rc;
+  if ((rc = to_device(ctx, ctx->dn_z, R, n, false, &d_R))) return rc;
+  double* res = ctx->dn_z.p;
   if (N <= DENSE_PANEL) {
-    const double* d_R = nullptr;
-    if ((rc = to_device(ctx, ctx->dn_z, R, n, dev, &d_R))) return rc;
-    if (!dev) res = ctx->dn_z.p;
     HIPCHK(launch_small_solve(d_L, (int)N, d_R, res, nrhs, mode, s));
   } else {
-    // the solves are out of place: from a copy of R into the result, and, for
-    // C^-1 R, through a second workspace
-    HIPCHK(ctx->dn_z.reserve(n));
     HIPCHK(ctx->dn_inv.reserve(tri_inverse_size(N)));
-    if (!dev || mode == 2) HIPCHK(ctx->dn_x.reserve(n));
-    if (!dev) res = ctx->dn_x.p;
-    HIPCHK(hipMemcpyAsync(ctx->dn_z.p, R, n * sizeof(double), dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-    HIPCHK(launch_tri_inverse(d_L, N, ctx->dn_inv.p, s));
-    if (mode == 2) {
-      HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_z.p, ctx->dn_x.p, nrhs, 0, s));
-      res = dev ? X : ctx->dn_z.p;
-      HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_x.p, res, nrhs, 1, s));
-    } else {
-      HIPCHK(launch_dense_solve(d_L, N, ctx->dn_inv.p, ctx->dn_z.p, res, nrhs, mode, s));
-    }
+    HIPCHK(ctx->dn_x.reserve(n));
+    if (mode != 2) res = ctx->dn_x.p;
+    HIPCHK(dense_solve_blocks(d_L, N, mode, ctx->dn_inv.p, ctx->dn_z.p, ctx->dn_x.p, res, nrhs, s));
   }
-  if (!dev) {
-    HIPCHK(hipMemcpyAsync(X, res, n * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-  }
+  HIPCHK(hipMemcpyAsync(X, res, n * sizeof(double), hipMemcpyDeviceToHost, s));
+  HIPCHK(hipStreamSynchronize(s));
+  return JC_OK;
+}
+
+int jc_dense_solve_workspace(int64_t N, int64_t nrhs, int32_t mode, int64_t* doubles) {
+  if (!doubles) return fail(JC_E_ARG, "null argument");
+  const int rc = check_dense_solve(N, nrhs, mode);
+  if (rc) return rc;
+  *doubles = N <= DENSE_PANEL ? 0 : (int64_t)tri_inverse_size(N) + (mode == 2 ? 2 : 1) * nrhs * N;
+  return JC_OK;
+}
+
+int jc_dense_solve_work(jc_ctx* ctx, const double* L, int64_t N, const double* R, int64_t nrhs, int32_t mode,
+                        double* X, double* work, int64_t n_work) {
+  int64_t need = 0;
+  int rc = jc_dense_solve_workspace(N, nrhs, mode, &need);
+  if (rc) return rc;
+  if (need == 0) return jc_dense_solve(ctx, L, N, R, nrhs, mode, X, JC_DEVICE_PTRS);
+  if (!ctx || !L || !R || !X || !work) return fail(JC_E_ARG, "null argument");
+  if (n_work < need) return fail(JC_E_ARG, "the solve needs a workspace of %lld doubles", (long long)need);
+  HIPCHK(hipSetDevice(ctx->device));
+  hipStream_t s = ctx->stream;
+  const size_t n = (size_t)nrhs * N;
+  double* z = work + tri_inverse_size(N);
+  HIPCHK(hipMemcpyAsync(z, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+  HIPCHK(dense_solve_blocks(L, N, mode, work, z, z + n, X, nrhs, s));
   return JC_OK;
 }
 

@@ -549,21 +549,21 @@ __global__ __launch_bounds__(256, 2) void k_solve_diag(const double* __restrict_
   X[(size_t)b * N + k0 + row] = s;
 }
 
-// k_solve_update: removes the solved block from the rows still to come
+// k_solve_update: removes the solved block of BS rows from the rows still to come
 // (forward: after it, r_i -= sum_t L[i][k0+t] x_{k0+t}; TR: before it,
 // r_i -= sum_t L[k0+t][i] x_{k0+t}), 32 rows x 16 WB right-hand sides a
 // workgroup.  Workgroups are numbered so that one XCD's L2 holds the same rows of
-// L for all right-hand sides.
-template <bool TR, int WB>
+// L for all right-hand sides.  X may be R (the rows read and written are others).
+template <bool TR, int WB, int BS>
 __global__ __launch_bounds__(256, 2) void k_solve_update(const double* __restrict__ L, int64_t N, int64_t k0, int64_t B,
                                                       int gy, const double* __restrict__ X, double* __restrict__ R) {
   __shared__ double red[4][2 * WB][4][64];
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nb = (int)min((int64_t)SB, N - k0);
+  const int nb = (int)min((int64_t)BS, N - k0);
   const int n = gridDim.x, q8 = n >> 3, r8 = n & 7, xc = blockIdx.x & 7;  // block b runs on XCD b % 8
   const int id = xc * q8 + min(xc, r8) + (blockIdx.x >> 3);
-  const int64_t row0 = (TR ? 0 : k0 + SB) + (int64_t)(id / gy) * 32, row_end = TR ? k0 : N;
+  const int64_t row0 = (TR ? 0 : k0 + BS) + (int64_t)(id / gy) * 32, row_end = TR ? k0 : N;
   const int64_t b0 = (int64_t)(id % gy) * (16 * WB);
   const double* x[WB];
   int64_t rw[2];
@@ -593,8 +593,8 @@ __global__ __launch_bounds__(256, 2) void k_solve_update(const double* __restric
 #pragma unroll
       for (int c = 0; c < 2; ++c) mma16(xv[q][a], lv[q][c], acc[a][c]);
   };
-  if (nb == SB)
-    pipelined<D>(SB / 64, [&](int s, int q) { load(s, q, 4); }, use);
+  if (nb == BS)
+    pipelined<D>(BS / 64, [&](int s, int q) { load(s, q, 4); }, use);
   else
     pipelined<D>((nb - 16 * wave + 63) / 64,
                  [&](int s, int q) { load(s, q, nb - (64 * s + 16 * wave) - 4 * g); }, use);
@@ -616,20 +616,20 @@ __global__ __launch_bounds__(256, 2) void k_solve_update(const double* __restric
 
 // Solves with at most 64 rows, all modes in one launch: a wave takes a
 // right-hand side, lane i row i, by substitution (10 rows, L^-T L^-1: 64 us a call with
-// three launches, 56 with one).  X may be R.
-__global__ __launch_bounds__(256) void k_solve_small(const double* __restrict__ L, int N, const double* R, double* X,
-                                                     int64_t B, int mode) {
+// three launches, 56 with one).  ld: row stride of all three.  X may be R.
+__global__ __launch_bounds__(256) void k_solve_small(const double* __restrict__ L, int N, int64_t ld, const double* R,
+                                                     double* X, int64_t B, int mode) {
   __shared__ double S[DB * LS];
   const int lane = threadIdx.x & 63;
   for (int e = threadIdx.x; e < DB * DB; e += 256) {
     const int r = e / DB, c = e - r * DB;
-    if (r < N && c <= r) S[r * LS + c] = L[(size_t)r * N + c];
+    if (r < N && c <= r) S[r * LS + c] = L[(size_t)r * ld + c];
   }
   __syncthreads();
   const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (b >= B) return;
   const double rd = lane < N ? 1.0 / S[lane * LS + lane] : 0.0;
-  double r = lane < N ? R[(size_t)b * N + lane] : 0.0;
+  double r = lane < N ? R[(size_t)b * ld + lane] : 0.0;
   if (mode != 1) {
     for (int k = 0; k < N; ++k) {
       const double x = lane_d(r, k) * lane_d(rd, k);
@@ -644,7 +644,7 @@ __global__ __launch_bounds__(256) void k_solve_small(const double* __restrict__ 
       else if (lane == k) r = x;
     }
   }
-  if (lane < N) X[(size_t)b * N + lane] = r;
+  if (lane < N) X[(size_t)b * ld + lane] = r;
 }
 
 // r = data - mu (FP64), [B][N]
@@ -717,20 +717,36 @@ hipError_t launch_tri_inverse(const double* L, int64_t N, double* inv, hipStream
   return hipGetLastError();
 }
 
+// (16 right-hand sides at most: half the products)
+template <bool TR, int BS>
+static void solve_update(const double* L, int64_t N, int64_t k0, int64_t B, const double* X, double* R, hipStream_t s) {
+  const int64_t rows = TR ? k0 : N - k0 - BS;
+  if (rows <= 0) return;
+  const int gy = (int)(B <= 16 ? 1 : (B + 31) / 32);
+  const dim3 gu((unsigned)((rows + 31) / 32 * gy));
+  if (B <= 16) hipLaunchKernelGGL((k_solve_update<TR, 1, BS>), gu, dim3(256), 0, s, L, N, k0, B, gy, X, R);
+  else hipLaunchKernelGGL((k_solve_update<TR, 2, BS>), gu, dim3(256), 0, s, L, N, k0, B, gy, X, R);
+}
+
 template <bool TR>
 static void solve_pass(const double* L, int64_t N, const double* inv, double* R, double* X, int64_t B, hipStream_t s) {
   const int64_t last = (N - 1) / SB * SB;
   for (int64_t step = 0; step <= last; step += SB) {
-    const int64_t k0 = TR ? last - step : step;
-    const int64_t nb = std::min<int64_t>(SB, N - k0), rows = TR ? k0 : N - k0 - SB;
+    const int64_t k0 = TR ? last - step : step, nb = std::min<int64_t>(SB, N - k0);
     const dim3 gd((unsigned)((B + 15) / 16), (unsigned)((nb + 15) / 16));
     hipLaunchKernelGGL((k_solve_diag<TR>), gd, dim3(256), 0, s, inv, N, k0, B, R, X);
-    if (rows <= 0) continue;
-    // (16 right-hand sides at most: half the products)
-    const int gy = (int)(B <= 16 ? 1 : (B + 31) / 32);
-    const dim3 gu((unsigned)((rows + 31) / 32 * gy));
-    if (B <= 16) hipLaunchKernelGGL((k_solve_update<TR, 1>), gu, dim3(256), 0, s, L, N, k0, B, gy, X, R);
-    else hipLaunchKernelGGL((k_solve_update<TR, 2>), gu, dim3(256), 0, s, L, N, k0, B, gy, X, R);
+    solve_update<TR, SB>(L, N, k0, B, X, R, s);
+  }
+}
+
+template <bool TR>
+static void solve_pass_in_place(const double* L, int64_t N, double* X, int64_t B, hipStream_t s) {
+  const int64_t last = (N - 1) / DB * DB;
+  for (int64_t step = 0; step <= last; step += DB) {
+    const int64_t k0 = TR ? last - step : step;
+    hipLaunchKernelGGL(k_solve_small, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, L + (size_t)k0 * N + k0,
+                       (int)std::min<int64_t>(DB, N - k0), N, X + k0, X + k0, B, TR ? 1 : 0);
+    solve_update<TR, DB>(L, N, k0, B, X, X, s);
   }
 }
 
@@ -744,7 +760,14 @@ hipError_t launch_dense_solve(const double* L, int64_t N, const double* inv, dou
 
 hipError_t launch_small_solve(const double* L, int N, const double* R, double* X, int64_t B, int mode, hipStream_t s) {
   if (N < 1 || N > DB || B < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_solve_small, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, L, N, R, X, B, mode);
+  hipLaunchKernelGGL(k_solve_small, dim3((unsigned)((B + 3) / 4)), dim3(256), 0, s, L, N, (int64_t)N, R, X, B, mode);
+  return hipGetLastError();
+}
+
+hipError_t launch_dense_solve_in_place(const double* L, int64_t N, double* X, int64_t B, int mode, hipStream_t s) {
+  if (N < 1 || B < 1) return hipErrorInvalidValue;
+  if (mode != 1) solve_pass_in_place<false>(L, N, X, B, s);
+  if (mode != 0) solve_pass_in_place<true>(L, N, X, B, s);
   return hipGetLastError();
 }
 

@@ -376,6 +376,9 @@ hipError_t launch_dense_solve(const double* L, int64_t N, const double* inv, dou
                               int transpose, hipStream_t s);
 // N <= DENSE_PANEL: X = L^-1 R (mode 0), L^-T R (1) or L^-T L^-1 R (2)
 hipError_t launch_small_solve(const double* L, int N, const double* R, double* X, int64_t B, int mode, hipStream_t s);
+// the same for any N, in X and without a workspace, by 64-row blocks: two launches a
+// block, an eighth of the rows a launch
+hipError_t launch_dense_solve_in_place(const double* L, int64_t N, double* X, int64_t B, int mode, hipStream_t s);
 hipError_t launch_dense_loglike(const float* mu, int64_t B, int64_t N, const double* data, const double* L, double c0,
                                 const double* inv, double* Z, double* X, double* loglike, float* dmu, hipStream_t s);
 // out[o] = sum of the forward partials of the launch's live slices, for o in
