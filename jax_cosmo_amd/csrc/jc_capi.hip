@@ -1263,8 +1263,8 @@ int jc_dense_cholesky(jc_ctx* ctx, const double* cov, int64_t N, double* L, doub
   // log L_ii, and the flag of a matrix that is not positive definite in the last word
   HIPCHK(ctx->dn_dlog.reserve((size_t)N + 1));
   int* d_bad = reinterpret_cast<int*>(ctx->dn_dlog.p + N);
-  HIPCHK(ctx->dn_inv.reserve((size_t)DENSE_PANEL * DENSE_PANEL));
-  HIPCHK(launch_dense_cholesky(A, N, ctx->dn_inv.p, ctx->dn_dlog.p, d_bad, s));
+  HIPCHK(ctx->dn_panel.reserve((size_t)DENSE_PANEL * DENSE_PANEL));
+  HIPCHK(launch_dense_cholesky(A, N, ctx->dn_panel.p, ctx->dn_dlog.p, d_bad, s));
   static_assert(PIN_OUT >= 65536 * sizeof(double), "the largest N fits");
   const double* dl = reinterpret_cast<const double*>(ctx->pin_out);
   HIPCHK(launch_stage(ctx->dn_dlog.p, ctx->pin_out, ((size_t)N + 1) * sizeof(double), s));
@@ -1377,20 +1377,20 @@ int jc_gaussian_loglike_dense(jc_ctx* ctx, const float* mu, int64_t B, int64_t N
   if (rc) return rc;
   HIPCHK(ctx->dn_inv.reserve(tri_inverse_size(N)));
   HIPCHK(launch_tri_inverse(d_L, N, ctx->dn_inv.p, s));
-  if ((rc = to_device(ctx, ctx->lk_data, data, (size_t)N, dev, &d_data))) return rc;
-  if ((rc = to_device(ctx, ctx->lk_mu, mu, nmu, dev, &d_mu))) return rc;
+  if ((rc = to_device(ctx, ctx->dn_data, data, (size_t)N, dev, &d_data))) return rc;
+  if ((rc = to_device(ctx, ctx->dn_mu, mu, nmu, dev, &d_mu))) return rc;
   float* d_s = dloglike_dmu;
   if (!dev && dloglike_dmu) {
-    HIPCHK(ctx->lk_s.reserve(nmu));
-    d_s = ctx->lk_s.p;
+    HIPCHK(ctx->dn_s.reserve(nmu));
+    d_s = ctx->dn_s.p;
   }
   const bool pinned = !dev && (size_t)B * sizeof(double) <= PIN_OUT;
   double* d_ll = loglike;
   if (pinned) {
     d_ll = reinterpret_cast<double*>(ctx->pin_out);
   } else if (!dev) {
-    HIPCHK(ctx->lk_out.reserve((size_t)B));
-    d_ll = ctx->lk_out.p;
+    HIPCHK(ctx->dn_out.reserve((size_t)B));
+    d_ll = ctx->dn_out.p;
   }
   HIPCHK(ctx->dn_z.reserve(nmu));
   HIPCHK(ctx->dn_x.reserve(nmu));

@@ -216,9 +216,14 @@ struct jc_ctx {
   // likelihood workspace: inputs staged from host, mean, cotangent, partials
   DevBuf<double> lk_cosmo, lk_ell, lk_data, lk_prec, lk_part, lk_out, lk_grad, lk_inv;
   DevBuf<float> lk_mu, lk_s;
-  // dense likelihood workspace: staged matrix, log L_ii and non-SPD flag, [B][N]
-  // solves, inverses of the factor's diagonal blocks
-  DevBuf<double> dn_mat, dn_dlog, dn_z, dn_x, dn_inv;
+  // dense likelihood workspace: staged matrix, [B][N] solves, inverses of the
+  // factor's diagonal blocks
+  DevBuf<double> dn_mat, dn_z, dn_x, dn_inv;
+  // apart from them and from lk_*: the factorisation (log L_ii and non-SPD flag, the
+  // panel's inverse) may run beside an unfinished dense call on device pointers on
+  // another stream, host means beside a block-diagonal one
+  DevBuf<double> dn_dlog, dn_panel, dn_data, dn_out;
+  DevBuf<float> dn_mu, dn_s;
   DevBuf<float> chitab, coef, crec, R, out, out_t, jac, cbar, theta_col, part;
   DevBuf<float4> ehtab;
   DevBuf<float> ehtab7;

@@ -1,5 +1,6 @@
 """Dense solves on device arrays take no memory of the context: solves on
-several streams side by side, a captured solve replayed between eager ones, and
+several streams side by side, a captured solve replayed between eager ones,
+calls that wait for their result beside an unfinished one on another stream, and
 the library's own in-place form, against LAPACK to 1e-10 as in the tests of the
 blocks' edges."""
 import ctypes
@@ -92,3 +93,68 @@ def test_captured_solve(n):
         torch.cuda.synchronize()
         want = solution(L, R, 2)
         np.testing.assert_allclose(X.cpu().numpy(), want, rtol=0, atol=1e-10 * max(1.0, np.abs(want).max()))
+
+
+def test_factorisation_beside_a_pending_likelihood():
+    # the likelihoods of many device means are queued on one stream; the call
+    # returns, and covariances are factored on another meanwhile
+    ctx = default_context()
+    n, B = 1200, 512
+    rng = np.random.default_rng(5)
+    L, Lt = factor(n, 7)
+    mu, data = rng.normal(size=(B, n)).astype(np.float32), rng.normal(size=n)
+    want = -0.5 * (solution(L, data - mu.astype(np.float64), 0) ** 2).sum(1)
+    mut, dt = torch.as_tensor(mu, device="cuda"), torch.as_tensor(data, device="cuda")
+    C = spd(700, 8)
+    ref = np.linalg.cholesky(C)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(5):
+        ll = torch.zeros(B, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        with ctx._lock:
+            ctx.set_stream(a.cuda_stream)
+            check(ctx.lib.jc_gaussian_loglike_dense(
+                ctx.handle, ctypes.c_void_p(mut.data_ptr()), B, n, ctypes.c_void_p(dt.data_ptr()),
+                ctypes.c_void_p(Lt.data_ptr()), 0.0, ctypes.c_void_p(ll.data_ptr()), None, JC_DEVICE_PTRS))
+            ctx.reset_stream()
+        with torch.cuda.stream(b):
+            F, _ = ctx.dense_cholesky(C)
+        torch.cuda.synchronize()
+        np.testing.assert_allclose(ll.cpu().numpy(), want, rtol=1e-10)
+        np.testing.assert_allclose(F.cpu().numpy(), ref, rtol=0, atol=1e-10)
+
+
+def test_host_means_beside_a_pending_gradient():
+    # log-likelihoods and gradients of a batch under a block-diagonal covariance
+    # are queued on one stream; host means take the dense algebra on another
+    import jax_cosmo_amd as jc
+    from test_gpu_forward_table import PARAMS, make_probes
+
+    ctx = default_context()
+    jc.cl._check_fns(jc.transfer.Eisenstein_Hu, jc.power.halofit)
+    probes, ell, n_z, B = make_probes(2, 2), np.geomspace(20.0, 2000.0, 70), 256, 256
+    sid, P = ctx.tracer_set(jc.cl.tracer_entries(probes)), 10
+    params = PARAMS[np.arange(B) % 3]
+    cl = ctx.angular_cl(PARAMS[:1], sid, ell, n_z, P)[0].astype(np.float64)
+    prec = np.ascontiguousarray(np.eye(P)[..., None] / (0.1 * np.abs(cl[None])) ** 2)
+    data = 1.05 * cl
+    ll0, g0 = ctx.gaussian_loglike_grad(params, sid, ell, n_z, data, prec)
+    n = 900
+    L, Lt = factor(n, 4)
+    mu, d = np.random.default_rng(2).normal(size=(64, n)).astype(np.float32), np.ones(n)
+    want = -0.5 * (solution(L, d - mu.astype(np.float64), 0) ** 2).sum(1)
+    dev = [torch.as_tensor(x, device="cuda") for x in (params, ell, data, prec)]
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(5):
+        ll = torch.zeros(B, dtype=torch.float64, device="cuda")
+        g = torch.zeros((B, 7), dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        ctx.gaussian_loglike_grad_dev(dev[0].data_ptr(), B, sid, dev[1].data_ptr(), len(ell), n_z, dev[2].data_ptr(),
+                                      dev[3].data_ptr(), 0.0, ll.data_ptr(), g.data_ptr(), stream=a.cuda_stream)
+        with torch.cuda.stream(b):
+            got, dmu = ctx.gaussian_loglike_dense(mu, d, Lt, want_dmu=True)
+        torch.cuda.synchronize()
+        ctx.reset_stream()
+        np.testing.assert_allclose(got, want, rtol=1e-10)
+        np.testing.assert_array_equal(ll.cpu().numpy(), ll0)  # the same sums in the same order
+        np.testing.assert_array_equal(g.cpu().numpy(), g0)
