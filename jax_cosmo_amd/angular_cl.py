@@ -7,6 +7,8 @@ The covariance helpers are float64: host arrays for host inputs, torch
 tensors (differentiable) when the C_ell come from a cosmology with torch
 parameters.
 """
+import threading
+
 import numpy as np
 
 from . import power
@@ -222,24 +224,30 @@ class BatchGraph:
 
 _ELL_CACHE = {}
 _ELL_CACHE_MAX = 16
+_ELL_LOCK = threading.Lock()  # backward passes run on autograd's threads
 
 
 def _device_ell(ell, device):
     """ell as a float64 tensor on ``device``.  A device tensor is used as it
     is; a host array is uploaded once and kept (keyed by its bytes), so that
-    repeated batches over the same multipoles copy nothing to the device."""
+    repeated batches over the same multipoles copy nothing to the device.  The
+    tensor may be read on the current stream: should it leave the cache, its
+    memory waits for what that stream has queued by then."""
     import torch
 
     if _is_torch(ell):
         return ell.to(device=device, dtype=torch.float64).contiguous()
     a = np.ascontiguousarray(np.atleast_1d(np.asarray(ell, dtype=np.float64)))
     key = (str(device), a.tobytes())
-    el = _ELL_CACHE.get(key)
-    if el is None:
-        if len(_ELL_CACHE) >= _ELL_CACHE_MAX:
-            _ELL_CACHE.pop(next(iter(_ELL_CACHE)))
-        el = torch.as_tensor(a, device=device).contiguous()
-        _ELL_CACHE[key] = el
+    with _ELL_LOCK:
+        el = _ELL_CACHE.get(key)
+        if el is None:
+            el = torch.as_tensor(a, device=device).contiguous()
+            if len(_ELL_CACHE) >= _ELL_CACHE_MAX:
+                _ELL_CACHE.pop(next(iter(_ELL_CACHE)))
+            _ELL_CACHE[key] = el
+    if el.is_cuda:
+        el.record_stream(torch.cuda.current_stream(el.device))
     return el
 
 

@@ -26,6 +26,13 @@ def _assemble(theta, omega_k):
     return params
 
 
+def _kept_ell(ell64, device):
+    # a graph would hold the kept tensor's address (and the context's buffers') for good
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("C_ell with gradients cannot be captured into a graph (BatchGraph captures a forward batch)")
+    return _device_ell(ell64, device)
+
+
 class AngularClFunction(torch.autograd.Function):
     """C[B, P, n_ell] = angular_cl(theta[B, 7]); float32 output."""
 
@@ -35,7 +42,7 @@ class AngularClFunction(torch.autograd.Function):
         params = _assemble(theta, omega_k)
         ell64 = np.ascontiguousarray(np.asarray(ell, dtype=np.float64).reshape(-1))
         if theta.is_cuda:
-            el = _device_ell(ell64, theta.device)
+            el = _kept_ell(ell64, theta.device)
             out = torch.empty((params.shape[0], n_pairs, el.shape[0]), dtype=torch.float32,
                               device=theta.device)
             dctx.angular_cl_dev(params.data_ptr(), params.shape[0], set_id, el.data_ptr(),
@@ -57,7 +64,7 @@ class AngularClFunction(torch.autograd.Function):
         dctx.set_growth(models[2])
         g32 = grad.detach().to(torch.float32).contiguous()
         if params.is_cuda:
-            el = _device_ell(ell64, params.device)
+            el = _kept_ell(ell64, params.device)
             th = torch.empty((params.shape[0], 7), dtype=torch.float64, device=params.device)
             dctx.angular_cl_vjp_dev(params.data_ptr(), params.shape[0], set_id, el.data_ptr(),
                                     el.shape[0], n_z, g32.data_ptr(), th.data_ptr(),
