@@ -431,7 +431,7 @@ __global__ __launch_bounds__(64 * ADJ_WAVES, 3) void k_ragged_adjoint(RaggedArgs
   extern __shared__ float4 lds4[];
   const int ngrp = adj_groups(A.Na), per = (A.Na + ngrp - 1) / ngrp;
   const int units = *A.njobs * ngrp;
-  const int nsl = adj_ragged_slices(units);
+  const int nsl = adj_ragged_slices(units, A.min_slices);
   const int live = units * nsl;
   const int xq = live >> 3, xr = live & 7, xx = blockIdx.x & 7, xi = blockIdx.x >> 3;
   if (xi >= xq + (xx < xr ? 1 : 0)) return;
@@ -439,7 +439,9 @@ __global__ __launch_bounds__(64 * ADJ_WAVES, 3) void k_ragged_adjoint(RaggedArgs
   const int y = b % nsl, u = b / nsl, grp = u % ngrp;
   const RJob& jb = A.jobs[u / ngrp];
   const int c = jb.c;
-  const int chunk = (jb.n_ell + nsl - 1) / nsl;
+  // (a request takes the slices that itself asks for; its other blocks are empty)
+  const int own = adj_ragged_slices(units, adj_min_slices(jb.n_ell));
+  const int chunk = (jb.n_ell + own - 1) / own;
   const float* cr = A.crec + (size_t)c * NCREC * 8;
   AdjIn in;
   in.coef = A.coef + (size_t)c * A.Na * NCOEF * 8;
@@ -474,8 +476,8 @@ __global__ __launch_bounds__(64 * ADJ_WAVES, 3) void k_ragged_adjoint(RaggedArgs
 }
 
 hipError_t launch_ragged_adjoint(int max_jobs, const RaggedArgs& a, hipStream_t s) {
-  if (max_jobs < 1 || !a.njobs || !a.ehtab || !a.ehtab7 || !a.theta_part) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_ragged_adjoint, dim3(adj_ragged_blocks(max_jobs, a.Na)), dim3(64 * ADJ_WAVES),
+  if (max_jobs < 1 || a.min_slices < 1 || !a.njobs || !a.ehtab || !a.ehtab7 || !a.theta_part) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_ragged_adjoint, dim3(adj_ragged_blocks(max_jobs, a.Na, a.min_slices)), dim3(64 * ADJ_WAVES),
                      AdjShape<MAXT>::LDS * sizeof(float), s, a);
   return hipGetLastError();
 }
@@ -488,7 +490,7 @@ __global__ __launch_bounds__(64) void k_ragged_reduce(RaggedArgs A, double* __re
   const int j = blockIdx.x;
   if (j >= *A.njobs) return;  // uniform across the block
   const int ngrp = adj_groups(A.Na);
-  const int n = ngrp * adj_ragged_slices(*A.njobs * ngrp);
+  const int n = ngrp * adj_ragged_slices(*A.njobs * ngrp, A.min_slices);
   const float* p = A.theta_part + (size_t)j * n * 7;
   const int t = threadIdx.x;
   if (t < 63) {

@@ -467,10 +467,12 @@ int auto_slices(const jc_ctx* ctx, int64_t ncols, int waves, int Na, int nd) {
 // turn of 8 multipoles.  Measured (100 ell, n_z 512, 10 tracers): twice the
 // blocks 46 against 31 us at 16 cosmologies and 65 against 61 at 64 (the tables
 // are staged and the derivatives contracted per block); turns of 4 multipoles
-// 31.6 against 22.1 us at 4 cosmologies, 16.1 against 17.2 at one.
+// 31.6 against 22.1 us at 4 cosmologies, 16.1 against 17.2 at one.  At least so
+// many that a block's sums stay short (ADJ_TERMS), up to the grid's limit.
 int adjoint_slices(const jc_ctx* ctx, int64_t B, int n_ell, int Na) {
   const int64_t units = B * adj_groups(Na);
-  return (int)std::max<int64_t>(1, std::min<int64_t>(3 * (int64_t)ctx->num_cu / units, n_ell / 8));
+  const int64_t fill = std::min<int64_t>(3 * (int64_t)ctx->num_cu / units, n_ell / 8);
+  return (int)std::min<int64_t>(std::max<int64_t>(fill, adj_min_slices(n_ell)), 65535);
 }
 // Timing events only: jc_profile_read synchronizes the stream before reading
 // them, so they need no system-scope release (without it each record cost

@@ -250,7 +250,8 @@ size_t layout_slot(jc_server* S, Slot* sl, unsigned char* base) {
     b.ehtab_d = (float4*)take((size_t)S->Gd * NEHQ * sizeof(float4));
     b.ehtab7 = (float*)take((size_t)S->Gd * (NEHQ + 1) * NEHD_ROW * 4);
     b.theta_part = (float*)take(
-        std::max((size_t)ADJ_ROWS * S->gcolcap, (size_t)adj_ragged_blocks(S->Gd, (int)Na)) * 7 * 4);
+        std::max((size_t)ADJ_ROWS * S->gcolcap,
+                 (size_t)adj_ragged_blocks(S->Gd, (int)Na, adj_min_slices(S->cfg.max_ell))) * 7 * 4);
   }
   return off;
 }
@@ -352,6 +353,7 @@ hipError_t enqueue_pass(jc_server* S, Slot* sl, int pass, hipStream_t ps, const 
         ra.cbar = sl->cbar;
         ra.njobs = cnt + 2;
         ra.theta_part = b.theta_part;
+        ra.min_slices = adj_min_slices(S->cfg.max_ell);
         ra.waves = S->waves;
         ra.ehtab = ta.ehtab;
         ra.ehtab7 = ta.ehtab7;
