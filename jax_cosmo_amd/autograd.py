@@ -76,16 +76,17 @@ class AngularClFunction(torch.autograd.Function):
 
 
 def angular_cl_torch(params, ell, probes, n_z=512):
-    """angular_cl for a Cosmology whose parameters are (some) torch scalars.
+    """angular_cl for a Cosmology whose parameters are torch scalars or numbers.
     Returns [B=1, n_cls, n_ell]; gradients reach the torch parameters."""
     from .angular_cl import _n_cls, tracer_entries
 
     vals = [params[i] for i in GRAD_INDEX]
-    first = next(p for p in params if isinstance(p, torch.Tensor))
+    first = next((p for p in params if isinstance(p, torch.Tensor)), None)  # None: numbers only, on the host
     if not all(isinstance(p, torch.Tensor) and p.dtype == first.dtype and p.is_floating_point() for p in vals):
         # numbers, or several types: one conversion (and its backward) each
+        dev = None if first is None else first.device
         vals = [p.to(torch.float64) if isinstance(p, torch.Tensor)
-                else torch.tensor(float(p), dtype=torch.float64, device=first.device) for p in vals]
+                else torch.tensor(float(p), dtype=torch.float64, device=dev) for p in vals]
     theta = torch.stack([p.reshape(()) for p in vals]).reshape(1, 7)
     ok = params[5]
     omega_k = float(ok.detach().cpu()) if isinstance(ok, torch.Tensor) else float(ok)
