@@ -172,6 +172,7 @@ class Context:
         self._lock = threading.RLock()
         self._models = [0, 0, None]  # transfer, nonlinear, gamma (the library's defaults)
         self.tables_variant = 0      # the table kernel's shape (jc_set_tables_variant)
+        self.forward_options = [1, 0]  # transfer_table, matrix_cores
 
     def close(self):
         if self.handle:
@@ -426,6 +427,9 @@ class Context:
         per-cosmology table instead of the EH98 closed form per point, and the
         pair contraction on the matrix cores instead of per-lane FMAs."""
         check(self.lib.jc_set_forward_options(self.handle, int(transfer_table), int(matrix_cores)))
+        for i, v in enumerate((int(transfer_table), int(matrix_cores))):
+            if v >= 0:
+                self.forward_options[i] = v
 
     def get_tiles(self):
         w = _I32()

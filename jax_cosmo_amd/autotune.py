@@ -1,13 +1,17 @@
 """Tile autotuner for the batched and served Limber paths.
 
 Tunables:
-  waves     -- waves per block of the Limber kernel, each taking a share of
+  waves     -- waves per block of the Limber kernels, each taking a share of
                the a-nodes of the same 64 (cosmology, ell) columns (1, 2, 4);
+               the forward kernel of transfer-table calls has its own;
   wl_ctile  -- cosmologies per block of the weak-lensing kernel, which reuse
-               every resident-table element they load (1, 4, 8).
-The batch tuner times each candidate with HIP events recorded around the
-launches (jc_profile_*), the server tuner by draining a sample stream.
-Results are cached as JSON keyed by device and shape.
+               every resident-table element they load (1, 4, 8, 16);
+  tables_variant -- shape of the table kernel (1, 2, 3).
+0 is the library's launch rule, which a batch keeps unless a fixed shape is
+faster by more than NOISE.  The batch tuner times each candidate with HIP events
+recorded around the launches (jc_profile_*), the server tuner by draining a
+sample stream.  Results are cached as JSON keyed by device, shape and kernel
+revision.
 """
 import json
 import os
@@ -20,11 +24,14 @@ from ._native import default_context
 WAVES = (1, 2, 4)
 CTILES = (1, 4, 8, 16)
 TABLE_VARIANTS = (1, 2, 3)
+NOISE = 0.06  # relative; two timings of one launch, the first included, differ by so much
+REVISION = 2  # of the kernels' launch shapes: tiles timed on others are not found
 
 
 def cache_path():
     """JSON cache of tuned tiles: $JAX_COSMO_AMD_TUNE_CACHE, else the file
-    shipped next to the package (tuned on MI355X)."""
+    shipped next to the package (the server's tiles on MI355X; batches take the
+    launch rules until they are tuned)."""
     return os.environ.get("JAX_COSMO_AMD_TUNE_CACHE",
                           os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuned_tiles.json"))
 
@@ -71,16 +78,23 @@ def _device_name():
 
 def batch_key(B, n_ell, n_z, T):
     b = 1 << max(0, int(np.ceil(np.log2(max(B, 1)))))  # power-of-two bucket
-    return "%s|batch|B%d|L%d|N%d|T%d" % (_device_name(), b, n_ell, n_z, T)
+    return "%s|k%d|batch|B%d|L%d|N%d|T%d" % (_device_name(), REVISION, b, n_ell, n_z, T)
 
 
 def lookup_batch(B, n_ell, n_z, T):
     return _load().get(batch_key(B, n_ell, n_z, T))
 
 
+def _best(results, key):
+    """The fastest, or the first (the launch rule) where it is as fast."""
+    best = min(results, key=key)
+    return results[0] if key(results[0]) <= (1.0 + NOISE) * key(best) else best
+
+
 def tune_batch(probes, B, n_ell=100, n_z=512, reps=3, seed=0, ctx=None):
-    """Time every (waves, wl_ctile) on a synthetic batch of the given shape;
-    cache and return the best {"waves", "wl_ctile", "ms"}."""
+    """Time the table kernel's shapes, then every (waves, wl_ctile), on a
+    synthetic batch of the given shape; cache and return the best {"waves",
+    "wl_ctile", "tables_variant", "ms"}."""
     from .angular_cl import _get_cl_ordering, tracer_entries
 
     ctx = ctx or default_context()
@@ -108,15 +122,16 @@ def tune_batch(probes, B, n_ell=100, n_z=512, reps=3, seed=0, ctx=None):
 
     try:
         # the three kernels are independent tunables: tables variant first,
-        # then (waves, wl_ctile) with the best variant
+        # then (waves, wl_ctile) with the best variant; the rule comes first
         tv = []
-        for v in TABLE_VARIANTS:
+        for v in (0,) + TABLE_VARIANTS:
             ctx.set_tables_variant(v)
             tv.append((timed()["tables"], v))
-        best_v = min(tv)[1]
+        best_v = _best(tv, key=lambda r: r[0])[1]
         ctx.set_tables_variant(best_v)
-        for w in WAVES:
-            for ct in CTILES:
+        table_call = ctx.forward_options == [1, 0] and n_ell >= 64  # its kernel ignores waves
+        for w in (0,) if table_call else (0,) + WAVES:
+            for ct in (0,) + CTILES:
                 ctx.set_tiles(w, ct)
                 t = timed()
                 results.append({"waves": w, "wl_ctile": ct, "tables_variant": best_v,
@@ -125,7 +140,7 @@ def tune_batch(probes, B, n_ell=100, n_z=512, reps=3, seed=0, ctx=None):
     finally:
         ctx.set_tiles(*old)
         ctx.set_tables_variant(0)
-    best = min(results, key=lambda r: r["ms"])
+    best = _best(results, key=lambda r: r["ms"])
     best["tables_candidates"] = [{"variant": v, "ms": ms} for ms, v in tv]
     db = dict(_load())
     db[batch_key(B, n_ell, n_z, T)] = dict(best, candidates=results, when=time.time())
@@ -146,7 +161,7 @@ def apply_batch(ctx, B, n_ell, n_z, T):
 
 
 def server_key(n_z, max_batch):
-    return "%s|server|N%s|C%d" % (_device_name(), ",".join(str(v) for v in n_z), max_batch)
+    return "%s|k%d|server|N%s|C%d" % (_device_name(), REVISION, ",".join(str(v) for v in n_z), max_batch)
 
 
 def lookup_server(n_z, max_batch):
