@@ -8,8 +8,8 @@
 // derivatives the table and lensing kernels stored.  So the sum over ell is
 // taken first, and the derivatives are contracted once per node instead of
 // once per point: lane = a-node, loop over ell,
-//   V_i = sum_j ct_ij R_j (ct symmetric, diagonal doubled),  G = 1/2 sum_i R_i V_i,
-//   Rbar_i += M V_i,   xbar += G dM/dx for each record field x,
+//   V_i = 1/2 sum_j ct_ij R_j (ct symmetric, diagonal doubled),  G = sum_i R_i V_i,
+//   Rbar_i += 2 M V_i,   xbar += G dM/dx for each record field x,
 // then theta-bar = sum_nodes (sum_x xbar dx/dtheta + sum_i Rbar_i dR_i/dtheta)
 // plus T(k)'s own derivative at fixed k, read from the table of theta
 // derivatives at every point (4-point Lagrange).  The lanes' 31 sums and the
@@ -17,8 +17,8 @@
 // constants are the same for all lanes and come from LDS as broadcasts.
 // With lane = (cosmology, ell) instead, every point reads the node's 224 dual
 // floats and spends 7 FMAs on each.  Measured, 256 cosmologies x 100 ell x n_z
-// 512: 10 tracers 610 -> 158 us; bound by VALU issue (300 instructions a point,
-// 120 of them the cotangents' share, which takes 35 of the 158 us) with the LDS
+// 512: 10 tracers 610 -> 160 us; bound by VALU issue (300 instructions a point,
+// 120 of them the cotangents' share, which takes 35 of the 160 us) with the LDS
 // reads of a point beside it (25 float4, 9 of them gathers: 9 us).  Staging the
 // tables costs 5-8 us and the contraction with the derivatives, 58 KB a block,
 // 9-13 us.
@@ -29,7 +29,7 @@ namespace jc {
 namespace {
 
 // multipoles staged per turn: two per wave, so that with the tables three
-// blocks fit a CU's LDS (two points unrolled: no gain, 158 us)
+// blocks fit a CU's LDS (two points unrolled: no gain)
 constexpr int ADJ_EC = 8;
 constexpr int ADJ_HDR = 64;  // multipole constants computed per turn
 
@@ -45,7 +45,7 @@ struct AdjShape {
   static constexpr int ROW = (P + 3) / 4 * 4 + 4;  // staged cotangents of a multipole; + 4 spreads the banks
   static constexpr int NQ = ADJ_NX + T;            // node sums
   static constexpr int LDS = 4 * NEHQ + 8 * (NEHQ + 1) + ADJ_EC * ROW + 8 * ADJ_HDR;  // floats
-  static_assert(ADJ_WAVES * NQ * 64 + 64 * NQ + 64 <= LDS, "the reduction reuses the tables' space");
+  static_assert(ADJ_WAVES * NQ * 64 + 2 * 64 * NQ + 64 <= LDS, "the reduction reuses the tables' space");
 };
 
 // What one block reads: `n1 - n0` <= 64 nodes of one cosmology, multipoles
@@ -107,7 +107,7 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
   for (int i = 0; i < T; ++i) Rv[i] = A.R[((size_t)(A.n0 + min(lane, nn - 1)) * A.Tpad + i) * 8];
 
   // staging of the cotangents: thread -> multipole t % EC, pairs t / EC + k NP;
-  // each pair's power of the lensing factor and its diagonal's 2
+  // each pair's power of the lensing factor and its share of V (1/2, diagonal 1)
   constexpr int NP = 64 * ADJ_WAVES / ADJ_EC, KP = (P + NP - 1) / NP;
   const int sl = t % ADJ_EC;
   int wlp[KP];
@@ -117,7 +117,7 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
     int q = t / ADJ_EC + k * NP, i = 0;
     while (i < T && q >= T - i) q -= T - i++;
     wlp[k] = (int)((A.wl_mask >> i) & 1u) + (int)((A.wl_mask >> min(i + q, 31)) & 1u);
-    dia[k] = q == 0 ? 2.0f : 1.0f;
+    dia[k] = q == 0 ? 1.0f : 0.5f;
   }
   auto fetch = [&](int l, float* v) {
 #pragma unroll
@@ -162,7 +162,7 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
     float G = 0.0f;
 #pragma unroll
     for (int i = 0; i < T; ++i) G = __builtin_fmaf(Rv[i], V[i], G);
-    G *= 0.5f;
+    G *= h1.z;  // here, not in the cotangents: l^-3 would take 40 bits of their range
     // the bracket S = q1 + q2 of fwd_point, q1 = d2l eq / d0, q2 = a_n yf1 / (A B)
     float ft;
     const int q = tab_piece(r, e, ft);
@@ -189,7 +189,7 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
     const float gy = G * (yf1 * r12); // G q2 / a_n
     const float p2 = r.d.z * gy;      // G q2
     aS += p1 + p2;
-    const float M = r.d.w * __builtin_fmaf(d2l, eq * r0, r.d.z * (yf1 * r12));
+    const float M = (r.d.w * h1.z) * __builtin_fmaf(d2l, eq * r0, r.d.z * (yf1 * r12));
 #pragma unroll
     for (int i = 0; i < T; ++i) Rb[i] = __builtin_fmaf(M, V[i], Rb[i]);
     // q1: d ln q1 = (1 - alpha d2l / d0 + beta d2l / (1 + d2l)) d ln d2l
@@ -255,12 +255,12 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
       __syncthreads();
     }
     {
-      const float2 f = *reinterpret_cast<const float2*>(hdr + (hl + sl) * 8 + 6);
+      const float lf = hdr[(hl + sl) * 8 + 7];
 #pragma unroll
       for (int k = 0; k < KP; ++k) {
-        const float F = wlp[k] == 0 ? 1.0f : (wlp[k] == 1 ? f.y : f.y * f.y);
+        const float F = wlp[k] == 0 ? 1.0f : (wlp[k] == 1 ? lf : lf * lf);
         const int p = t / ADJ_EC + k * NP;
-        if (p < P) rows[sl * ROW + p] = nv[k] * F * (f.x * dia[k]);
+        if (p < P) rows[sl * ROW + p] = nv[k] * (F * dia[k]);
       }
     }
     __syncthreads();
@@ -273,8 +273,8 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
   // the waves' sums of each node, in order; then wave 0's lanes turn them into
   // cotangents of the record fields
   float* red = reinterpret_cast<float*>(lds4);
-  float* xs = red + ADJ_WAVES * NQ * 64;
-  double* wsum = reinterpret_cast<double*>(xs + 64 * NQ);  // [ADJ_WAVES][8]
+  double* xs = reinterpret_cast<double*>(red + ADJ_WAVES * NQ * 64);  // (the weight's cotangent needs the range)
+  double* wsum = xs + 64 * NQ;  // [ADJ_WAVES][8]
   const float sums[ADJ_NX] = {aS, aG3, aY, aAL, aB, aAN, aF1, aBN, aF2, aC, aGAM, aMU, aNU, aSL};
   __syncthreads();
 #pragma unroll
@@ -292,12 +292,12 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
     float v[ADJ_NX];
 #pragma unroll
     for (int k = 0; k < ADJ_NX; ++k) v[k] = node_sum(k);
-    const float AW = r.d.w;
-    const float cA = (float)(2.0 * PI * PI) * (chi1 * chi1 * chi1);
+    const double AW = r.d.w;
+    const double cA = (2.0 * PI * PI) * ((double)chi1 * chi1 * chi1);
     const float yy = 0.25f * v[2];                                   // d / d ln y
     const float la = r.c.x * (r.d.z * v[5]) + r.c.y * (r.d.y * v[7]) + r.c.z * v[9];  // d / d ln y of the powers
     const float mn = r.b.y * v[11] + 2.0f * r.b.z * v[12];
-    float* x = xs + lane * NQ;
+    double* x = xs + lane * NQ;
     // G3, AW, y and the position of the table all carry chi; y and mu / y carry R_nl
     x[0] = AW * (3.0f * (r.a.z * v[1] - v[0]) + (yy + la - mn) + A.invh * v[13]);
     x[1] = cA * v[0];
@@ -316,18 +316,18 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
   } else {
 #pragma unroll
     for (int i = 0; i < T; ++i)
-      if (i % (ADJ_WAVES - 1) == wave - 1) xs[lane * NQ + ADJ_NX + i] = node_sum(ADJ_NX + i);
+      if (i % (ADJ_WAVES - 1) == wave - 1) xs[lane * NQ + ADJ_NX + i] = 2.0 * (double)node_sum(ADJ_NX + i);
   }
   __syncthreads();
   // contraction with the stored derivatives in FP64: even threads read
   // (value, d0, d1, d2) of a field, odd threads (d3 .. d6); coalesced
   double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  auto add = [&](float x, const float* p) {
+  auto add = [&](double x, const float* p) {
     const float4 d = *reinterpret_cast<const float4*>(p + (t & 1) * 4);
-    s0 += (double)x * (double)(t & 1 ? d.x : d.y);
-    s1 += (double)x * (double)(t & 1 ? d.y : d.z);
-    s2 += (double)x * (double)(t & 1 ? d.z : d.w);
-    if (t & 1) s3 += (double)x * (double)d.w;
+    s0 += x * (double)(t & 1 ? d.x : d.y);
+    s1 += x * (double)(t & 1 ? d.y : d.z);
+    s2 += x * (double)(t & 1 ? d.z : d.w);
+    if (t & 1) s3 += x * (double)d.w;
   };
   for (int e = t >> 1; e < nn * ADJ_NX; e += 32 * ADJ_WAVES) {
     const int n = e / ADJ_NX, j = e - n * ADJ_NX;
