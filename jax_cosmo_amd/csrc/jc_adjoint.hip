@@ -363,19 +363,13 @@ JC_D void adjoint_block(const AdjIn& A, float4* lds4) {
   }
 }
 
-// contiguous ranges of blocks per XCD (block b runs on XCD b % 8)
-JC_D int xcd_range(int b, int n) {
-  const int q = n >> 3, r = n & 7, x = b & 7;
-  return x * q + min(x, r) + (b >> 3);
-}
-
 }  // namespace
 
 template <int T>
 __global__ __launch_bounds__(64 * ADJ_WAVES, 3) void k_adjoint(LimberArgs A) {
   extern __shared__ float4 lds4[];
   const int ngrp = adj_groups(A.Na), per = (A.Na + ngrp - 1) / ngrp;
-  const int b = xcd_range(blockIdx.x, gridDim.x);
+  const int b = xcd_order(blockIdx.x, gridDim.x);
   const int c = b / ngrp, grp = b - c * ngrp;
   const int chunk = (A.n_ell + A.slices - 1) / A.slices;
   const float* cr = A.crec + (size_t)c * NCREC * 8;
@@ -433,9 +427,10 @@ __global__ __launch_bounds__(64 * ADJ_WAVES, 3) void k_ragged_adjoint(RaggedArgs
   const int units = *A.njobs * ngrp;
   const int nsl = adj_ragged_slices(units, A.min_slices);
   const int live = units * nsl;
-  const int xq = live >> 3, xr = live & 7, xx = blockIdx.x & 7, xi = blockIdx.x >> 3;
-  if (xi >= xq + (xx < xr ? 1 : 0)) return;
-  const int b = xx * xq + min(xx, xr) + xi;
+  const XcdShare xs = xcd_share(blockIdx.x, live);
+  const int xi = blockIdx.x >> 3;
+  if (xi >= xs.count) return;
+  const int b = xs.first + xi;
   const int y = b % nsl, u = b / nsl, grp = u % ngrp;
   const RJob& jb = A.jobs[u / ngrp];
   const int c = jb.c;

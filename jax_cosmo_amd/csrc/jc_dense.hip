@@ -561,8 +561,7 @@ __global__ __launch_bounds__(256, 2) void k_solve_update(const double* __restric
   const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nb = (int)min((int64_t)BS, N - k0);
-  const int n = gridDim.x, q8 = n >> 3, r8 = n & 7, xc = blockIdx.x & 7;  // block b runs on XCD b % 8
-  const int id = xc * q8 + min(xc, r8) + (blockIdx.x >> 3);
+  const int id = xcd_order(blockIdx.x, gridDim.x);
   const int64_t row0 = (TR ? 0 : k0 + BS) + (int64_t)(id / gy) * 32, row_end = TR ? k0 : N;
   const int64_t b0 = (int64_t)(id % gy) * (16 * WB);
   const double* x[WB];

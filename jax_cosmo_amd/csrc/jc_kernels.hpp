@@ -272,6 +272,20 @@ struct RaggedArgs {
   int64_t part_stride;
 };
 
+// The dispatcher deals blocks to the 8 XCDs in turn (block b to XCD b % 8), and each
+// XCD has its own L2.  Neighbouring units of work read the same records, so units are
+// renumbered to give each XCD one contiguous range of them: a record is then fetched
+// into one L2 instead of two or three.  xcd_share: the range of block b's XCD;
+// xcd_order: the unit of block b of n (a bijection of [0, n) for any n).
+struct XcdShare {
+  int first, count;
+};
+__device__ inline XcdShare xcd_share(int b, int n) {
+  const int q = n >> 3, r = n & 7, x = b & 7;
+  return {x * q + (x < r ? x : r), q + (x < r ? 1 : 0)};
+}
+__device__ inline int xcd_order(int b, int n) { return xcd_share(b, n).first + (b >> 3); }
+
 // The adjoint's blocks (jc_adjoint.hip): a cosmology's a-nodes in groups of up
 // to 64 (lanes), its multipoles dealt to ADJ_WAVES waves and, where that leaves
 // the chip idle, to several blocks.

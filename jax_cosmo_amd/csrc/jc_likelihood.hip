@@ -23,12 +23,6 @@ namespace jc {
 
 constexpr int LK_MAXP = 64;  // pairs per block (10 tracers give 55)
 
-// block b of n on XCD b % 8 (a bijection of [0, n))
-__device__ __forceinline__ int xcd_order(int b, int n) {
-  const int q = n >> 3, r = n & 7, x = b & 7;
-  return x * q + min(x, r) + (b >> 3);
-}
-
 // element (p, q) of block l of a precision array
 __device__ __forceinline__ size_t prec_at(const PrecLayout& a, int P, int p, int q, int l) {
   return ((size_t)p * P + q) * a.pair + (size_t)l * a.ell;

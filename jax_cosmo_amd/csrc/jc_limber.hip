@@ -163,16 +163,6 @@ JC_D Dual<float, 7> adj_tn_closed(const EHc<Dual<float, 7>>& eh, const Dual<floa
   return eh_transfer(eh, kd, invkd, lnkd) * jm::exp(ns * (0.5f * lnkd));
 }
 
-// The dispatcher deals blocks to the 8 XCDs in turn (block b to XCD b % 8),
-// and each XCD has its own L2.  Neighbouring column groups read the same
-// cosmology's records, so blocks are renumbered to give each XCD one
-// contiguous range of groups (a bijection of [0, n) for any n): a record is
-// then fetched into one L2 instead of two or three.
-__device__ inline int xcd_group(int b, int n) {
-  const int q = n >> 3, r = n & 7, x = b & 7;
-  return x * q + min(x, r) + (b >> 3);
-}
-
 // accumulators reduced through LDS per pass (bounds the LDS a block needs)
 template <int NACC>
 struct RedChunk { static constexpr int value = NACC < 32 ? NACC : 32; };
@@ -191,7 +181,7 @@ __global__ __launch_bounds__(256, (ND == 0 ? 4 : 1)) void k_limber(LimberArgs A)
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int nwv = A.waves;
-  const int grp = xcd_group(blockIdx.x, gridDim.x);
+  const int grp = xcd_order(blockIdx.x, gridDim.x);
   const int g = grp * 64 + lane;
   const bool valid = g < A.ncols;
   const int gc = valid ? g : A.ncols - 1;
@@ -605,7 +595,7 @@ __global__ __launch_bounds__(64 * FWD_WAVES, 4) void k_limber_tab(LimberArgs A) 
   float4* srec = lds4 + 2 * NEHQ + wave * (S::WAVE_LDS / 4);  // [2][FCH][4]
   float4* sR = srec + 2 * FCH * 4;                            // [2][FCH][TP / 4]
 
-  const int g0 = xcd_group(blockIdx.x, gridDim.x) * 64;
+  const int g0 = xcd_order(blockIdx.x, gridDim.x) * 64;
   const int g = g0 + lane;
   const bool valid = g < A.ncols;
   const int gc = valid ? g : A.ncols - 1;
@@ -990,11 +980,11 @@ __global__ __launch_bounds__(256, 4) void k_limber_ragged_fwd(RaggedArgs A) {
   // live tiles dealt to the 8 XCDs in contiguous ranges (the grid is a multiple of 8)
   const int live = (ncols + 63) >> 6;
   const int nsl = ragged_slices(live, A.waves, A.Na, A.max_slices);
-  const int xq = live >> 3, xr = live & 7, xx = blockIdx.x & 7, u = blockIdx.x >> 3;
-  const int mine = xq + (xx < xr ? 1 : 0);  // this XCD's tiles
+  const XcdShare xs = xcd_share(blockIdx.x, live);  // this XCD's tiles
+  const int u = blockIdx.x >> 3, mine = xs.count;
   if (u >= mine * nsl) return;
   const int slice = u / mine;
-  const int tile0 = (xx * xq + min(xx, xr) + u - slice * mine) * 64;
+  const int tile0 = (xs.first + u - slice * mine) * 64;
   const int first = A.cols[tile0].job;
   const int T = __builtin_amdgcn_readfirstlane(A.jobs[first].T);
   // the requests of the tile: a new one starts at each lane whose job
