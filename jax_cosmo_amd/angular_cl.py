@@ -155,10 +155,10 @@ def angular_cl_batch(cosmo_params, ell, probes, n_z=DEFAULT_N_Z, transfer_fn=tkl
         import torch
 
         cp = cosmo_params.to(torch.float64).reshape(B, 8).contiguous()
-        el = _device_ell(ell, cp.device).reshape(-1)
+        stream = torch.cuda.current_stream(cp.device).cuda_stream
+        el = _device_ell(ell, cp.device, stream).reshape(-1)
         out = torch.empty((B, P, el.shape[0]), dtype=torch.float32, device=cp.device)
-        ctx.angular_cl_dev(cp.data_ptr(), B, set_id, el.data_ptr(), el.shape[0], n_z,
-                           out.data_ptr(), stream=torch.cuda.current_stream(cp.device).cuda_stream)
+        ctx.angular_cl_dev(cp.data_ptr(), B, set_id, el.data_ptr(), el.shape[0], n_z, out.data_ptr(), stream=stream)
         return out
     cp = np.asarray(cosmo_params, dtype=np.float64).reshape(-1, 8)
     if _is_torch(ell):
@@ -227,18 +227,21 @@ _ELL_CACHE_MAX = 16
 _ELL_LOCK = threading.Lock()  # backward passes run on autograd's threads
 
 
-def _device_ell(ell, device):
-    """ell as a float64 tensor on ``device``.  A device tensor is used as it
-    is; a host array is uploaded once and kept (keyed by its bytes), so that
-    repeated batches over the same multipoles copy nothing to the device.  The
-    tensor may be read on the current stream: should it leave the cache, its
-    memory waits for what that stream has queued by then."""
+def _device_ell(ell, device, stream=None):
+    """ell as a float64 tensor on ``device``, to be read on the current stream
+    (``stream``: its handle, where the caller has it).  A device tensor is used
+    as it is; a host array is uploaded once and kept (keyed by its bytes), so that
+    repeated batches over the same multipoles copy nothing to the device.  Each
+    stream has its own copy: its memory goes back to that stream when the copy
+    leaves the cache, behind what the stream has queued by then."""
     import torch
 
     if _is_torch(ell):
         return ell.to(device=device, dtype=torch.float64).contiguous()
     a = np.ascontiguousarray(np.atleast_1d(np.asarray(ell, dtype=np.float64)))
-    key = (str(device), a.tobytes())
+    if stream is None and device.type == "cuda":
+        stream = torch.cuda.current_stream(device).cuda_stream
+    key = (str(device), stream, a.tobytes())
     with _ELL_LOCK:
         el = _ELL_CACHE.get(key)
         if el is None:
@@ -246,8 +249,6 @@ def _device_ell(ell, device):
             if len(_ELL_CACHE) >= _ELL_CACHE_MAX:
                 _ELL_CACHE.pop(next(iter(_ELL_CACHE)))
             _ELL_CACHE[key] = el
-    if el.is_cuda:
-        el.record_stream(torch.cuda.current_stream(el.device))
     return el
 
 

@@ -26,11 +26,11 @@ def _assemble(theta, omega_k):
     return params
 
 
-def _kept_ell(ell64, device):
+def _kept_ell(ell64, device, stream):
     # a graph would hold the kept tensor's address (and the context's buffers') for good
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError("C_ell with gradients cannot be captured into a graph (BatchGraph captures a forward batch)")
-    return _device_ell(ell64, device)
+    return _device_ell(ell64, device, stream)
 
 
 class AngularClFunction(torch.autograd.Function):
@@ -42,12 +42,12 @@ class AngularClFunction(torch.autograd.Function):
         params = _assemble(theta, omega_k)
         ell64 = np.ascontiguousarray(np.asarray(ell, dtype=np.float64).reshape(-1))
         if theta.is_cuda:
-            el = _kept_ell(ell64, theta.device)
+            stream = torch.cuda.current_stream(theta.device).cuda_stream
+            el = _kept_ell(ell64, theta.device, stream)
             out = torch.empty((params.shape[0], n_pairs, el.shape[0]), dtype=torch.float32,
                               device=theta.device)
             dctx.angular_cl_dev(params.data_ptr(), params.shape[0], set_id, el.data_ptr(),
-                                el.shape[0], n_z, out.data_ptr(),
-                                stream=torch.cuda.current_stream(theta.device).cuda_stream)
+                                el.shape[0], n_z, out.data_ptr(), stream=stream)
         else:
             out = torch.from_numpy(dctx.angular_cl(params.numpy(), set_id, ell64, n_z, n_pairs))
         ctx.save_for_backward(params)
@@ -64,11 +64,11 @@ class AngularClFunction(torch.autograd.Function):
         dctx.set_growth(models[2])
         g32 = grad.detach().to(torch.float32).contiguous()
         if params.is_cuda:
-            el = _kept_ell(ell64, params.device)
+            stream = torch.cuda.current_stream(params.device).cuda_stream
+            el = _kept_ell(ell64, params.device, stream)
             th = torch.empty((params.shape[0], 7), dtype=torch.float64, device=params.device)
             dctx.angular_cl_vjp_dev(params.data_ptr(), params.shape[0], set_id, el.data_ptr(),
-                                    el.shape[0], n_z, g32.data_ptr(), th.data_ptr(),
-                                    stream=torch.cuda.current_stream(params.device).cuda_stream)
+                                    el.shape[0], n_z, g32.data_ptr(), th.data_ptr(), stream=stream)
         else:
             th = torch.from_numpy(dctx.angular_cl_vjp(params.numpy(), set_id, ell64, n_z,
                                                       g32.numpy()))

@@ -49,9 +49,9 @@ def test_evicted_list_waits_for_the_other_stream():
     x = torch.randn(4096, 4096, device="cuda")
     torch.cuda.synchronize()
     with torch.cuda.stream(side):
+        ptr = acl._device_ell(np.full(n, 3.0), dev).data_ptr()  # as a call on `side` takes it
         for _ in range(60):
             x = (x @ x).clamp_(-1, 1)
-        ptr = acl._device_ell(np.full(n, 3.0), dev).data_ptr()  # as a call on `side` takes it
     for k in range(acl._ELL_CACHE_MAX):
         acl._device_ell(np.array([7.0 + k]), dev)
     assert not side.query(), "the side stream was meant to be busy still"
