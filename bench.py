@@ -39,20 +39,25 @@ PEAK_LANE_OPS = 256 * 64 * 2.4e9
 # FP32 VALU lane-ops (add/mul/fma/compare = 1; div, exp, log, sin, sqrt = 4;
 # non-integer pow = 9) for the minimal direct formulation: EH98 with wiggles
 # 123 + linear power 12 + halofit 85 + k and Limber weight 4 = 224, plus one
-# FMA per tracer pair for the contraction.  The transfer function is evaluated
-# once per node of a per-cosmology table (1024 nodes, built at the end of the
-# table kernel), and what depends on a alone is folded into the a-node records,
-# so the dominant kernel executes much less than that.
+# FMA per tracer pair for the contraction.  The dominant kernel performs the
+# linear power, halofit, k / weight and contraction pieces (101 + pairs); the
+# EH98 transfer function is evaluated once per node of a per-cosmology table
+# (1024 nodes, built at the end of the table kernel) and only interpolated per
+# point, so its 123 are charged to the table build, not to this kernel.
+# `roofline.achieved` = (101 + pairs) x points per launch / launch time.  What
+# depends on a alone is folded into the a-node records, so the kernel executes
+# fewer than that, and `frac` can exceed 1.
 OPS_PER_POINT = 224
+OPS_PER_POINT_LIMBER = 12 + 85 + 4
 # What the kernel issues per point, one per VALU instruction:
 #   table position (add, compare, fraction, add with carry, clamp, address)  6
 #   cubic Hermite piece, Delta_L^2                                           6
 #   y, log2 y, f(y)                                                          5
 #   halofit: 4 exp2 + 1 log2 + 1 reciprocal and 17 simple                   23
 # = 40, plus per tracer one multiply and per pair one FMA: 105 on the
-# 10-tracer workload, the instructions of the compiled loop.
-# `roofline.achieved` = (40 + tracers + pairs) x points per launch / launch time.
-OPS_PER_POINT_LIMBER = 40
+# 10-tracer workload, the instructions of the compiled loop.  `issued_frac`
+# uses it.
+INSTS_PER_POINT = 40
 # HBM bytes per k_limber_tab launch on this workload, from two rocprofv3 --pmc
 # runs of `bench.py --batch-only` (FETCH_SIZE 42552 KiB x 2.0 + WRITE_SIZE 22086
 # KiB x 1.0 per dispatch; the factors make a plain 256 MiB copy read the
@@ -582,9 +587,10 @@ def main():
     lim_ms, lim_n = prof["limber"]
     lim_avg_ms = lim_ms / max(lim_n, 1)
     Na = n_z + 1
-    ops_launch = float(B) * Na * len(ell) * (OPS_PER_POINT_LIMBER + T + P)
+    ops_launch = float(B) * Na * len(ell) * (OPS_PER_POINT_LIMBER + P)
     achieved = ops_launch / (lim_avg_ms * 1e-3)
     direct_launch = float(B) * Na * len(ell) * (OPS_PER_POINT + P)
+    issued_launch = float(B) * Na * len(ell) * (INSTS_PER_POINT + T + P)
     # whole step: the per-point work plus the per-cosmology tables (n_eff/C
     # 257 Na 14, sigma^2(R) 257 x 256 x 8, lensing 40 and clustering 20 per
     # bin and node, background tables 60 k), the same lane-op weights
@@ -596,13 +602,22 @@ def main():
         "achieved": achieved / 1e12,
         "peak": PEAK_LANE_OPS / 1e12,
         "unit": "TFLOP/s",
-        "unit_note": "10^12 FP32 VALU lane instructions/s (peak: one per lane and clock); instructions per "
-                     "launch = B x (n_z+1) x n_ell x (40 + tracers + pairs), those of the compiled loop",
+        "unit_note": "10^12 FP32 VALU lane-ops/s (one per lane per clock; div and transcendentals "
+                     "weigh 4); algorithmic ops per launch = B x (n_z+1) x n_ell x (101 + pairs): the "
+                     "linear power (12), halofit (85), k and weight (4) and contraction (1 per pair) "
+                     "pieces of the per-point count, which this kernel performs; the EH98 piece (123 "
+                     "per point in the direct form) is done once per node of the per-cosmology "
+                     "transfer table in the table kernel; parts that depend on a alone are folded into "
+                     "the a-node records, so frac can exceed 1: issued_frac is the kernel's issue rate",
         "frac": achieved / PEAK_LANE_OPS,
         "direct_formulation_ops_per_launch": direct_launch,
         "direct_formulation_note": "B x (n_z+1) x n_ell x (224 + pairs): EH98 evaluated at every point; "
                                    "this over the launch time is what the kernel would have to sustain "
                                    "to match it without the transfer table",
+        "issued_per_launch": issued_launch,
+        "issued_frac": issued_launch / (lim_avg_ms * 1e-3) / PEAK_LANE_OPS,
+        "issued_note": "VALU instructions of the compiled loop x lanes, B x (n_z+1) x n_ell x (40 + tracers + "
+                       "pairs), over the peak of one per lane and clock",
         "traffic": LIMBER_HBM_BYTES,
         "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated)",
         "traffic_rate_GBps": LIMBER_HBM_BYTES / (lim_avg_ms * 1e-3) / 1e9,
