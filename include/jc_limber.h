@@ -383,7 +383,7 @@ typedef struct jc_server_config {
   int32_t max_ell;    /* ell values per request (default 256)                     */
   int32_t slots;      /* batches in flight (default 2)                            */
   int32_t waves;      /* Limber kernel waves per block, 1/2/4 (0 = 2)             */
-  int32_t wl_ctile;   /* weak-lensing cosmologies per block, 1/4/8 (0 = 4)        */
+  int32_t wl_ctile;   /* weak-lensing cosmologies per block, 1/4/8/16 (0 = 4)     */
   int32_t use_graph;  /* 1: replay a captured hipGraph per batch                  */
   int32_t n_nz;       /* number of Simpson sizes served (1..4)                    */
   int32_t n_z[4];     /* the sizes, e.g. 256, 512, 1024                           */

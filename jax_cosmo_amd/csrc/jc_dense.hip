@@ -435,8 +435,9 @@ __global__ void k_zero_upper(double* __restrict__ A, int64_t N) {
 // Inverses of the SB x SB diagonal blocks of L, one block after another in
 // inv ([ceil(N / SB)][SB][SB], row-major; rows past N count as identity; the
 // 64 x 64 sub-blocks above the diagonal are not written).  The forward error
-// of a product with a triangle's inverse has the bound of substitution,
-// |L^-1| |L| |x|, and the 64 divisions and broadcasts a substitution chains
+// of a solve by products with the triangles' inverses has the bound of
+// substitution, |L^-1| |L| |x| (its residual has not: a factorisation corrects for
+// that, k_chol_panel), and the 64 divisions and broadcasts a substitution chains
 // per block are gone.
 // k_tri_inv64: the 64 x 64 diagonal blocks.
 __global__ __launch_bounds__(256, 2) void k_tri_inv64(const double* __restrict__ L, int64_t N, double* __restrict__ inv) {

@@ -846,10 +846,9 @@ hipError_t launch_pk_eval(const PkArgs& a, hipStream_t s) {
 // uniform across a wave.  Row c of R holds request c's tracers in its own
 // order.  Every request's cosmology has its own transfer table (built over
 // its own ell range by the table kernel).  The a range of a tile is split
-// over the waves of its block and over ragged_slices(live tiles) blocks
-// (grid y), so small batches still fill the GPU; the slices' partials are
-// added in a fixed order by k_ragged_slice_sum (forward) or k_ragged_reduce
-// (adjoint).
+// over the waves of its block and over ragged_slices(live tiles) blocks, so
+// small batches still fill the GPU; the slices' partials are added in a fixed
+// order by k_ragged_slice_sum.  (The adjoint of served batches: jc_adjoint.hip.)
 
 // The forward ragged kernel with the tile's tracer count T as a constant
 // (one body per T, chosen by a block-uniform switch): fixed pair loops

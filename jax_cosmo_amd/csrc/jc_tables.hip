@@ -1,4 +1,4 @@
-// Per-cosmology tables (FP64) and the weak-lensing radial kernels.
+// Per-cosmology tables (FP64), and the KDE n(z).
 //
 // k_tables: one workgroup per cosmology builds, in FP64,
 //   * the chi(a) table: RK4 in ln a of a y-independent right-hand side, i.e.
@@ -25,12 +25,7 @@
 //   * for calls in table mode, beside the a-nodes, the cosmology's transfer
 //     table T(k) k^(n_s/2) over the call's ln k range.
 // Measured (n_z 512, 100 ell): 1 cosmology 50 -> 31 us, 1024 112 -> 92 us, the
-// 7-direction dual form for 256 cosmologies 195 -> 125 us.
-// k_wl: the weak-lensing radial kernel (probes.py:16-51) with the
-//   reference's own per-z 256-interval Simpson over [z, zmax]: the
-//   cosmology-independent parts (n(z') and Simpson weights, the chi-table
-//   segment and offset of every z') are resident tables, so per cosmology
-//   only the chi lookup and the (chi' - chi)/chi' factor are evaluated.
+// 7-direction dual form for 256 cosmologies 195 -> 119 us.
 #include <type_traits>
 
 #include "jc_records.hpp"
